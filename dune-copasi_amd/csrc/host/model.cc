@@ -566,7 +566,8 @@ void Model::setup_device() {
     ilu_sweep_ = widest <= kIluSweepWidth;
     lo_lev_.upload(lo_ptr_, stream_);
     up_lev_.upload(up_ptr_, stream_);
-    if (ilu_sweep_) build_ilu_sweep_tables(rows, rows_u);
+    ilu_stencil_ = build_ilu_stencil(rows, rows_u);
+    if (ilu_sweep_ && !ilu_stencil_) build_ilu_sweep_tables(rows, rows_u);
     lu_.resize(static_cast<size_t>(matrix_values()));
   }
   {
@@ -1260,6 +1261,132 @@ void Model::build_ilu_sweep_tables(const std::vector<int>& lrows, const std::vec
   ilu_tab_ = t;
 }
 
+// Tables of the stencil form of ILU0 (k::IluStencil) from the level
+// schedules.  It takes structured 1D and 2D grids with blocks of at most 2
+// species whose rows hold only the 3 x 3 neighbours of their own compartment
+// (no blocks across an interface), where every level's rows (times the
+// species) fit half a workgroup and the ring of results fits LDS; everything
+// else keeps the table-driven sweeps, which take any pattern.
+bool Model::build_ilu_stencil(const std::vector<int>& lrows, const std::vector<int>& urows) {
+  const Grid& g = L_.grid;
+  const long ns = L_.nslot;
+  if (g.unstructured || g.dim > 2 || L_.B > 2 || extra_pos_.size() || ns <= 0) return false;
+  const int shift = g.dim == 1 ? 3 : 0;  // 1D offsets are the middle row of the 3 x 3 stencil
+  constexpr int NP = k::kIluPlaces;
+  k::IluStencil t;
+  t.nrows = static_cast<int>(ns);
+  t.nlo = static_cast<int>(lo_ptr_.size()) - 1;
+  t.nup = static_cast<int>(up_ptr_.size()) - 1;
+  t.lo_lev = lo_lev_.get();
+  t.up_lev = up_lev_.get();
+  t.lo_rows = lo_rows_.get();
+  t.up_rows = up_rows_.get();
+  std::vector<int> llev(ns), lpos(ns), ulev(ns), upos(ns);
+  auto positions = [](const std::vector<int>& ptr, const std::vector<int>& rows, std::vector<int>& lev,
+                      std::vector<int>& pos, int& width) {
+    for (size_t l = 0; l + 1 < ptr.size(); ++l) {
+      width = std::max(width, ptr[l + 1] - ptr[l]);
+      for (int q = ptr[l]; q < ptr[l + 1]; ++q) {
+        lev[rows[q]] = static_cast<int>(l);
+        pos[rows[q]] = q - ptr[l];
+      }
+    }
+  };
+  positions(lo_ptr_, lrows, llev, lpos, t.width);
+  positions(up_ptr_, urows, ulev, upos, t.width);
+  // a row's neighbours: column of stencil place o (-1: absent)
+  auto neighbour = [&](long i, unsigned mask, int o) -> int {
+    return (mask >> o) & 1u ? L_.col[L_.own_start[i] + __builtin_popcount(mask & ((1u << o) - 1u))] : -1;
+  };
+  int dist = 0;
+  for (long i = 0; i < ns; ++i) {
+    if (L_.own_start[i] != L_.row_ptr[i] ||
+        L_.row_ptr[i + 1] - L_.row_ptr[i] != __builtin_popcount(L_.own_mask[i]))
+      return false;
+    for (int p = L_.row_ptr[i]; p < L_.row_ptr[i + 1]; ++p) {
+      const int k = L_.col[p];
+      dist = std::max(dist, k < i ? llev[i] - llev[k] : k > i ? ulev[i] - ulev[k] : 0);
+    }
+  }
+  t.ring = 1;
+  while (t.ring < dist + 1) t.ring *= 2;
+  {
+    // places whose rows are never in the level right before the reader's
+    bool near[NP] = {};
+    for (long i = 0; i < ns; ++i)
+      for (int a = 0; a < NP; ++a) {
+        const int k = neighbour(i, L_.own_mask[i] << shift, a);
+        if (k >= 0 && llev[i] - llev[k] < 2) near[a] = true;
+      }
+    while (t.lo_early < NP - 1 && !near[t.lo_early]) ++t.lo_early;
+  }
+  int lds = 64 * 1024;
+  {
+    int v = 0;
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMaxSharedMemoryPerBlock, device_) == hipSuccess)
+      lds = std::max(lds, std::min(v, 160 * 1024));
+  }
+  if (!k::ilu_stencil_fits(t, L_.B, static_cast<size_t>(lds))) return false;
+  const int LW = k::ilu_stencil_lower_words(L_.B), UW = k::ilu_stencil_upper_words(L_.B);
+  if (ns * UW > 0x7fffffffL) return false;
+  const int zero = t.ring * t.width;
+  std::vector<int4> frow(ns);
+  std::vector<int> first(ns);
+  std::vector<ushort4> lsrc(ns), usrc(ns);
+  std::vector<int2> up(ns);
+  for (int pass = 0; pass < 2; ++pass) {
+    const auto& rows = pass ? urows : lrows;
+    const auto& ptr = pass ? up_ptr_ : lo_ptr_;
+    const auto& lev = pass ? ulev : llev;
+    const auto& pos = pass ? upos : lpos;
+    // replayed on the host: every slot holds the neighbour's row when its
+    // reader runs
+    std::vector<int> held(static_cast<size_t>(zero), -1);
+    for (size_t l = 0; l + 1 < ptr.size(); ++l) {
+      for (int q = ptr[l]; q < ptr[l + 1]; ++q) {
+        const int i = rows[q];
+        const unsigned mask = L_.own_mask[i] << shift;
+        unsigned short s[NP];
+        for (int a = 0; a < NP; ++a) {
+          const int k = neighbour(i, mask, pass ? NP + 1 + a : a);
+          const int slot = k < 0 ? zero : (lev[k] % t.ring) * t.width + pos[k];
+          if (k >= 0 && (held[slot] != k || lev[k] >= static_cast<int>(l)))
+            throw Error("internal: ILU0 stencil ring table");
+          s[a] = static_cast<unsigned short>(slot);
+        }
+        (pass ? usrc : lsrc)[q] = make_ushort4(s[0], s[1], s[2], s[3]);
+        if (!pass) {
+          frow[q] = make_int4(i, ptr[l], ptr[l + 1] - ptr[l], static_cast<int>(mask));
+          first[q] = L_.own_start[i];
+          const int ul = ulev[i], ub = up_ptr_[ul];
+          up[q] = make_int2(ub * UW + upos[i], up_ptr_[ul + 1] - ub);
+        }
+      }
+      for (int q = ptr[l]; q < ptr[l + 1]; ++q)
+        held[(static_cast<int>(l) % t.ring) * t.width + (q - ptr[l])] = rows[q];
+    }
+  }
+  st_frow_.upload(frow, stream_);
+  st_first_.upload(first, stream_);
+  st_lsrc_.upload(lsrc, stream_);
+  st_usrc_.upload(usrc, stream_);
+  st_upos_.upload(up, stream_);
+  const size_t N = static_cast<size_t>(ns);
+  st_pack_.resize(N * (2 * NP + 1) * L_.B * L_.B);
+  st_lower_.resize(N * LW * 2);
+  st_upper_.resize(N * UW * 2);
+  k::fill(st_lower_.get(), 0.0, static_cast<long>(N) * LW * 2, stream_);
+  k::fill(st_upper_.get(), 0.0, static_cast<long>(N) * UW * 2, stream_);
+  t.frow = st_frow_.get();
+  t.first = st_first_.get();
+  t.lo_src = st_lsrc_.get();
+  t.up_src = st_usrc_.get();
+  t.upos = st_upos_.get();
+  ilu_st_ = t;
+  synchronize();  // the host tables end here
+  return true;
+}
+
 void Model::precond_setup(const KrylovWork& w) {
   const int B = L_.B;
   const int ns = static_cast<int>(L_.nslot);
@@ -1269,6 +1396,10 @@ void Model::precond_setup(const KrylovWork& w) {
   } else if (jacobi_kind()) {
     k::block_inverse(B, ns, w.val, diag_pos_.get(), w.dinv, w.status, cfg_.precond == Preconditioner::Jacobi, stream_);
   } else if (cfg_.precond == Preconditioner::ILU0) {
+    if (ilu_stencil_) {
+      k::ilu_stencil_factor(B, ilu_st_, w.val, st_pack_.get(), st_lower_.get(), st_upper_.get(), w.status, stream_);
+      return;
+    }
     DCG_HIP(hipMemcpyAsync(w.lu, w.val, matrix_values() * sizeof(double), hipMemcpyDeviceToDevice, stream_));
     if (ilu_sweep_) {
       k::ilu_factor_sweep(B, ilu_tab_, row_ptr_.get(), col_.get(), diag_pos_.get(), w.lu, w.dinv, w.status, stream_);
@@ -1301,6 +1432,10 @@ int Model::bicgstab64(const double* b, double* x, double rtol, double abstol, in
   const bool point_jacobi = cfg_.precond == Preconditioner::Jacobi;
   const bool ilu = cfg_.precond == Preconditioner::ILU0;
   auto apply_ilu = [&](const double* in, double* out) {
+    if (ilu_stencil_) {
+      k::ilu_stencil_apply<double>(B, ilu_st_, st_lower_.get(), st_upper_.get(), in, tmp, out, sc, stream_);
+      return;
+    }
     if (ilu_sweep_) {
       k::ilu_apply_sweep<double>(B, ilu_tab_, row_ptr_.get(), col_.get(), diag_pos_.get(), w.lu, w.dinv, in, tmp,
                                  out, sc, stream_);
@@ -1403,6 +1538,10 @@ int Model::bicgstab32(const double* b, float* x, double rtol, int maxit, int* it
   const bool point_jacobi = cfg_.precond == Preconditioner::Jacobi;
   const bool ilu = cfg_.precond == Preconditioner::ILU0;
   auto apply_ilu = [&](const float* in, float* out) {
+    if (ilu_stencil_) {
+      k::ilu_stencil_apply<float>(B, ilu_st_, st_lower_.get(), st_upper_.get(), in, tmp, out, sc_.get(), stream_);
+      return;
+    }
     if (ilu_sweep_) {
       k::ilu_apply_sweep<float>(B, ilu_tab_, row_ptr_.get(), col_.get(), diag_pos_.get(), lu_.get(), dinv_.get(), in,
                                 tmp, out, sc_.get(), stream_);
@@ -2021,7 +2160,8 @@ size_t Model::device_bytes() const {
              lin_x_.bytes() + lo_ent_.bytes() + lo_blk_.bytes() + lo_src_.bytes() + up_ent_.bytes() + up_blk_.bytes() +
              up_src_.bytes() + lo_chunk_.bytes() + up_chunk_.bytes() +
              ilu_frow_.bytes() + ilu_fub_.bytes() + ilu_fm_.bytes() + ilu_fpush_.bytes() + ilu_packed_.bytes() +
-             ilu_inbox_.bytes();
+             ilu_inbox_.bytes() + st_frow_.bytes() + st_first_.bytes() + st_lsrc_.bytes() + st_usrc_.bytes() +
+             st_upos_.bytes() + st_pack_.bytes() + st_lower_.bytes() + st_upper_.bytes();
   for (const auto& v : pc_) b += v.bytes();
   for (const auto& v : pc32_) b += v.bytes();
   for (const auto& v : stage_) b += v.bytes();

@@ -390,6 +390,17 @@ class Model {
   k::IluSweep ilu_tab_;
   static constexpr size_t kIluLdsBytes = 64 * 1024;  // dynamic LDS of the sweeps
   void build_ilu_sweep_tables(const std::vector<int>& lrows, const std::vector<int>& urows);
+  // the stencil form (structured 1D / 2D grids, blocks of at most 2 species):
+  // its tables, packed blocks and solve streams; false when the model's rows
+  // or levels do not suit it
+  k::IluStencil ilu_st_;
+  bool ilu_stencil_ = false;
+  DeviceArray<int4> st_frow_;
+  DeviceArray<int> st_first_;
+  DeviceArray<ushort4> st_lsrc_, st_usrc_;
+  DeviceArray<int2> st_upos_;
+  DeviceArray<double> st_pack_, st_lower_, st_upper_;
+  bool build_ilu_stencil(const std::vector<int>& lrows, const std::vector<int>& urows);
   bool ilu_ready_ = false;
   std::vector<std::pair<int, double>> tuning_;
   // profiling

@@ -287,6 +287,41 @@ void ilu_apply_sweep(int B, const IluSweep& t, const int* rp, const int* col, co
                      const double* dinv, const V* in, V* tmp, V* out, const BicgScalars* sc, hipStream_t s);
 // LDS bytes of the chunked apply's stage and ring for values of vbytes bytes
 size_t ilu_chunk_lds_bytes(const IluSweep& t, int B, int vbytes);
+// The stencil form of ILU0 (ilu_stencil.hip): structured 1D / 2D grids whose
+// rows hold only their own compartment's 3 x 3 neighbours, blocks of at most
+// 2 species.  The four neighbours before and after the diagonal have places
+// fixed by their stencil offset.  Rows are taken by position in level order:
+//   frow[q]: row, first position and rows of its level, 9-bit stencil mask;
+//   first[q]: the row's first block of the matrix;
+//   lo_src / up_src[q]: ring slots of the row's neighbours before / after it
+//   (slot (level mod ring) * width + position in the level; absent
+//   neighbours take the zero row, slot ring * width);
+//   lo_early: the first places whose rows lie two or more levels back
+//   everywhere (at most 3);
+//   upos[q]: (first 16-byte word of the row in the backward solve's stream,
+//   rows of its backward level).
+// The streams hold 16-byte words word-major per level: word k of the row at
+// position lr of a level of n rows beginning at b0 is [b0 * words + k * n + lr].
+constexpr int kIluPlaces = 4;
+struct IluStencil {
+  int nrows = 0, nlo = 0, nup = 0, width = 0, ring = 0;
+  int lo_early = 0;
+  const int *lo_lev = nullptr, *lo_rows = nullptr, *up_lev = nullptr, *up_rows = nullptr;
+  const int4* frow = nullptr;
+  const int* first = nullptr;
+  const ushort4 *lo_src = nullptr, *up_src = nullptr;
+  const int2* upos = nullptr;
+};
+int ilu_stencil_lower_words(int B);
+int ilu_stencil_upper_words(int B);
+// whether the kernels take these levels within `lds` bytes of LDS
+bool ilu_stencil_fits(const IluStencil& t, int B, size_t lds);
+// pack: 9 B^2 doubles per row; ls, us: the streams of the two solves
+void ilu_stencil_factor(int B, const IluStencil& t, const double* val, double* pack, double* ls, double* us,
+                        int* status, hipStream_t s);
+template <typename V>
+void ilu_stencil_apply(int B, const IluStencil& t, const double* ls, const double* us, const V* in, V* tmp, V* out,
+                       const BicgScalars* sc, hipStream_t s);
 template <typename V>
 void ilu_lower(int B, int nrows, const int* rows, const int* rp, const int* col, const int* diag_pos,
                const double* lu, const V* b, V* y, const BicgScalars* sc, hipStream_t s);

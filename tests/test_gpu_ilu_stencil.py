@@ -1,0 +1,125 @@
+"""The stencil form of ILU0 (1D and 2D structured grids, blocks of 1 and 2
+species) against the oracle at the sizes where its level schedule changes
+shape: single-cell grids, levels of 63 to 65 rows (one and two waves), of 128
+and more (the widest it takes), odd sizes, boxes and triangles, a compartment
+that covers a part of the grid.  The preconditioner is the same ILU0, so the
+Newton iterations are equal, the BiCGSTAB iterations equal within one and the
+states equal to the parity bar of the other sweeps (1e-8)."""
+import numpy as np
+import pytest
+
+from tests.oracle_lib import OracleModel, rel_l2_per_species
+
+pytestmark = pytest.mark.gpu
+
+
+def _gray_scott(wl, n, cell, precision="fp64"):
+    return wl.gray_scott(n=n, cell_type=cell, precond="ILU", nl_rtol=1e-20, lin_rtol=1e-12, precision=precision)
+
+
+def _compare(dca, w, state=None, mixed=False):
+    o = OracleModel(w.ini)
+    m = dca.Model(w.ini, "", 0)
+    u0 = w.initial_state(m) if state is None else state(m)
+    o.set_state(u0, 0.0)
+    m.set_state(u0, 0.0)
+    t = 0.0
+    for _ in range(2):
+        st = m.step(t, w.dt)
+        rc, newton, linear = o.step(w.dt)
+        assert (st.status, rc) == (0, 0)
+        if not mixed:
+            assert st.newton_iterations == newton
+            assert abs(st.linear_iterations - linear) <= max(1, linear // 50), (st.linear_iterations, linear)
+        t += w.dt
+    u, _ = m.get_state()
+    uo, _ = o.get_state()
+    assert max(rel_l2_per_species(m.compartments(), u, uo)) < 1e-8
+    o.close()
+    m.close()
+
+
+@pytest.mark.parametrize("cell", ["cube", "simplex"])
+@pytest.mark.parametrize("n", [1, 2, 7, 62, 63, 64, 125, 128, 131])
+def test_two_species_2d(dca, wl, n, cell):
+    print(f"case: stencil ILU0, 2 species, {cell} {n}", flush=True)
+    _compare(dca, _gray_scott(wl, n, cell))
+
+
+@pytest.mark.parametrize("n", [3, 64, 127])
+def test_mixed_precision(dca, wl, n):
+    print(f"case: stencil ILU0, mixed, {n}", flush=True)
+    _compare(dca, _gray_scott(wl, n, "cube", "mixed"), mixed=True)
+
+
+def _ilu0(n, rp, col, J):
+    """Block ILU0 on the host (row by row, the reference's SeqILU order) and its solve."""
+    a = [dict(zip(col[rp[i]:rp[i + 1]], J[rp[i]:rp[i + 1]].copy())) for i in range(n)]
+    dinv = [None] * n
+    for i in range(n):
+        for k in sorted(c for c in a[i] if c < i):
+            a[i][k] = a[i][k] @ dinv[k]
+            for j, u in a[k].items():
+                if j > k and j in a[i]:
+                    a[i][j] = a[i][j] - a[i][k] @ u
+        dinv[i] = np.linalg.inv(a[i][i])
+
+    def solve(v):
+        y = v.reshape(n, -1).copy()
+        for i in range(n):
+            for k, l in a[i].items():
+                if k < i:
+                    y[i] -= l @ y[k]
+        for i in reversed(range(n)):
+            for k, u in a[i].items():
+                if k > i:
+                    y[i] -= u @ y[k]
+            y[i] = dinv[i] @ y[i]
+        return y.reshape(-1)
+
+    return solve
+
+
+@pytest.mark.parametrize("dim,n,cell", [(1, 1, "cube"), (1, 70, "cube"), (2, 5, "cube"), (2, 5, "simplex"),
+                                        (2, 63, "simplex"), (2, 130, "cube")])
+@pytest.mark.parametrize("species", [1, 2])
+def test_first_iteration_against_host_ilu0(dca, wl, dim, n, cell, species):
+    """x after one BiCGSTAB iteration from zero is alpha M^-1 b + omega M^-1 s:
+    with M an ILU0 written out on the host.  Both sides round in FP64 over at
+    most 400 levels of a diagonally dominant solve: 1e-11."""
+    if species == 2 and dim == 1:
+        pytest.skip("the two-species workload is 2D")
+    print(f"case: first iteration, {species} species {dim}D {cell} {n}", flush=True)
+    w = (wl.exponential_decay(dim=dim, n=n, cell_type=cell, D=0.02) if species == 1 else _gray_scott(wl, n, cell))
+    m = dca.Model(w.ini, "", 0)
+    rng = np.random.default_rng(n)
+    _, J = m.assemble(0.5 + 0.3 * rng.random(m.n_dof), 0.0, 1.0, 0.1)
+    b = rng.standard_normal(m.n_dof)
+    rp, col = m.pattern()
+    solve = _ilu0(m.n_slots, rp, col, J)
+
+    def apply(x):
+        xb, y = x.reshape(m.n_slots, -1), np.zeros((m.n_slots, species))
+        np.add.at(y, np.repeat(np.arange(m.n_slots), np.diff(rp)), np.einsum("kij,kj->ki", J, xb[col]))
+        return y.reshape(-1)
+
+    ph = solve(b)
+    v = apply(ph)
+    alpha = (b @ b) / (b @ v)
+    s = b - alpha * v
+    sh = solve(s)
+    t = apply(sh)
+    omega = (t @ s) / (t @ t) if t @ t > 0 else 0.0
+    x, _, its = m.linear_solve(J, b, 1e-30, 1)
+    assert its == 1
+    ref = alpha * ph + omega * sh
+    assert np.linalg.norm(x - ref) <= 1e-11 * np.linalg.norm(ref)
+    m.close()
+
+
+def test_partial_compartment(dca, wl):
+    print("case: stencil ILU0, disk compartment", flush=True)
+    w = _gray_scott(wl, 40, "cube")
+    ini = w.ini.replace("domain.expression = 1", "domain.expression = (position_x-0.5)^2 + (position_y-0.45)^2 < 0.16")
+    w.ini = ini
+    _compare(dca, w, state=lambda m: 0.5 + 0.1 * np.random.default_rng(2).random(m.n_dof))
