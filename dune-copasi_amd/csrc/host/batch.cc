@@ -259,12 +259,12 @@ void Batch::rebuild() {
       for (int j = 0; j < M; ++j) {
         Model& m = *members_[g.mem[j]].m;
         size_t c0 = 0;
-        while (c0 < m.pc_.size() && !m.pc_[c0].size()) ++c0;
+        while (c0 < m.pc_.size() && !m.pc_[c0].size() && !m.gen_.corner[c0]) ++c0;
         if (c0 >= m.pc_.size()) throw Error("internal: point member without coefficients");
         k::PcMember& pm = pcm[j];
         pm.g2l = m.comp_dev_[c0].g2l_identity ? nullptr : m.comp_dev_[c0].g2l.get();
         pm.cmask = m.comp_dev_[c0].cell_mask_grid.get();
-        pm.pc = m.pc_[c0].get();
+        pm.pc = m.gen_.corner[c0] ? m.lin_x_.get() : m.pc_[c0].get();
         pm.pc32 = c0 < m.pc32_.size() ? m.pc32_[c0].get() : nullptr;
         pm.tca = m.pc_tca_.get();
         pm.prm = m.prm_.get();
@@ -292,7 +292,7 @@ void Batch::rebuild() {
             pl.f32s.push_back(opt_.precision == Precision::Mixed ? m.module_->function(name + "_pfbatch" + id)
                                                                  : nullptr);
             pl.tiles.push_back(m.gen_.apply_tiles[c0][k2]);
-            pl.nts.push_back(apply_tile_threads(m.L_.grid.dim, m.gen_.apply_tiles[c0][k2], m.L_.comps[c0].b));
+            pl.nts.push_back(m.gen_.apply_threads[c0][k2]);
           }
           pl.module = m.module_;
           items.emplace_back(nk);
@@ -410,14 +410,23 @@ void Batch::rebuild() {
       const auto& names = e.m->gen_.tile_batch_kernel;
       a.fn.assign(names.size(), nullptr);
       a.qfn.assign(names.size(), nullptr);
+      a.rfn.assign(names.size(), nullptr);
+      a.rthreads.assign(names.size(), 0);
       a.points = e.m->point_storage();
       for (size_t c = 0; c < names.size(); ++c)
         if (!names[c].empty()) {
           a.fn[c] = a.module->function(names[c]);
           if (a.points) a.qfn[c] = a.module->function(e.m->gen_.tile_kernel[c] + "_qbatch");
+          if (e.m->gen_.corner[c]) {
+            const int dim = e.m->L_.grid.dim;
+            a.rfn[c] = a.module->function(e.m->gen_.tile_kernel[c] + "_rbatch");
+            a.rthreads[c] = apply_tile_threads(dim, corner_tiles(dim).front(), e.m->L_.comps[c].b, true);
+          }
         }
       a.work.resize(names.size());
       a.nwork.assign(names.size(), 0);
+      a.rwork.resize(names.size());
+      a.nrwork.assign(names.size(), 0);
     }
     e.ag = it->second;
     e.ai = static_cast<int>(agroups_[e.ag].mem.size());
@@ -426,7 +435,7 @@ void Batch::rebuild() {
   for (auto& a : agroups_) {
     const int M = static_cast<int>(a.mem.size());
     std::vector<k::AsmMember> am(M);
-    std::vector<std::vector<int2>> work(a.fn.size());
+    std::vector<std::vector<int2>> work(a.fn.size()), rwork(a.fn.size());
     for (int j = 0; j < M; ++j) {
       Model& m = *members_[a.mem[j]].m;
       const auto v = m.view();
@@ -445,7 +454,7 @@ void Batch::rebuild() {
       }
       if (a.points) {
         for (size_t c = 0; c < m.pc_.size() && c < static_cast<size_t>(k::kAsmComps); ++c)
-          am[j].pc[c] = m.pc_[c].size() ? m.pc_[c].get() : nullptr;
+          am[j].pc[c] = m.gen_.corner[c] ? m.lin_x_.get() : m.pc_[c].size() ? m.pc_[c].get() : nullptr;
         am[j].pdiag = m.pdiag_.get();
         am[j].tca = m.pc_tca_.get();
       }
@@ -459,12 +468,20 @@ void Batch::rebuild() {
           DCG_HIP(hipMemcpy(tiles.data(), m.comp_dev_[c].tiles.get(), tiles.size() * sizeof(int),
                             hipMemcpyDeviceToHost));
         for (int t : tiles) work[c].push_back(make_int2(j, t));
+        if (!a.rfn[c]) continue;
+        tiles.resize(m.comp_dev_[c].nrtiles);
+        if (!tiles.empty())
+          DCG_HIP(hipMemcpy(tiles.data(), m.comp_dev_[c].rtiles.get(), tiles.size() * sizeof(int),
+                            hipMemcpyDeviceToHost));
+        for (int t : tiles) rwork[c].push_back(make_int2(j, t));
       }
     }
     a.am.upload(am, stream_);
     for (size_t c = 0; c < a.fn.size(); ++c) {
       a.work[c].upload(work[c], stream_);
       a.nwork[c] = static_cast<int>(work[c].size());
+      a.rwork[c].upload(rwork[c], stream_);
+      a.nrwork[c] = static_cast<int>(rwork[c].size());
     }
     a.coef.resize(static_cast<size_t>(kCalls) * M * 4);
     a.act.resize(2 * static_cast<size_t>(M));
@@ -633,11 +650,21 @@ void Batch::assemble(int call, const std::vector<char>& on, int xsel, int bsel, 
       const int2* work = a.work[c].get();
       const k::AsmMember* mem = a.am.get();
       int xs = xsel, bs = bsel, rs = rsel, md = mode;
+      const bool corner = a.rfn[c] != nullptr;
+      const int2* rwork = a.rwork[c].get();
       if (a.points && mode == 2) {
         // the point coefficients and diagonal blocks replace the matrix
-        void* qargs[] = {&work, &mem, &coef, &act, &xs};
-        DCG_HIP(hipModuleLaunchKernel(a.qfn[c], static_cast<unsigned>(a.nwork[c]), 1, 1, 256, 1, 1, 0, stream_,
-                                      qargs, nullptr));
+        int full = jacobi_kind() == 1 ? 1 : 0;  // the corner form: whole blocks or their diagonals
+        void* qargs[] = {corner ? &rwork : &work, &mem, &coef, &act, &xs, &full};
+        DCG_HIP(hipModuleLaunchKernel(a.qfn[c], static_cast<unsigned>(corner ? a.nrwork[c] : a.nwork[c]), 1, 1,
+                                      static_cast<unsigned>(corner ? a.rthreads[c] : 256), 1, 1, 0, stream_, qargs,
+                                      nullptr));
+        continue;
+      }
+      if (corner && mode == 1) {
+        void* rargs[] = {&rwork, &mem, &coef, &act, &xs, &bs, &rs, &md};
+        DCG_HIP(hipModuleLaunchKernel(a.rfn[c], static_cast<unsigned>(a.nrwork[c]), 1, 1,
+                                      static_cast<unsigned>(a.rthreads[c]), 1, 1, 0, stream_, rargs, nullptr));
         continue;
       }
       void* args[] = {&work, &mem, &coef, &act, &xs, &bs, &rs, &md};

@@ -151,6 +151,11 @@ class Batch {
     // point storage: the batched point set-up per compartment replaces the
     // Jacobian pass
     std::vector<hipFunction_t> qfn;
+    // corner form: the batched residual, its and the set-up's work items and
+    // workgroup size (0: not in the corner form)
+    std::vector<hipFunction_t> rfn;
+    std::vector<DeviceArray<int2>> rwork;
+    std::vector<int> nrwork, rthreads;
     bool points = false;
     std::vector<int> mem;
     DeviceArray<k::AsmMember> am;

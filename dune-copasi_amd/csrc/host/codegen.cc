@@ -258,6 +258,17 @@ struct dcg_pc_member {
 };
 static_assert(sizeof(dcg_asm_member) == %ASM_BYTES%, "batch member descriptor layout");
 static_assert(sizeof(dcg_pc_member) == %PCM_BYTES%, "point member descriptor layout");
+// whether an optional array argument is there: known at compile time for a
+// local array (compared with null at run time, such an array would stay in
+// scratch memory) and for nullptr
+template <typename M>
+struct dcg_ptr {
+  static __device__ __forceinline__ bool on(M p) { return p != nullptr; }
+};
+template <typename X, int N>
+struct dcg_ptr<X (&)[N]> {
+  static __device__ __forceinline__ constexpr bool on(X (&)[N]) { return true; }
+};
 __device__ __forceinline__ double dcg_sign(double v) { return (double)((v > 0.0) - (v < 0.0)); }
 __device__ __forceinline__ int dcg_pos(const int* own_start, const unsigned* own_mask, int s, int o) {
   return own_start[s] + __popc(own_mask[s] & ((1u << o) - 1u));
@@ -827,12 +838,15 @@ std::string gen_volume(const ModelSpec& m, const Grid& g, int comp, const std::s
     }
   }
   // quadrature point kernel
+  if (!with_kernel) o << "template <typename M>\n";
   o << "__device__ __forceinline__ void qp(int q, const double (&u)[BC], const double (&g)[BC][3], double px, double py, "
        "double pz, double t, double cm, double ca, double (&rs)[BC], double (&rf)[BC][DIM], "
-    << (with_kernel ? "double (*mc)[BC], " : "double* mc, ")
+    << (with_kernel ? "double (*mc)[BC], " : "M&& mcv, ")
     << "double (*gc)[BC][DIM], double (*dc)[BC][DIM][DIM], const double* __restrict__ prm, "
        "const double* __restrict__ eg) {\n";
   o << "  (void)px; (void)py; (void)pz; (void)t; (void)g; (void)gc; (void)dc; (void)prm; (void)eg;\n";
+  o << (with_kernel ? "  const bool mc_on = mc != nullptr;\n"
+                    : "  double* mc = mcv;\n  const bool mc_on = dcg_ptr<M>::on(mcv);\n");
   o << "  const double fac = FACQ(q);\n";
   o << "#pragma unroll\n  for (int i = 0; i < BC; ++i) { rs[i] = 0.0;\n#pragma unroll\n for (int k = 0; k < DIM; ++k) rf[i][k] = 0.0; }\n";
   // tiled compartments keep only the structural nonzeros of mc, in the
@@ -845,9 +859,9 @@ std::string gen_volume(const ModelSpec& m, const Grid& g, int comp, const std::s
     throw Error("internal: coefficient outside the point pattern");
   };
   if (with_kernel)
-    o << "  if (mc) {\n#pragma unroll\n  for (int i = 0; i < BC; ++i)\n#pragma unroll\n for (int j = 0; j < BC; ++j) mc[i][j] = 0.0;}\n";
+    o << "  if (mc_on) {\n#pragma unroll\n  for (int i = 0; i < BC; ++i)\n#pragma unroll\n for (int j = 0; j < BC; ++j) mc[i][j] = 0.0;}\n";
   else if (!mcnz.empty())
-    o << "  if (mc) {\n#pragma unroll\n  for (int n = 0; n < " << mcnz.size() << "; ++n) mc[n] = 0.0;}\n";
+    o << "  if (mc_on) {\n#pragma unroll\n  for (int n = 0; n < " << mcnz.size() << "; ++n) mc[n] = 0.0;}\n";
   if (has_gc)
     o << "  if (gc) {\n#pragma unroll\n for (int i = 0; i < BC; ++i)\n#pragma unroll\n for (int j = 0; j < BC; ++j)\n#pragma unroll\n for (int k = 0; k < DIM; ++k) gc[i][j][k] = 0.0;}\n";
   if (has_dc)
@@ -859,7 +873,7 @@ std::string gen_volume(const ModelSpec& m, const Grid& g, int comp, const std::s
     if (sp.storage) {
       o << "    const double S = " << E(sp.storage) << ";\n";
       o << "    rs[" << I << "] += fac * cm * S * u[" << I << "];\n";
-      o << "    if (mc) { " << MC(i, i) << " += fac * cm * S;\n";
+      o << "    if (mc_on) { " << MC(i, i) << " += fac * cm * S;\n";
       for (const auto& pj : sp.storage_jac) {
         if (m.species[pj.wrt].comp != comp) continue;
         o << "      " << MC(i, m.species[pj.wrt].local) << " += fac * cm * (" << E(pj.e) << ") * u[" << I << "];\n";
@@ -868,7 +882,7 @@ std::string gen_volume(const ModelSpec& m, const Grid& g, int comp, const std::s
     }
     if (sp.reaction) {
       o << "    rs[" << I << "] -= fac * ca * (" << E(sp.reaction) << ");\n";
-      o << "    if (mc) {\n";
+      o << "    if (mc_on) {\n";
       for (const auto& pj : sp.reaction_jac) {
         if (m.species[pj.wrt].comp != comp) continue;
         o << "      " << MC(i, m.species[pj.wrt].local) << " -= fac * ca * (" << E(pj.e) << ");\n";
@@ -2080,8 +2094,7 @@ __device__ __forceinline__ void pc_apply(int tile, dcg_gp<const int> __restrict_
     %C%::tile_body<M>(tiles[blockIdx.x], g2l, cmask, x, base, t, cm, ca, r, val, own_start, own_mask, n0, n1, n2,  \
                       ox, oy, oz, hx, hy, hz, mode, prm);                                                         \
   }
-DCG_TILE_ENTRY(%KERNEL%_r, 1)
-DCG_TILE_ENTRY(%KERNEL%_j, 2)
+%R_ENTRY%DCG_TILE_ENTRY(%KERNEL%_j, 2)
 DCG_TILE_ENTRY(%KERNEL%_a, 4)
 #undef DCG_TILE_ENTRY
 )";
@@ -2196,9 +2209,404 @@ extern "C" __global__ void __launch_bounds__(256)
 }
 )";
 
+// Box cells with blocks of more than 4 species: one lane per (cell, corner).
+// A thread that holds all corners of a cell would need 2^DIM values per
+// species several times over; here a lane holds one corner's values, which
+// become its point's values and its corner's sums in place.  The trilinear
+// basis at the 2-point Gauss rule is a product of 1D maps, and each 1D map is
+// sum and difference of the two ends with one weight each: with H the
+// (sum, difference) butterfly over the corners and S the weights,
+//   values at the points = H S H (values at the corners),
+//   corner sums of point terms = H S H (point terms),
+//   element stiffness = H kap H with diagonal kap
+// (1D mass and stiffness are diagonal in sums and differences).  A butterfly
+// is one lane exchange per axis (DPP, no LDS) and one FMA.  The coefficients
+// of the Jacobian are evaluated at the linearisation point inside the apply,
+// so an apply reads two vectors instead of a matrix or stored coefficients.
+// A workgroup takes the cells around TX x TY row vertices of a layer and walks
+// TM layers along the last axis; a layer's corner sums meet in LDS, and what
+// it adds to the next layer's vertices stays in a register.
+// 7 species on 40^3 (68,921 vertices, 34 coefficients per point): apply FP32
+// 27 us and FP64 29 us (SpMV on the assembled matrix 83 and 220 us), set-up
+// 37 us (Jacobian pass 3,330 us and its FP32 copy 200 us), residual 28 us
+// (360 us with the corner values in LDS).  About 500 vector instructions per
+// wave and layer of 8 cells; bound by their issue and by the two barriers of
+// a layer, not by memory (12 MB per apply).
+const char* kCorner = R"(
+namespace %C% {
+template <int X, int Y, int Z>
+struct CornerTile {
+  static constexpr int TX = X, TY = DIM > 2 ? Y : 1;           // row vertices of a layer
+  static constexpr int TM = DIM > 2 ? Z : Y;                   // layers of row vertices
+  static constexpr int CX = TX + 1, CY = DIM > 2 ? TY + 1 : 1;  // cells of a layer
+  static constexpr int NT = CX * CY * NCORNER, ROWS = TX * TY;
+};
+%CORNER_SHAPES%
+%CORNER_TABLES%
+
+// the value of the lane at the other end of the cell along axis A: lanes of a
+// cell are l = (b0 | b1 << 1) ^ (b2 ? 7 : 0), so the three axes are the lane
+// exchanges xor 1, xor 2 and xor 7 (quad_perm, quad_perm, row_half_mirror)
+template <int A>
+__device__ __forceinline__ int corner_dpp(int v) {
+  return __builtin_amdgcn_mov_dpp(v, A == 0 ? 0xB1 : A == 1 ? 0x4E : 0x141, 0xF, 0xF, true);
+}
+template <int A>
+__device__ __forceinline__ float other_end(float v) {
+  return __int_as_float(corner_dpp<A>(__float_as_int(v)));
+}
+template <int A>
+__device__ __forceinline__ double other_end(double v) {
+  const long long u = __double_as_longlong(v);
+  const int lo = corner_dpp<A>((int)u), hi = corner_dpp<A>((int)(u >> 32));
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+// sums (bit 0) and differences (bit 1) over the corners along every axis
+template <typename T, int N>
+__device__ __forceinline__ void butterfly(T (&v)[N], const T (&sg)[3]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = fma(v[i], sg[0], other_end<0>(v[i]));
+    v[i] = fma(v[i], sg[1], other_end<1>(v[i]));
+    if constexpr (DIM > 2) v[i] = fma(v[i], sg[2], other_end<2>(v[i]));
+  }
+}
+
+// OP 1: y = base + residual at x (T = double).  OP 4: y = J(x) v and, with
+// part, the partial dots (y.w1, y.w2).  OP 8: diagonal blocks of J(x) into y
+// (all entries with `full`, else the diagonal) and the rows' x into lin.
+template <typename TL, int OP, typename T>
+__device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restrict__ g2l,
+                                            dcg_gp<const unsigned char> __restrict__ cmask,
+                                            dcg_gp<const double> x, dcg_gp<const T> v, dcg_gp<T> y,
+                                            dcg_gp<double> lin, double t, double cm, double ca, int n0, int n1, int n2,
+                                            double ox, double oy, double oz, double hx, double hy, double hz,
+                                            const double* __restrict__ prm, bool full, dcg_gp<const T> w1,
+                                            dcg_gp<const T> w2, double* __restrict__ part) {
+  constexpr int TX = TL::TX, TY = TL::TY, TM = TL::TM, CX = TL::CX, NT = TL::NT;
+  constexpr int PER = (TL::ROWS * DCG_B + NT - 1) / NT;
+  __shared__ T out[BC * NT];
+  const int tid = threadIdx.x, l = tid % NCORNER, cell = tid / NCORNER;
+  const int cx = cell % CX, cy = cell / CX;
+  const int b2 = DIM > 2 ? l >> 2 : 0, la = l ^ (b2 ? 7 : 0), b0 = la & 1, b1 = (la >> 1) & 1;
+  const int mb = DIM > 2 ? b2 : b1;  // the lane's end along the last axis
+  const T sg[3] = {b0 ? T(-1) : T(1), b1 ? T(-1) : T(1), b2 ? T(-1) : T(1)};
+  const double sd[3] = {b0 ? -1.0 : 1.0, b1 ? -1.0 : 1.0, b2 ? -1.0 : 1.0};
+  constexpr double G2 = 0.28867513459481288225;  // 1 / (2 sqrt 3)
+  const double S = (b0 ? G2 : 0.5) * (b1 ? G2 : 0.5) * (DIM > 2 ? (b2 ? G2 : 0.5) : 1.0);
+  // the stiffness of sums and differences along each axis, and their sum
+  double kap[4];
+  {
+    const double m0 = b0 ? KH[0] / 12.0 : KH[0] / 4.0, m1 = b1 ? KH[1] / 12.0 : KH[1] / 4.0;
+    const double m2 = DIM > 2 ? (b2 ? KH[2] / 12.0 : KH[2] / 4.0) : 1.0;
+    kap[0] = b0 ? m1 * m2 / KH[0] : 0.0;
+    kap[1] = b1 ? m0 * m2 / KH[1] : 0.0;
+    kap[2] = DIM > 2 && b2 ? m0 * m1 / KH[2] : 0.0;
+#if DCG_GEO
+#pragma unroll
+    for (int k = 0; k < DIM; ++k) kap[k] *= prm[6] * prm[3 + k] * prm[3 + k];
+#endif
+    kap[3] = kap[0] + kap[1] + kap[2];
+  }
+  double dp[NEP > 0 ? NEP : 1];
+  pair_diffusion(t, prm, dp);
+  const int ntx = (n0 + 1 + TX - 1) / TX;
+  const int nty = DIM > 2 ? (n1 + 1 + TY - 1) / TY : (n1 + 1 + TM - 1) / TM;
+  const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
+  const int vi0 = tx * TX - 1, vj0 = DIM > 2 ? ty * TY - 1 : 0, vm0 = (DIM > 2 ? tz : ty) * TM - 1;
+  const int nm = DIM > 2 ? n2 : n1;  // cells along the last axis
+  const int gi = vi0 + cx, gj = vj0 + cy;
+  const int gx = gi + b0, gy = DIM > 2 ? gj + b1 : 0;
+  const bool vin = gx >= 0 && gx <= n0 && gy >= 0 && gy <= (DIM > 2 ? n1 : 0);
+  const bool cin = gi >= 0 && gi < n0 && gj >= 0 && gj < (DIM > 2 ? n1 : 1);
+  const int vstep = DIM > 2 ? (n0 + 1) * (n1 + 1) : n0 + 1, cstep = DIM > 2 ? n0 * n1 : n0;
+  const int v00 = gx + (DIM > 2 ? (n0 + 1) * gy : 0), c00 = gi + (DIM > 2 ? n0 * gj : 0);
+  const double px = ox + (gi + (b0 ? 0.5 + G2 : 0.5 - G2)) * hx;
+  const double pyc = oy + (gj + (b1 ? 0.5 + G2 : 0.5 - G2)) * hy;
+  // row items of this thread: (vertex of the layer, species)
+  double d1 = 0.0, d2 = 0.0;
+  const int chunks = OP == 8 && full ? BC : 1;
+  for (int ch = 0; ch < chunks; ++ch) {
+    T carry[PER];
+#pragma unroll
+    for (int p = 0; p < PER; ++p) carry[p] = T(0);
+    for (int s = 0; s <= TM; ++s) {
+      const int k = vm0 + s;
+      if (k > nm) break;  // no vertex at or above this layer (uniform)
+      // the lane's corner
+      const int vk = k + mb;
+      int slot = -1;
+      if (vin && vk >= 0 && vk <= nm) {
+        const int vid = v00 + vstep * vk;
+        slot = g2l ? g2l[vid] : vid;
+      }
+      const bool on = cin && k >= 0 && k < nm && (cmask[c00 + cstep * k] & 1);
+      double u[BC];
+#pragma unroll
+      for (int i = 0; i < BC; ++i) u[i] = slot >= 0 ? x[(size_t)slot * DCG_B + i] : 0.0;
+      T vh[BC];
+      if constexpr (OP == 4)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) vh[i] = slot >= 0 ? v[(size_t)slot * DCG_B + i] : T(0);
+      double uh[OP == 1 ? BC : 1];
+      butterfly(u, sd);
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        if constexpr (OP == 1) uh[i] = u[i];
+        u[i] *= S;
+      }
+      butterfly(u, sd);
+      const double py = DIM > 2 ? pyc : oy + (k + (b1 ? 0.5 + G2 : 0.5 - G2)) * hy;
+      const double pz = DIM > 2 ? oz + (k + (b2 ? 0.5 + G2 : 0.5 - G2)) * hz : 0.0;
+      double rs[BC], rf[BC][DIM], g[BC][3], mc[NMC > 0 ? NMC : 1];
+#pragma unroll
+      for (int i = 0; i < BC; ++i) g[i][0] = g[i][1] = g[i][2] = 0.0;
+      if constexpr (OP == 1) qp(0, u, g, px, py, pz, t, cm, ca, rs, rf, nullptr, nullptr, nullptr, prm, nullptr);
+      else qp(0, u, g, px, py, pz, t, cm, ca, rs, rf, mc, nullptr, nullptr, prm, nullptr);
+      T o[BC];
+      if constexpr (OP == 1) {
+#pragma unroll
+        for (int i = 0; i < BC; ++i) o[i] = rs[i];
+        butterfly(o, sg);
+#pragma unroll
+        for (int i = 0; i < BC; ++i) o[i] *= S;
+#pragma unroll
+        for (int n = 0; n < NEP; ++n) o[EPI[n]] += ca * dp[n] * (kap[EPK[n]] * uh[EPJ[n]]);
+        butterfly(o, sg);
+      } else if constexpr (OP == 4) {
+        butterfly(vh, sg);
+        T q[BC];
+#pragma unroll
+        for (int i = 0; i < BC; ++i) q[i] = T(S) * vh[i];
+        butterfly(q, sg);
+        point_block(mc, q, o);
+        butterfly(o, sg);
+#pragma unroll
+        for (int i = 0; i < BC; ++i) o[i] *= T(S);
+#pragma unroll
+        for (int n = 0; n < NEP; ++n) o[EPI[n]] += T(ca * dp[n] * kap[EPK[n]]) * vh[EPJ[n]];
+        butterfly(o, sg);
+      } else {
+        // entries (j, j), or row ch of the block; the squared basis functions
+        // have weights 1/3 and 1/(2 sqrt 3) in sums and differences
+#pragma unroll
+        for (int j = 0; j < BC; ++j) o[j] = T(0);
+#pragma unroll
+        for (int n = 0; n < NMC; ++n)
+          if (full ? MCI[n] == ch : MCI[n] == MCJ[n]) o[MCJ[n]] += mc[n];
+        butterfly(o, sg);
+        const double S2 = (b0 ? G2 : 1.0 / 3.0) * (b1 ? G2 : 1.0 / 3.0) * (DIM > 2 ? (b2 ? G2 : 1.0 / 3.0) : 1.0);
+#pragma unroll
+        for (int j = 0; j < BC; ++j) o[j] *= S2;
+        butterfly(o, sg);
+        double kd[4];
+        kd[0] = KH[1] * (DIM > 2 ? KH[2] / 3.0 : 1.0) / (3.0 * KH[0]);
+        kd[1] = KH[0] * (DIM > 2 ? KH[2] / 3.0 : 1.0) / (3.0 * KH[1]);
+        kd[2] = DIM > 2 ? KH[0] * KH[1] / (9.0 * KH[2]) : 0.0;
+#if DCG_GEO
+#pragma unroll
+        for (int k2 = 0; k2 < DIM; ++k2) kd[k2] *= prm[6] * prm[3 + k2] * prm[3 + k2];
+#endif
+        kd[3] = kd[0] + kd[1] + kd[2];
+#pragma unroll
+        for (int n = 0; n < NEP; ++n)
+          if (full ? EPI[n] == ch : EPI[n] == EPJ[n]) o[EPJ[n]] += ca * dp[n] * kd[EPK[n]];
+      }
+#pragma unroll
+      for (int i = 0; i < BC; ++i) out[i * NT + tid] = on ? o[i] : T(0);
+      __syncthreads();
+#pragma unroll
+      for (int p = 0; p < PER; ++p) {
+        const int it = tid + p * NT, row = it / DCG_B, i = it % DCG_B;
+        const int rx = row % TX, ry = row / TX;
+        const int wx = vi0 + 1 + rx, wy = DIM > 2 ? vj0 + 1 + ry : 0;
+        if (row >= TL::ROWS || wx > n0 || wy > (DIM > 2 ? n1 : 0)) continue;
+        T low = T(0), up = T(0);
+        if (i < BC) {
+#pragma unroll
+          for (int ey = 0; ey < (DIM > 2 ? 2 : 1); ++ey)
+#pragma unroll
+            for (int ex = 0; ex < 2; ++ex) {
+              const int c = (rx + ex) + CX * (ry + ey);
+              const int e = (1 - ex) | (DIM > 2 ? (1 - ey) << 1 : 0);  // the vertex's corner, lower layer end
+              const T* oc = out + i * NT + c * NCORNER;
+              low += oc[e];
+              up += oc[DIM > 2 ? e ^ 7 : e | 2];
+            }
+        }
+        const T sum = carry[p] + low;
+        carry[p] = up;
+        if (s == 0) continue;  // the layer below the tile's rows
+        const int vid = wx + (DIM > 2 ? (n0 + 1) * wy : 0) + vstep * k;
+        const int sr = g2l ? g2l[vid] : vid;
+        if (sr < 0) continue;
+        const size_t at = (size_t)sr * DCG_B + i;
+        if constexpr (OP == 8) {
+          auto blk = y + (size_t)sr * (DCG_B * DCG_B);
+          if (full) {
+            if (i < BC) blk[ch * DCG_B + i] = sum;
+            else blk[ch * DCG_B + i] = T(0);
+            if (ch == 0 && i >= BC)
+              for (int j = 0; j < DCG_B; ++j) blk[i * DCG_B + j] = i == j ? T(1) : T(0);
+          } else {
+            for (int j = 0; j < DCG_B; ++j) blk[i * DCG_B + j] = i == j ? (i < BC ? sum : T(1)) : T(0);
+          }
+          if (ch == 0) lin[at] = x[at];
+        } else if constexpr (OP == 1) {
+          const T b = v ? v[at] : T(0);  // the vector passed as v is the base
+          y[at] = b + (i < BC ? sum : T(0));
+        } else {
+          const T acc = i < BC ? sum : v[at];  // padding species: identity rows
+          y[at] = acc;
+          if (part) {
+            d1 += (double)acc * (double)(w1 == y ? acc : w1[at]);
+            if (w2) d2 += (double)acc * (double)(w2 == y ? acc : w2[at]);
+          }
+        }
+      }
+      __syncthreads();
+    }
+  }
+  if constexpr (OP == 4) {
+    if (part) {
+      // workgroup sums of the two partial dots (fixed order)
+      __shared__ double red[2 * (NT / 64)];
+#pragma unroll
+      for (int o2 = 32; o2 > 0; o2 >>= 1) {
+        d1 += __shfl_down(d1, o2, 64);
+        d2 += __shfl_down(d2, o2, 64);
+      }
+      if ((tid & 63) == 0) {
+        red[2 * (tid >> 6)] = d1;
+        red[2 * (tid >> 6) + 1] = d2;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        double a = 0.0, b = 0.0;
+        for (int k = 0; k < NT / 64; ++k) {
+          a += red[2 * k];
+          b += red[2 * k + 1];
+        }
+        part[0] = a;
+        part[1] = b;
+      }
+    }
+  }
+}
+}  // namespace %C%
+
+extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
+%KERNEL%_r(const int* __restrict__ tiles, const int* __restrict__ g2l, const unsigned char* __restrict__ cmask,
+           const double* __restrict__ x, const double* base, double t, double cm, double ca, double* r,
+           double* __restrict__ val, const int* __restrict__ own_start, const unsigned* __restrict__ own_mask, int n0,
+           int n1, int n2, double ox, double oy, double oz, double hx, double hy, double hz, int mode,
+           const double* __restrict__ prm, const int* __restrict__ stop) {
+  %C%::corner_body<%C%::CornerShape0, 1, double>(
+      tiles[blockIdx.x], (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,
+      (%C%::dcg_gp<const double>)x, (%C%::dcg_gp<const double>)base, (%C%::dcg_gp<double>)r, nullptr, t, cm, ca, n0, n1,
+      n2, ox, oy, oz, hx, hy, hz, prm, false, nullptr, nullptr, nullptr);
+}
+)";
+
+// the corner form of the point-storage entry points (kTiledPoints): pc is the
+// linearisation point, tca = (t, ca, cm, origin, spacing) as the set-up left it
+const char* kCornerPoints = R"(
+extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
+%KERNEL%_q(const int* __restrict__ tiles, const int* __restrict__ g2l, const unsigned char* __restrict__ cmask,
+           const double* x, const double* __restrict__ base, double t, double cm, double ca, double* __restrict__ r,
+           double* lin, const int* __restrict__ own_start, const unsigned* __restrict__ own_mask, int n0, int n1,
+           int n2, double ox, double oy, double oz, double hx, double hy, double hz, int mode,
+           const double* __restrict__ prm, double* __restrict__ tca) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) %C%::set_tca(tca, t, ca, cm, ox, oy, oz, hx, hy, hz);
+  %C%::corner_body<%C%::CornerShape0, 8, double>(
+      tiles[blockIdx.x], (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,
+      (%C%::dcg_gp<const double>)x, nullptr, (%C%::dcg_gp<double>)r, (%C%::dcg_gp<double>)lin, t, cm, ca, n0, n1, n2,
+      ox, oy, oz, hx, hy, hz, prm, (mode & 16) != 0, nullptr, nullptr, nullptr);
+}
+#define DCG_CORNER_ENTRY(NAME, T, TL)                                                                             \
+  extern "C" __global__ void __launch_bounds__(TL::NT)                                                            \
+  NAME(const int* __restrict__ tiles, int ntile, const int* __restrict__ g2l,                                     \
+       const unsigned char* __restrict__ cmask, const double* __restrict__ lin, const T* __restrict__ v,           \
+       T* __restrict__ y, const double* __restrict__ tca, int n0, int n1, int n2, const double* __restrict__ prm,  \
+       const int* __restrict__ stop, const T* w1, const T* w2, double* __restrict__ part) {                       \
+    if (stop && *stop) return;                                                                                    \
+    const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
+    if (c >= ntile) return;                                                                                       \
+    %C%::corner_body<TL, 4, T>(tiles[c], (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,    \
+                               (%C%::dcg_gp<const double>)lin, (%C%::dcg_gp<const T>)v, (%C%::dcg_gp<T>)y,         \
+                               nullptr, tca[0], tca[2], tca[1], n0, n1, n2, tca[3], tca[4], tca[5], tca[6],       \
+                               tca[7], tca[8], prm, false, (%C%::dcg_gp<const T>)w1, (%C%::dcg_gp<const T>)w2,    \
+                               part ? part + 2 * (size_t)c : nullptr);                                            \
+  }
+%CORNER_ENTRIES%
+#undef DCG_CORNER_ENTRY
+)";
+
+// batched residual, set-up and apply of the corner form (as kTiledBatch and
+// kTiledPointBatch)
+const char* kCornerBatch = R"(
+extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
+%KERNEL%_rbatch(const int2* __restrict__ work, const dcg_asm_member* __restrict__ mem,
+                const double* __restrict__ coef, const int* __restrict__ act, int xsel, int bsel, int rsel, int mode) {
+  const int2 w = work[blockIdx.x];
+  if (act && !act[w.x]) return;
+  const double* cf = coef + 4 * (size_t)w.x;
+  if (cf[3] == 0.0) return;
+  const dcg_asm_member& M = mem[w.x];
+  using GX = %C%::dcg_gp<const double>;
+  %C%::corner_body<%C%::CornerShape0, 1, double>(
+      w.y, (%C%::dcg_gp<const int>)M.g2l[%COMP%], (%C%::dcg_gp<const unsigned char>)M.cmask[%COMP%],
+      (GX)M.vec[xsel], bsel >= 0 ? (GX)M.vec[bsel] : (GX) nullptr, (%C%::dcg_gp<double>)M.vec[rsel], nullptr, cf[0],
+      cf[1], cf[2], M.n[0], M.n[1], M.n[2], M.origin[0], M.origin[1], M.origin[2], M.h[0], M.h[1], M.h[2], M.prm,
+      false, nullptr, nullptr, nullptr);
+}
+)";
+
+const char* kCornerPointBatch = R"(
+extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
+%KERNEL%_qbatch(const int2* __restrict__ work, const dcg_asm_member* __restrict__ mem,
+                const double* __restrict__ coef, const int* __restrict__ act, int xsel, int full) {
+  const int2 w = work[blockIdx.x];
+  if (act && !act[w.x]) return;
+  const double* cf = coef + 4 * (size_t)w.x;
+  if (cf[3] == 0.0) return;
+  const dcg_asm_member& M = mem[w.x];
+  if (threadIdx.x == 0)  // every workgroup of the member writes the same values
+    %C%::set_tca(M.tca, cf[0], cf[2], cf[1], M.origin[0], M.origin[1], M.origin[2], M.h[0], M.h[1], M.h[2]);
+  %C%::corner_body<%C%::CornerShape0, 8, double>(
+      w.y, (%C%::dcg_gp<const int>)M.g2l[%COMP%], (%C%::dcg_gp<const unsigned char>)M.cmask[%COMP%],
+      (%C%::dcg_gp<const double>)M.vec[xsel], nullptr, (%C%::dcg_gp<double>)M.pdiag,
+      (%C%::dcg_gp<double>)M.pc[%COMP%], cf[0], cf[1], cf[2], M.n[0], M.n[1], M.n[2], M.origin[0], M.origin[1],
+      M.origin[2], M.h[0], M.h[1], M.h[2], M.prm, full != 0, nullptr, nullptr, nullptr);
+}
+#define DCG_CORNER_BENTRY(NAME, T, VEC, TL)                                                                       \
+  extern "C" __global__ void __launch_bounds__(TL::NT)                                                            \
+  NAME(const int2* __restrict__ work, int nwork, int part_off, const dcg_pc_member* __restrict__ mem, int xsel,   \
+       int ysel, int w1sel, int w2sel, int skip, double* __restrict__ part) {                                      \
+    const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
+    if (c >= nwork) return;                                                                                       \
+    const int2 w = work[c];                                                                                       \
+    const dcg_pc_member& M = mem[w.x];                                                                            \
+    if (skip == 0 && *M.done) return;                                                                             \
+    if (skip == 1 && *M.irdone) return;                                                                           \
+    using GT = %C%::dcg_gp<const T>;                                                                              \
+    const double* tca = M.tca;                                                                                    \
+    %C%::corner_body<TL, 4, T>(w.y, (%C%::dcg_gp<const int>)M.g2l, (%C%::dcg_gp<const unsigned char>)M.cmask,    \
+                               (%C%::dcg_gp<const double>)M.pc, (GT)M.VEC[xsel], (%C%::dcg_gp<T>)M.VEC[ysel],     \
+                               nullptr, tca[0], tca[2], tca[1], M.n[0], M.n[1], M.n[2], tca[3], tca[4], tca[5],   \
+                               tca[6], tca[7], tca[8], M.prm, false, w1sel >= 0 ? (GT)M.VEC[w1sel] : nullptr,     \
+                               w2sel >= 0 ? (GT)M.VEC[w2sel] : nullptr,                                           \
+                               part ? part + 2 * (size_t)(part_off + c) : nullptr);                               \
+  }
+%CORNER_BENTRIES%
+#undef DCG_CORNER_BENTRY
+)";
+
 }  // namespace
 
-int apply_tile_threads(int dim, std::array<int, 3> t, int species) {
+int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner) {
+  // corner form: a lane per corner of a layer's cells
+  if (corner) return (t[0] + 1) * (dim > 2 ? t[1] + 1 : 1) << dim;
   // one cell of the cell box per thread (corner sums scattered in LDS) for
   // blocks of up to 4 species; larger blocks loop over the cells
   int ncb = t[0] + 1;
@@ -2206,6 +2614,48 @@ int apply_tile_threads(int dim, std::array<int, 3> t, int species) {
   if (dim > 2) ncb *= t[2] + 1;
   if (species > 4 || ncb <= 256 || ncb > 1024) return 256;
   return ncb <= 512 ? 512 : 1024;
+}
+
+// The corner form's tile shapes: layers of 8 x 8 (4 x 8) cells in 3D and of
+// 64 (32) in a row in 2D, so that a layer fills 512 (256) lanes.  The first
+// one also serves the residual and the set-up.
+std::vector<std::array<int, 3>> corner_tiles(int dim) {
+  if (dim == 3) return {{7, 7, 7}, {7, 3, 7}};
+  return {{63, 15, 1}, {31, 7, 1}};
+}
+
+// The corner form takes box cells in 2D and 3D whose equations suit the tiled
+// kernel (tile_eligible), with diffusion tensors diagonal in space (the sums
+// and differences of a cell's corners diagonalise no mixed derivatives) and
+// reactions that read no gradients, in blocks of more than 4 species: there
+// the tiled kernels keep a cell's corner values in LDS (40^3, 7 species:
+// residual 360 us, Jacobian pass 3,330 us).  Up to 4 species a thread holds a
+// whole cell in registers, without the lane exchanges.
+bool corner_eligible(const ModelSpec& m, const Grid& g, int comp) {
+  if (g.unstructured || !g.cube || g.dim < 2 || m.comp_species[comp].size() <= 4 || !tile_eligible(m, comp))
+    return false;
+  auto gradient_free = [](const Ex& e) {
+    if (!e) return true;
+    std::vector<std::string> vars;
+    expr::collect_vars(e, vars);
+    for (const auto& v : vars)
+      if (v.rfind("grad_", 0) == 0) return false;
+    return true;
+  };
+  for (int s : m.comp_species[comp]) {
+    const auto& sp = m.species[s];
+    if (!gradient_free(sp.storage) || !gradient_free(sp.reaction)) return false;
+    for (const auto& pj : sp.storage_jac)
+      if (!gradient_free(pj.e)) return false;
+    for (const auto& pj : sp.reaction_jac)
+      if (!gradient_free(pj.e)) return false;
+    for (const auto& dt : sp.diffusion)
+      if (dt.D.tensor)
+        for (int k = 0; k < 3; ++k)
+          for (int l = 0; l < 3; ++l)
+            if (k != l && dt.D.d[k][l]) return false;
+  }
+  return true;
 }
 
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
@@ -2267,7 +2717,7 @@ std::array<int, 3> choose_tile(const Grid& g, int bc, int nmc) {
 }
 
 std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::string& ns, const std::string& kname,
-                      std::array<int, 3> tile, bool geo, bool points,
+                      std::array<int, 3> tile, bool geo, bool points, bool corner,
                       const std::vector<std::array<int, 3>>& apply_tiles, const std::vector<int>& apply_waves) {
   const auto T = element_tables(geo ? unit_cell(g) : g);
   std::ostringstream o;
@@ -2387,10 +2837,71 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
   o << "}\n";
   o << "}  // namespace " << ns << "\n";
   std::string body = kTiled;
-  if (points) body += kTiledPoints;
   if (geo && comp < 4) body += kTiledBatch;
-  if (geo && comp < 4 && points) body += kTiledPointBatch;
-  {
+  replace_all(body, "%R_ENTRY%", corner ? "" : "DCG_TILE_ENTRY(%KERNEL%_r, 1)\n");
+  if (corner) {
+    body += kCorner;
+    if (points) body += kCornerPoints;
+    if (geo && comp < 4) body += kCornerBatch;
+    if (geo && comp < 4 && points) body += kCornerPointBatch;
+    const auto shapes = corner_tiles(d);
+    std::string cs, ce, cb;
+    for (size_t k2 = 0; k2 < shapes.size(); ++k2) {
+      const std::string id = std::to_string(k2), tl = ns + "::CornerShape" + id;
+      cs += "using CornerShape" + id + " = CornerTile<" + std::to_string(shapes[k2][0]) + ", " +
+            std::to_string(shapes[k2][1]) + ", " + std::to_string(shapes[k2][2]) + ">;\n";
+      ce += "DCG_CORNER_ENTRY(%KERNEL%_p" + id + ", double, " + tl + ")\n";
+      ce += "DCG_CORNER_ENTRY(%KERNEL%_pf" + id + ", float, " + tl + ")\n";
+      cb += "DCG_CORNER_BENTRY(%KERNEL%_pbatch" + id + ", double, v, " + tl + ")\n";
+      cb += "DCG_CORNER_BENTRY(%KERNEL%_pfbatch" + id + ", float, f, " + tl + ")\n";
+    }
+    // diffusion per species pair: D_ij of an isotropic term (axis 3: all
+    // axes) or of each axis; KH: the cell's sides (1: run-time spacing)
+    std::ostringstream ct;
+    std::vector<int> pi, pj, pk;
+    std::vector<std::string> pe;
+    for (size_t i = 0; i < species.size(); ++i)
+      for (const auto& dt : m.species[species[i]].diffusion)
+        for (int k2 = 0; k2 < (dt.D.tensor ? d : 1); ++k2) {
+          Ex e = dt.D.tensor ? dt.D.d[k2][k2] : dt.D.d[0][0];
+          if (!e) continue;
+          pi.push_back(static_cast<int>(i));
+          pj.push_back(m.species[dt.wrt].local);
+          pk.push_back(dt.D.tensor ? k2 : 3);
+          pe.push_back(expr::emit(e, vars));
+        }
+    std::vector<double> kh(3, 1.0);
+    for (int k2 = 0; k2 < d && !geo; ++k2) kh[k2] = g.h[k2];
+    ct << "__device__ constexpr double KH[3] = " << array_init(kh) << ";\n";
+    ct << "constexpr int NEP = " << pi.size() << ";\n";
+    ct << "__device__ constexpr int EPI[NEP > 0 ? NEP : 1] = " << ints(pi) << ";\n";
+    ct << "__device__ constexpr int EPJ[NEP > 0 ? NEP : 1] = " << ints(pj) << ";\n";
+    ct << "__device__ constexpr int EPK[NEP > 0 ? NEP : 1] = " << ints(pk) << ";\n";
+    // o = (point block) q, one statement per entry, in FP64 as the block is
+    // (FP64 FMAs run at the FP32 rate; converting every entry would cost more)
+    ct << "template <typename T>\n__device__ __forceinline__ void point_block(const double (&mc)[NMC > 0 ? NMC : 1], "
+          "const T (&q)[BC], T (&o)[BC]) {\n  (void)mc; (void)q;\n";
+    for (size_t i = 0; i < species.size(); ++i) {
+      ct << "  {\n    double s = 0.0;\n";
+      for (size_t n = 0; n < nz.size(); ++n)
+        if (nz[n].first == static_cast<int>(i)) ct << "    s += mc[" << n << "] * (double)q[" << nz[n].second << "];\n";
+      ct << "    o[" << i << "] = T(s);\n  }\n";
+    }
+    ct << "}\n";
+    ct << "__device__ __forceinline__ void pair_diffusion(double t, const double* __restrict__ prm, "
+          "double (&dp)[NEP > 0 ? NEP : 1]) {\n  (void)t; (void)prm; dp[0] = 0.0;\n";
+    for (size_t n = 0; n < pe.size(); ++n) ct << "  dp[" << n << "] = " << pe[n] << ";\n";
+    ct << "}\n__device__ __forceinline__ void set_tca(double* tca, double t, double ca, double cm, double ox, double oy, "
+          "double oz, double hx, double hy, double hz) {\n  tca[0] = t; tca[1] = ca; tca[2] = cm; tca[3] = ox; "
+          "tca[4] = oy; tca[5] = oz; tca[6] = hx; tca[7] = hy; tca[8] = hz;\n}\n";
+    replace_all(body, "%CORNER_TABLES%", ct.str());
+    replace_all(body, "%CORNER_SHAPES%", cs);
+    replace_all(body, "%CORNER_ENTRIES%", ce);
+    replace_all(body, "%CORNER_BENTRIES%", cb);
+    replace_all(body, "%APPLY_SHAPES%", "");
+  } else {
+    if (points) body += kTiledPoints;
+    if (geo && comp < 4 && points) body += kTiledPointBatch;
     // one point apply (and batched point apply) per candidate tile shape k:
     // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k>
     std::string pe, pb;
@@ -2407,7 +2918,8 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     for (size_t k2 = 0; k2 < apply_tiles.size(); ++k2)
       as += "using ApplyShape" + std::to_string(k2) + " = ApplyTile<" + std::to_string(apply_tiles[k2][0]) + ", " +
             std::to_string(apply_tiles[k2][1]) + ", " + std::to_string(apply_tiles[k2][2]) + ", " +
-            std::to_string(apply_tile_threads(g.dim, apply_tiles[k2], static_cast<int>(m.comp_species[comp].size()))) +
+            std::to_string(apply_tile_threads(g.dim, apply_tiles[k2], static_cast<int>(m.comp_species[comp].size()),
+                                              false)) +
             ", " + std::to_string(k2 < apply_waves.size() ? apply_waves[k2] : 1) + ">;\n";
     replace_all(body, "%APPLY_SHAPES%", as);
     replace_all(body, "%POINT_ENTRIES%", pe);
@@ -2440,6 +2952,8 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       out.tile_batch_kernel.push_back("");
       out.tile_dims.push_back({0, 0, 0});
       out.point_words.push_back(0);
+      out.corner.push_back(0);
+      out.apply_threads.push_back({});
       continue;
     }
     std::string ns = "vol" + std::to_string(c);
@@ -2451,20 +2965,29 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       auto tile = choose_tile(L.grid, static_cast<int>(spec.comp_species[c].size()),
                               static_cast<int>(mc_pattern(spec, static_cast<int>(c)).size()));
       std::string tk = "dcg_tile_" + std::to_string(c);
-      std::vector<int> waves;
-      const auto shapes = points ? apply_tile_candidates(L.grid, static_cast<int>(spec.comp_species[c].size()), tile,
-                                                         &waves)
-                                 : std::vector<std::array<int, 3>>{};
-      src << gen_tiled(spec, L.grid, static_cast<int>(c), ns, tk, tile, geo, points, shapes, waves);
+      std::vector<int> waves, threads;
+      const int nsp = static_cast<int>(spec.comp_species[c].size());
+      const bool corner = corner_eligible(spec, L.grid, static_cast<int>(c));
+      std::vector<std::array<int, 3>> shapes;
+      if (points && corner) {
+        shapes = corner_tiles(L.grid.dim);
+        waves.assign(shapes.size(), 1);
+      } else if (points) {
+        shapes = apply_tile_candidates(L.grid, nsp, tile, &waves);
+      }
+      for (const auto& t : shapes) threads.push_back(apply_tile_threads(L.grid.dim, t, nsp, corner));
+      src << gen_tiled(spec, L.grid, static_cast<int>(c), ns, tk, tile, geo, points, corner, shapes, waves);
+      out.corner.push_back(corner ? 1 : 0);
+      out.apply_threads.push_back(threads);
       out.tile_kernel.push_back(tk);
       out.apply_tiles.push_back(shapes);
       out.apply_waves.push_back(waves);
       out.tile_batch_kernel.push_back(geo && c < 4 ? tk + "_batch" : "");
       out.tile_dims.push_back(tile);
       const int nq = static_cast<int>(element_rule(L.grid.dim, L.grid.cube).w.size());
-      out.point_words.push_back(points ? L.grid.nclass * nq *
-                                             static_cast<int>(mc_pattern(spec, static_cast<int>(c)).size())
-                                       : 0);
+      out.point_words.push_back(points && !corner ? L.grid.nclass * nq *
+                                                        static_cast<int>(mc_pattern(spec, static_cast<int>(c)).size())
+                                                  : 0);
     } else {
       out.tile_kernel.push_back("");
       out.apply_tiles.push_back({});
@@ -2472,6 +2995,8 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       out.tile_batch_kernel.push_back("");
       out.tile_dims.push_back({0, 0, 0});
       out.point_words.push_back(0);
+      out.corner.push_back(0);
+      out.apply_threads.push_back({});
     }
   }
   // facet kernels for every (in, out, boundary) combination present

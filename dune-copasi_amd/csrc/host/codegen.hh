@@ -40,8 +40,13 @@ struct GeneratedSource {
   // <tile_kernel>_p<k>, _pf<k> and the batched _pbatch<k>, _pfbatch<k>);
   // the first is the assembly tile
   std::vector<std::vector<std::array<int, 3>>> apply_tiles;
-  // per compartment and candidate: the waves per SIMD its registers are bounded for (1: none)
-  std::vector<std::vector<int>> apply_waves;
+  // per compartment and candidate: the waves per SIMD its registers are
+  // bounded for (1: none), and the workgroup size
+  std::vector<std::vector<int>> apply_waves, apply_threads;
+  // compartments in the corner form: the residual and the point set-up run
+  // over corner_tiles(dim).front(), and the point applies evaluate their
+  // coefficients at the linearisation point (no stored words)
+  std::vector<char> corner;
   std::vector<FacetKernel> facet_kernels;
 };
 
@@ -58,8 +63,11 @@ bool tile_eligible(const ModelSpec& m, int comp);
 // tile shapes the point apply is generated for (the set-up tile first)
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
                                                       std::vector<int>* waves = nullptr);
-// workgroup size of the point apply with tile t (cells per workgroup along x, y, z)
-int apply_tile_threads(int dim, std::array<int, 3> t, int species);
+// workgroup size of the point apply with tile t (row vertices along x, y, z)
+int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner);
+// the compartment's kernels take the corner form, and its tile shapes
+bool corner_eligible(const ModelSpec& m, const Grid& g, int comp);
+std::vector<std::array<int, 3>> corner_tiles(int dim);
 
 // points: also emit the point-coefficient Jacobian entry points (_q, _p, _pf)
 // of every tiled compartment

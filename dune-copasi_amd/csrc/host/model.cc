@@ -206,11 +206,14 @@ void Model::build(const std::string& ini, const std::string& overrides) {
     else if (cfg_.precond == Preconditioner::ILU0) why = "an ILU0 preconditioner";
     else if (!all_tile_eligible()) why = "compartments outside the tiled kernel";
     if (st == "points" && !why.empty()) throw NotImplemented("linear_solver.storage = points with " + why);
-    // auto: box cells, and blocks of up to 4 species (larger blocks keep their
-    // corner sums in LDS, where the assembled SpMV is still faster)
-    int bmax = 0;
-    for (const auto& C : L_.comps) bmax = std::max(bmax, C.b);
-    cfg_.points = why.empty() && (st == "points" || (st == "auto" && L_.grid.cube && bmax <= 4));
+    // auto: box cells, with blocks of up to 4 species or in the corner form
+    // (40^3, 7 species, FP32 operator: apply 27 us against 83 us for the
+    // SpMV, and no Jacobian pass of 3.3 ms; larger blocks outside the corner
+    // form keep their corner sums in LDS, where the SpMV is faster)
+    bool suits = L_.grid.cube;
+    for (size_t c = 0; c < L_.comps.size(); ++c)
+      suits = suits && (L_.comps[c].b <= 4 || corner_eligible(spec_, L_.grid, static_cast<int>(c)));
+    cfg_.points = why.empty() && (st == "points" || (st == "auto" && suits));
   }
   {
     const std::string pt = c.get(p + "linear_solver.point_tile", std::string("auto"));
@@ -258,6 +261,12 @@ bool Model::all_tile_eligible() const {
   for (size_t c = 0; c < L_.comps.size(); ++c)
     if (L_.comps[c].b && !tile_eligible(spec_, static_cast<int>(c))) return false;
   return true;
+}
+
+bool Model::any_corner() const {
+  for (char c : gen_.corner)
+    if (c) return true;
+  return false;
 }
 
 bool Model::can_apply_jacobian() const {
@@ -382,6 +391,11 @@ void Model::setup_device() {
     comp_dev_[c].cell_mask_grid.upload(cm, stream_);
     comp_dev_[c].tiles.upload(tiles, stream_);
     comp_dev_[c].ntiles = static_cast<int>(tiles.size());
+    if (gen_.corner[c]) {
+      const auto rt = tile_list(corner_tiles(gr.dim).front());
+      comp_dev_[c].rtiles.upload(rt, stream_);
+      comp_dev_[c].nrtiles = static_cast<int>(rt.size());
+    }
   }
   {
     // blocks outside a row's own-compartment run couple two compartments
@@ -496,8 +510,9 @@ void Model::setup_device() {
       if (cfg_.precision == Precision::Mixed) pc32_[c].resize(words);
     }
     pdiag_.resize(static_cast<size_t>(ns) * B * B);
-    pc_tca_.resize(2);
-    if (!L_.facets.empty()) lin_x_.resize(nv);  // the facet terms apply from the linearisation point
+    pc_tca_.resize(kTca);
+    // the facet terms and the corner form apply from the linearisation point
+    if (!L_.facets.empty() || any_corner()) lin_x_.resize(nv);
     dinv_.resize(static_cast<size_t>(ns) * B * B);
     std::vector<int> id(ns);
     for (long i = 0; i < ns; ++i) id[i] = static_cast<int>(i);
@@ -673,7 +688,8 @@ void Model::tune_points() {
       pc_bytes += a.size() * sizeof(double);
     }
   for (int i = 0; i < 4; ++i) k::fill(kv_[i].get(), 0.0, L_.nslot * L_.B, stream_);
-  k::fill(pc_tca_.get(), 0.0, 2, stream_);
+  k::fill(pc_tca_.get(), 0.0, static_cast<long>(kTca), stream_);
+  if (any_corner()) k::fill(lin_x_.get(), 0.0, L_.nslot * L_.B, stream_);
   // the eviction copy: only where the coefficients could stay cached
   constexpr long kFlushBytes = 384L << 20;
   DeviceArray<char> fa, fb;
@@ -802,10 +818,15 @@ void Model::launch_assembly(const double* x, double t, double cm, double ca, con
       for (int part : {1, 2}) {
         if (!(mode & part) || comp_dev_[c].ntiles <= 0) continue;
         int pmode = part;
-        void* args[] = {&tiles, &g2l, &cmask, &x, &base_eff, &t, &cm, &ca, &r, &val, &own_start, &own_mask,
+        const bool corner = part == 1 && gen_.corner[c];
+        const int* list = corner ? comp_dev_[c].rtiles.get() : tiles;
+        const unsigned grid = static_cast<unsigned>(corner ? comp_dev_[c].nrtiles : comp_dev_[c].ntiles);
+        const unsigned block = static_cast<unsigned>(
+            corner ? apply_tile_threads(g.dim, corner_tiles(g.dim).front(), C.b, true) : 256);
+        void* args[] = {&list, &g2l, &cmask, &x, &base_eff, &t, &cm, &ca, &r, &val, &own_start, &own_mask,
                         &n0, &n1, &n2, &ox, &oy, &oz, &hx, &hy, &hz, &pmode, &prm, &stop};
-        DCG_HIP(hipModuleLaunchKernel(part == 1 ? tile_fn_[c] : tile_jac_fn_[c], comp_dev_[c].ntiles, 1, 1, 256, 1, 1,
-                                      0, stream_, args, nullptr));
+        DCG_HIP(hipModuleLaunchKernel(part == 1 ? tile_fn_[c] : tile_jac_fn_[c], grid, 1, 1, block, 1, 1, 0, stream_,
+                                      args, nullptr));
       }
       continue;
     }
@@ -893,18 +914,23 @@ void Model::launch_points_setup(const double* x, double t, double cm, double ca)
   const unsigned* own_mask = own_mask_.get();
   const double* prm = prm_.get();
   const double* base = nullptr;
-  const int* stop = nullptr;
+  double* tca = pc_tca_.get();
   double* diag = pdiag_.get();
-  int mode = 8;
+  // 16: the corner form writes whole blocks, not their diagonals alone
+  int mode = 8 | (cfg_.precond == Preconditioner::VertexBlockJacobi ? 16 : 0);
   for (size_t c = 0; c < L_.comps.size(); ++c) {
     if (!pc_set_fn_[c] || comp_dev_[c].ntiles <= 0) continue;
-    const int* tiles = comp_dev_[c].tiles.get();
+    const bool corner = gen_.corner[c];
+    const int* tiles = corner ? comp_dev_[c].rtiles.get() : comp_dev_[c].tiles.get();
+    const unsigned grid = static_cast<unsigned>(corner ? comp_dev_[c].nrtiles : comp_dev_[c].ntiles);
+    const unsigned block = static_cast<unsigned>(
+        corner ? apply_tile_threads(g.dim, corner_tiles(g.dim).front(), L_.comps[c].b, true) : 256);
     const int* g2l = comp_dev_[c].g2l.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
-    double* pc = pc_[c].get();
+    double* pc = corner ? lin_x_.get() : pc_[c].get();
     void* args[] = {&tiles, &g2l, &cmask, &x, &base, &t, &cm, &ca, &diag, &pc, &own_start, &own_mask,
-                    &n0, &n1, &n2, &ox, &oy, &oz, &hx, &hy, &hz, &mode, &prm, &stop};
-    DCG_HIP(hipModuleLaunchKernel(pc_set_fn_[c], comp_dev_[c].ntiles, 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
+                    &n0, &n1, &n2, &ox, &oy, &oz, &hx, &hy, &hz, &mode, &prm, &tca};
+    DCG_HIP(hipModuleLaunchKernel(pc_set_fn_[c], grid, 1, 1, block, 1, 1, 0, stream_, args, nullptr));
   }
   k::fill(pc_tca_.get(), t, 1, stream_);
   k::fill(pc_tca_.get() + 1, ca, 1, stream_);
@@ -947,7 +973,9 @@ int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp3
     if (!pc_app_fn_[c] || comp_dev_[c].ntiles <= 0) continue;
     const int* g2l = comp_dev_[c].g2l_identity ? nullptr : comp_dev_[c].g2l.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
-    const void* pc = fp32 ? static_cast<const void*>(pc32_[c].get()) : static_cast<const void*>(pc_[c].get());
+    const void* pc = gen_.corner[c] ? static_cast<const void*>(lin_x_.get())
+                     : fp32         ? static_cast<const void*>(pc32_[c].get())
+                                    : static_cast<const void*>(pc_[c].get());
     double* pp = part && facet_fn_.empty() ? part + 2 * static_cast<size_t>(nparts) : nullptr;
     // the apply's own tile shape (chosen at set-up) and its tile list
     const int k2 = apply_shape_[c];
@@ -955,8 +983,7 @@ int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp3
     int ntile = comp_dev_[c].natiles[k2];
     void* args[] = {&tiles, &ntile, &g2l, &cmask, &pc, &v, &y, &tca, &n0, &n1, &n2, &prm, &stop, &w1, &w2, &pp};
     const unsigned grid = static_cast<unsigned>((ntile + 7) / 8 * 8);  // the kernel maps workgroups to XCD runs
-    const unsigned nt = static_cast<unsigned>(
-        apply_tile_threads(L_.grid.dim, gen_.apply_tiles[c][k2], L_.comps[c].b));
+    const unsigned nt = static_cast<unsigned>(gen_.apply_threads[c][k2]);
     DCG_HIP(hipModuleLaunchKernel(fp32 ? pc_appf_fns_[c][k2] : pc_app_fns_[c][k2], grid, 1, 1, nt, 1, 1, 0, stream_,
                                   args, nullptr));
     nparts += ntile;
@@ -1971,6 +1998,8 @@ double Model::point_apply_bytes(int value_bytes, int extra_vectors) const {
   const double N = static_cast<double>(L_.nslot), B = L_.B;
   double b = (2.0 + extra_vectors) * value_bytes * B * N;
   for (size_t c = 0; c < L_.comps.size(); ++c) {
+    if (gen_.corner[c])  // the linearisation point, class masks, slots
+      b += L_.comps[c].nslot * (8.0 * B + 4.0) + static_cast<double>(L_.comps[c].cells.size());
     if (!gen_.point_words[c]) continue;
     const double cells = static_cast<double>(L_.comps[c].cells.size());
     b += cells * (value_bytes * gen_.point_words[c] + 1.0) + 4.0 * L_.comps[c].nslot;
@@ -1984,6 +2013,8 @@ double Model::point_setup_bytes() const {
   const double N = static_cast<double>(L_.nslot), B = L_.B;
   double b = 8.0 * B * N + 8.0 * B * B * N;
   for (size_t c = 0; c < L_.comps.size(); ++c) {
+    if (gen_.corner[c])  // the linearisation point written, class masks, slots
+      b += L_.comps[c].nslot * (8.0 * B + 4.0) + static_cast<double>(L_.comps[c].cells.size());
     if (!gen_.point_words[c]) continue;
     const double cells = static_cast<double>(L_.comps[c].cells.size());
     b += cells * (8.0 * gen_.point_words[c] + 1.0) + 4.0 * L_.comps[c].nslot;
@@ -2169,7 +2200,7 @@ size_t Model::device_bytes() const {
   for (const auto& v : kf_) b += v.bytes();
   for (const auto& c : comp_dev_)
     b += c.cells.bytes() + c.cell_slots.bytes() + c.cell_mask.bytes() + c.g2l.bytes() + c.tiles.bytes() +
-         c.cell_mask_grid.bytes();
+         c.cell_mask_grid.bytes() + c.rtiles.bytes();
   for (const auto& f : facet_dev_) b += f.fint.bytes() + f.fdbl.bytes();
   return b;
 }
@@ -2212,6 +2243,7 @@ k::MemberView Model::view() const {
         v.pc32 = c < pc32_.size() ? pc32_[c].get() : nullptr;
         v.npc = static_cast<long>(pc_[c].size());
       }
+    if (any_corner()) v.npc = -1;  // no stored coefficients to convert
   }
   v.v[k::kVU] = u_.get();
   v.v[k::kVHist] = hist_.get();

@@ -219,6 +219,7 @@ class Model {
   // compartments without a batched tile kernel, or facets: per-model launches
   bool needs_own_assembly() const;
   bool all_tile_eligible() const;
+  bool any_corner() const;
   // point-coefficient Jacobian: coefficients and diagonal blocks at x, and
   // y = J v from them (v, y FP64 or FP32 as fp32 says); stop as in launch_apply
   void launch_points_setup(const double* x, double t, double cm, double ca);
@@ -332,6 +333,9 @@ class Model {
     std::vector<DeviceArray<int>> atiles;
     std::vector<int> natiles;
     DeviceArray<unsigned char> cell_mask_grid;
+    // corner form: the tiles of the residual and the point set-up
+    DeviceArray<int> rtiles;
+    int nrtiles = 0;
     int ntiles = 0;
     bool g2l_identity = false;  // the compartment's slots are the grid's vertices in order
     // unstructured cells: geometry words and block positions per cell
@@ -350,7 +354,8 @@ class Model {
   DeviceArray<double> weights_;  // lumped mass per slot (mass sums)
   DeviceArray<double> prm_;      // geometry words + run-time parameters
   DeviceArray<double> u_, hist_, r_, z_, xs_, packed_;
-  // matrix-free: the Newton iterate the Jacobian is applied at, and its weights
+  // matrix-free, interface terms and the corner form: the Newton iterate the
+  // Jacobian is applied at, and its weights
   DeviceArray<double> lin_x_;
   double lin_t_ = 0.0, lin_cm_ = 0.0, lin_ca_ = 0.0;
   // point-coefficient Jacobian: per compartment the coefficients of every grid
@@ -361,7 +366,10 @@ class Model {
   std::vector<DeviceArray<float>> pc32_;
   DeviceArray<double> pdiag_;
   DeviceArray<int> diag_id_;
-  DeviceArray<double> pc_tca_;  // (t, ca) of the point coefficients, read by the applies
+  // (t, ca) of the point coefficients, read by the applies; the corner form
+  // also reads cm and the grid's origin and spacing (kTca words)
+  DeviceArray<double> pc_tca_;
+  static constexpr size_t kTca = 9;
   bool use_points_ = false;  // the Krylov operator is the point-coefficient one
   std::vector<DeviceArray<double>> stage_;
   DeviceArray<double> val_, lu_, dinv_;
