@@ -649,7 +649,9 @@ def main():
             # the generated apply of compartment 0 with the tile shape in use
             shapes = [ch for c, _, _, ch in ptuning if c == 0]
             k = shapes.index(True) if True in shapes else 0
-            kernel = f"dcg_tile_0_p{'f' if spmv_kind.endswith('32') else ''}{k}"
+            # (e: coefficients evaluated in the apply, p: stored ones)
+            form = "e" if "dcg_tile_0_e0" in m.generated_source() else "p"
+            kernel = f"dcg_tile_0_{form}{'f' if spmv_kind.endswith('32') else ''}{k}"
         else:
             kernel = VARIANT_KERNELS.get(chosen, "?")
         roofline = {"bound": "hbm", "kernel": spmv_kind, "kernel_name": kernel, "achieved": sp["gbs"],

@@ -259,12 +259,12 @@ void Batch::rebuild() {
       for (int j = 0; j < M; ++j) {
         Model& m = *members_[g.mem[j]].m;
         size_t c0 = 0;
-        while (c0 < m.pc_.size() && !m.pc_[c0].size() && !m.gen_.corner[c0]) ++c0;
+        while (c0 < m.pc_.size() && !m.pc_[c0].size() && !m.gen_.eval[c0]) ++c0;
         if (c0 >= m.pc_.size()) throw Error("internal: point member without coefficients");
         k::PcMember& pm = pcm[j];
         pm.g2l = m.comp_dev_[c0].g2l_identity ? nullptr : m.comp_dev_[c0].g2l.get();
         pm.cmask = m.comp_dev_[c0].cell_mask_grid.get();
-        pm.pc = m.gen_.corner[c0] ? m.lin_x_.get() : m.pc_[c0].get();
+        pm.pc = m.gen_.eval[c0] ? m.lin_x_.get() : m.pc_[c0].get();
         pm.pc32 = c0 < m.pc32_.size() ? m.pc32_[c0].get() : nullptr;
         pm.tca = m.pc_tca_.get();
         pm.prm = m.prm_.get();
@@ -285,11 +285,11 @@ void Batch::rebuild() {
           it = by_mod.emplace(key, g.plaunch.size()).first;
           g.plaunch.emplace_back();
           auto& pl = g.plaunch.back();
-          const std::string name = m.gen_.tile_kernel[c0];
+          const std::string name = m.gen_.tile_kernel[c0] + (m.gen_.eval[c0] ? "_e" : "_p");
           for (size_t k2 = 0; k2 < nk; ++k2) {
             const std::string id = std::to_string(k2);
-            pl.f64s.push_back(m.module_->function(name + "_pbatch" + id));
-            pl.f32s.push_back(opt_.precision == Precision::Mixed ? m.module_->function(name + "_pfbatch" + id)
+            pl.f64s.push_back(m.module_->function(name + "batch" + id));
+            pl.f32s.push_back(opt_.precision == Precision::Mixed ? m.module_->function(name + "fbatch" + id)
                                                                  : nullptr);
             pl.tiles.push_back(m.gen_.apply_tiles[c0][k2]);
             pl.nts.push_back(m.gen_.apply_threads[c0][k2]);
@@ -454,7 +454,7 @@ void Batch::rebuild() {
       }
       if (a.points) {
         for (size_t c = 0; c < m.pc_.size() && c < static_cast<size_t>(k::kAsmComps); ++c)
-          am[j].pc[c] = m.gen_.corner[c] ? m.lin_x_.get() : m.pc_[c].size() ? m.pc_[c].get() : nullptr;
+          am[j].pc[c] = m.gen_.eval[c] ? m.lin_x_.get() : m.pc_[c].size() ? m.pc_[c].get() : nullptr;
         am[j].pdiag = m.pdiag_.get();
         am[j].tca = m.pc_tca_.get();
       }

@@ -10,6 +10,9 @@
 #include "error.hh"
 #include "reduce.hh"
 
+#define DCG_STR2(...) #__VA_ARGS__
+#define DCG_STR(...) DCG_STR2(__VA_ARGS__)
+
 namespace dcopasi {
 
 namespace {
@@ -258,7 +261,7 @@ struct dcg_pc_member {
 };
 static_assert(sizeof(dcg_asm_member) == %ASM_BYTES%, "batch member descriptor layout");
 static_assert(sizeof(dcg_pc_member) == %PCM_BYTES%, "point member descriptor layout");
-// whether an optional array argument is there: known at compile time for a
+%KRYLOV%// whether an optional array argument is there: known at compile time for a
 // local array (compared with null at run time, such an array would stay in
 // scratch memory) and for nullptr
 template <typename M>
@@ -692,6 +695,67 @@ __device__ __forceinline__ void facet_body(const int* __restrict__ fint, const d
     }
   }
 }
+#if !NUMERICAL_JAC
+template <int N>
+struct FacetSlots {
+  static constexpr int value = N;
+};
+// acc += J(x) dir of one row of facet id (row f: the in side's vertex f, NVF +
+// f: the out side's); dir(slots, values, count) gives the direction at slots
+template <typename Dir>
+__device__ __forceinline__ void facet_row(const int* __restrict__ fint, const double* __restrict__ fdbl, int id, int row,
+                                          const double* __restrict__ x, double t, double ca,
+                                          const double* __restrict__ prm, Dir&& dir, double (&acc)[DCG_B]) {
+  const int* fi = fint + (size_t)id * FINT;
+  const double* fd = fdbl + (size_t)id * FDBL;
+  double xi[NVF][BI > 0 ? BI : 1], xo[NVF][BO > 0 ? BO : 1], v[2 * NVF][DCG_B];
+  int sl[2 * NVF];
+#pragma unroll
+  for (int f = 0; f < 2 * NVF; ++f) sl[f] = fi[f];
+#pragma unroll
+  for (int f = 0; f < NVF; ++f) {
+#pragma unroll
+    for (int i = 0; i < BI; ++i) xi[f][i] = x[(size_t)sl[f] * DCG_B + i];
+#pragma unroll
+    for (int i = 0; i < BO; ++i) xo[f][i] = x[(size_t)sl[NVF + f] * DCG_B + i];
+  }
+  dir(sl, v, FacetSlots<2 * NVF>());
+  double ri[NVF][BI > 0 ? BI : 1], ro[NVF][BO > 0 ? BO : 1];
+  double Jii[NVF * NVF * (BI > 0 ? BI * BI : 1)], Jio[NVF * NVF * (BI * BO > 0 ? BI * BO : 1)],
+      Joi[NVF * NVF * (BI * BO > 0 ? BI * BO : 1)], Joo[NVF * NVF * (BO > 0 ? BO * BO : 1)];
+#pragma unroll
+  for (int k = 0; k < NVF * NVF * BI * BI; ++k) Jii[k] = 0.0;
+#pragma unroll
+  for (int k = 0; k < NVF * NVF * BI * BO; ++k) { Jio[k] = 0.0; Joi[k] = 0.0; }
+#pragma unroll
+  for (int k = 0; k < NVF * NVF * BO * BO; ++k) Joo[k] = 0.0;
+  facet_residual(xi, xo, fd, t, ca, ri, ro, Jii, Jio, Joi, Joo, prm);
+#pragma unroll
+  for (int f = 0; f < NVF; ++f) {
+    if (row == f)
+#pragma unroll
+      for (int i = 0; i < BI; ++i)
+#pragma unroll
+        for (int g = 0; g < NVF; ++g) {
+#pragma unroll
+          for (int j = 0; j < BI; ++j) acc[i] += Jii[((f * NVF + g) * BI + i) * BI + j] * v[g][j];
+#pragma unroll
+          for (int j = 0; j < BO; ++j) acc[i] += Jio[((f * NVF + g) * BI + i) * (BO > 0 ? BO : 1) + j] * v[NVF + g][j];
+        }
+    if (BO > 0 && row == NVF + f)
+#pragma unroll
+      for (int i = 0; i < BO; ++i)
+#pragma unroll
+        for (int g = 0; g < NVF; ++g) {
+#pragma unroll
+          for (int j = 0; j < BI; ++j) acc[i] += Joi[((f * NVF + g) * (BO > 0 ? BO : 1) + i) * BI + j] * v[g][j];
+#pragma unroll
+          for (int j = 0; j < BO; ++j)
+            acc[i] += Joo[((f * NVF + g) * (BO > 0 ? BO : 1) + i) * (BO > 0 ? BO : 1) + j] * v[NVF + g][j];
+        }
+  }
+}
+#endif
 }  // namespace %F%
 
 extern "C" __global__ void __launch_bounds__(64)
@@ -1071,6 +1135,137 @@ std::string gen_facet(const ModelSpec& m, const Grid& g, int cin, int cout, bool
 }
 
 
+// A box cell's corner sums of J v with the point coefficients evaluated at
+// the linearisation point (EVAL): what a cell reads is the two vectors at its
+// corners, 2 * 8 * BC values where the stored form reads NQ * NMC (3D, 2
+// species and 3 coefficients: 24 words per cell against 2 per vertex).  One
+// thread holds the cell.  Values at the points, point terms and element
+// stiffness are sums and differences over the corners along each axis with
+// one weight per mode (as in the corner form of larger blocks): with H the
+// butterfly and S the weights, points = H S H corners, corner sums = H S H
+// point terms, stiffness = H kap H.  FP32 applies evaluate in FP64 too.
+// FP64 applies alone: Mitchell-Schaefer 96^3 66 -> 44 us, two
+// compartments 1024^2 80 -> 48 us; FP32 at 47^3, where coefficients stay in
+// cache, 9.0 -> 10.4 us, which the fewer launches of the fused iteration
+// outweigh.
+const char* kEvalCell = R"(
+struct EvalAt {
+  const double* xs;  // the linearisation point over the vertex box (LDS)
+  double t, cm, ca, ox, oy, oz, hx, hy, hz;
+  int vi0, vj0, vk0;
+  const double* prm;
+};
+constexpr double G2 = 0.28867513459481288225;  // 1 / (2 sqrt 3)
+__device__ constexpr double mode_weight(int a) {
+  double w = 1.0;
+  for (int k = 0; k < DIM; ++k) w *= ((a >> k) & 1) ? G2 : 0.5;
+  return w;
+}
+// stiffness of mode a along axis k: 1D stiffness 1/h on differences, 1D mass
+// h/4 on sums and h/12 on differences
+__device__ constexpr double mode_kap(int a, int k) {
+  double w = ((a >> k) & 1) ? 1.0 / KH[k] : 0.0;
+  for (int l = 0; l < DIM; ++l)
+    if (l != k) w *= ((a >> l) & 1) ? KH[l] / 12.0 : KH[l] / 4.0;
+  return w;
+}
+// sums (bit 0) and differences (bit 1) over the corners along every axis
+template <typename T>
+__device__ __forceinline__ void corner_modes(T (&v)[NV][BC]) {
+#pragma unroll
+  for (int k = 0; k < DIM; ++k)
+#pragma unroll
+    for (int a = 0; a < NV; ++a) {
+      if ((a >> k) & 1) continue;
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        const T lo = v[a][i], hi = v[a | (1 << k)][i];
+        v[a][i] = lo + hi;
+        v[a | (1 << k)][i] = lo - hi;
+      }
+    }
+}
+template <typename TL, typename T, typename Put>
+__device__ __forceinline__ void eval_cell(const EvalAt& E, const T* vs, int ci, int cj, int ck, Put&& put) {
+  constexpr int XB = TL::XB, YB = TL::YB;
+  double u[NV][BC];
+  T v[NV][BC], vm[NV][BC];
+#pragma unroll
+  for (int a = 0; a < NV; ++a) {
+    const int b = (ci + (a & 1)) + XB * ((cj + ((a >> 1) & 1)) + YB * (ck + ((a >> 2) & 1)));
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      u[a][i] = E.xs[b * BC + i];
+      v[a][i] = vs[b * BC + i];
+    }
+  }
+  corner_modes(u);
+#pragma unroll
+  for (int a = 0; a < NV; ++a)
+#pragma unroll
+    for (int i = 0; i < BC; ++i) u[a][i] *= mode_weight(a);
+  corner_modes(u);
+  corner_modes(v);
+#pragma unroll
+  for (int a = 0; a < NV; ++a)
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      vm[a][i] = v[a][i];
+      v[a][i] *= T(mode_weight(a));
+    }
+  corner_modes(v);
+#pragma unroll
+  for (int q = 0; q < NQ; ++q) {
+    const double px = E.ox + (E.vi0 + ci + ((q & 1) ? 0.5 + G2 : 0.5 - G2)) * E.hx;
+    const double py = DIM > 1 ? E.oy + (E.vj0 + cj + ((q & 2) ? 0.5 + G2 : 0.5 - G2)) * E.hy : 0.0;
+    const double pz = DIM > 2 ? E.oz + (E.vk0 + ck + ((q & 4) ? 0.5 + G2 : 0.5 - G2)) * E.hz : 0.0;
+    double mc[NMC > 0 ? NMC : 1];
+    point_jacobian(u[q], px, py, pz, E.t, E.cm, E.ca, mc, E.prm);
+    T w[BC];
+    point_block(mc, v[q], w);
+#pragma unroll
+    for (int i = 0; i < BC; ++i) v[q][i] = w[i];
+  }
+  corner_modes(v);
+#pragma unroll
+  for (int a = 0; a < NV; ++a)
+#pragma unroll
+    for (int i = 0; i < BC; ++i) v[a][i] *= T(mode_weight(a));
+  double dp[NEP > 0 ? NEP : 1], gk[3] = {1.0, 1.0, 1.0};
+  pair_diffusion(E.t, E.prm, dp);
+#if DCG_GEO
+#pragma unroll
+  for (int k = 0; k < DIM; ++k) gk[k] = E.prm[6] * E.prm[3 + k] * E.prm[3 + k];
+#endif
+#pragma unroll
+  for (int n = 0; n < NEP; ++n)
+#pragma unroll
+    for (int a = 1; a < NV; ++a) {
+      double kk = 0.0;
+#pragma unroll
+      for (int k = 0; k < DIM; ++k)
+        if (EPK[n] == 3 || EPK[n] == k) kk += mode_kap(a, k) * gk[k];
+      v[a][EPI[n]] += T(E.ca * dp[n] * kk) * vm[a][EPJ[n]];
+    }
+  corner_modes(v);
+#pragma unroll
+  for (int a = 0; a < NV; ++a)
+#pragma unroll
+    for (int i = 0; i < BC; ++i) put(a, i, v[a][i]);
+}
+)";
+// what the stored form puts in its place
+const char* kNoEvalCell = R"(
+struct EvalAt {
+  const double* xs;
+  double t, cm, ca, ox, oy, oz, hx, hy, hz;
+  int vi0, vj0, vk0;
+  const double* prm;
+};
+template <typename TL, typename T, typename Put>
+__device__ __forceinline__ void eval_cell(const EvalAt&, const T*, int, int, int, Put&&) {}
+)";
+
 // Tiled write-once volume kernel.  One workgroup owns a TX x TY x TZ box of
 // vertices; it stages the state of the surrounding vertex box and the class
 // masks of the surrounding cells in LDS, computes per (cell, class, point)
@@ -1244,6 +1439,62 @@ struct ApplyTile {
   static constexpr int NVB = XB * YB * ZB, NCB = CXB * CYB * CZB, NROW = TX * TY * TZ;
 };
 %APPLY_SHAPES%
+// The corner sums oc of the cells, one cell per thread, added to the vertex box:
+// corner by corner, for one corner the cells' vertices are distinct, so no two
+// threads add to the same vertex between two barriers, and every vertex
+// sums its cells in a fixed order.  When a box row of cells lies within
+// one wave (CXB divides 64), the x neighbour's corner sums arrive by lane
+// shuffle instead: lane ci holds vertex x = ci's sums of cells ci-1 and
+// ci (own first), which halves the rounds; when a whole xy layer lies
+// within one wave the y neighbour's arrive the same way (CXB lanes away)
+// and the rounds halve again.  Only the tile's own rows are read back,
+// so the halo vertices (x = 0 and x = CXB, likewise in y) need no sums.
+template <typename TL, typename T>
+__device__ __forceinline__ void scatter_corners(const T (&oc)[NCORNER][BC], bool in, bool has, int ci, int cj, int ck,
+                                                T* accv) {
+  constexpr int XB = TL::XB, YB = TL::YB, CXB = TL::CXB, CYB = TL::CYB;
+  constexpr bool CMB_X = DIM > 1 && 64 % CXB == 0;
+  constexpr bool CMB_Y = CMB_X && 64 % (CXB * CYB) == 0;
+  constexpr int NFOLD = CMB_Y ? 4 : CMB_X ? 2 : 1;  // corners folded into one round
+  constexpr int NR = NCORNER / NFOLD;             // rounds
+  // rs[r]: the sums of round r's vertex; round r takes corner r * NFOLD
+  T rs[NR][BC];
+  if constexpr (CMB_X) {
+    T fx[NCORNER / 2][BC];
+#pragma unroll
+    for (int h = 0; h < NCORNER / 2; ++h)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) fx[h][i] = oc[2 * h][i] + __shfl_up(oc[2 * h + 1][i], 1, 64);
+    if constexpr (CMB_Y) {
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) rs[r][i] = fx[2 * r][i] + __shfl_up(fx[2 * r + 1][i], CXB, 64);
+    } else {
+#pragma unroll
+      for (int r = 0; r < NR; ++r)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) rs[r][i] = fx[r][i];
+    }
+  } else {
+#pragma unroll
+    for (int r = 0; r < NR; ++r)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) rs[r][i] = oc[r][i];
+  }
+  const bool add = CMB_Y ? in && ci > 0 && cj > 0 : CMB_X ? in && ci > 0 : has;
+#pragma unroll
+  for (int r = 0; r < NR; ++r) {
+    if (r) __syncthreads();
+    if (add) {
+      const int c = r * NFOLD;
+      const int b = (ci + (c & 1)) + XB * ((cj + ((c >> 1) & 1)) + YB * (ck + ((c >> 2) & 1)));
+#pragma unroll
+      for (int i = 0; i < BC; ++i) accv[b * BC + i] += rs[r][i];
+    }
+  }
+}
+
 // The rows of one tile from point coefficients coef(box cell, (p*NQ + q)*NMC +
 // n) (read from the grid-wide array in HBM, or the set-up's staged LDS array)
 // and the direction staged in vs over the vertex box (slots sl, class masks cms): per
@@ -1256,8 +1507,10 @@ struct ApplyTile {
 // caller) when SCATTER, else out.
 // VP, YP: pointer types of the vectors read and of y (global-memory pointers
 // from the point apply, plain ones from the matrix-free apply).
-template <typename TL, typename T, typename CF, typename VP, typename YP>
-__device__ __forceinline__ void cells_apply(CF coef, const T* vs, const int* sl,
+// EV: the cells' sums from eval_cell (ev: where and at what to evaluate).
+%EVAL_CELL%
+template <typename TL, typename T, bool EV, typename CF, typename VP, typename YP>
+__device__ __forceinline__ void cells_apply(CF coef, const EvalAt* ev, const T* vs, const int* sl,
                                             const unsigned char* cms, T* out, T* accv, VP __restrict__ v,
                                             YP __restrict__ y, double ca, const double (&dv)[NDV > 0 ? NDV : 1],
                                             VP __restrict__ w1, VP __restrict__ w2,
@@ -1356,20 +1609,6 @@ __device__ __forceinline__ void cells_apply(CF coef, const T* vs, const int* sl,
     }
   };
   if constexpr (SCATTER) {
-    // one cell per thread; its corner sums are added to the vertices corner
-    // by corner: for one corner the cells' vertices are distinct, so no two
-    // threads add to the same vertex between two barriers, and every vertex
-    // sums its cells in a fixed order.  When a box row of cells lies within
-    // one wave (CXB divides 64), the x neighbour's corner sums arrive by lane
-    // shuffle instead: lane ci holds vertex x = ci's sums of cells ci-1 and
-    // ci (own first), which halves the rounds; when a whole xy layer lies
-    // within one wave the y neighbour's arrive the same way (CXB lanes away)
-    // and the rounds halve again.  Only the tile's own rows are read back,
-    // so the halo vertices (x = 0 and x = CXB, likewise in y) need no sums.
-    constexpr bool CMB_X = DIM > 1 && 64 % CXB == 0;
-    constexpr bool CMB_Y = CMB_X && 64 % (CXB * CYB) == 0;
-    constexpr int NFOLD = CMB_Y ? 4 : CMB_X ? 2 : 1;  // corners folded into one round
-    constexpr int NR = NCORNER / NFOLD;             // rounds
     const int cl = threadIdx.x;
     const bool in = cl < NCB;
     const bool has = in && cms[in ? cl : 0];
@@ -1378,44 +1617,13 @@ __device__ __forceinline__ void cells_apply(CF coef, const T* vs, const int* sl,
     for (int c = 0; c < NCORNER; ++c)
 #pragma unroll
       for (int i = 0; i < BC; ++i) oc[c][i] = T(0);
-    if (has) cell_corner_sums(cl, cms[cl], [&](int c, int i, T v2) { oc[c][i] += v2; });
     const int ci = cl % CXB, cj = (cl / CXB) % CYB, ck = cl / (CXB * CYB);
-    // rs[r]: the sums of round r's vertex; round r takes corner r * NFOLD
-    T rs[NR][BC];
-    if constexpr (CMB_X) {
-      T fx[NCORNER / 2][BC];
-#pragma unroll
-      for (int h = 0; h < NCORNER / 2; ++h)
-#pragma unroll
-        for (int i = 0; i < BC; ++i) fx[h][i] = oc[2 * h][i] + __shfl_up(oc[2 * h + 1][i], 1, 64);
-      if constexpr (CMB_Y) {
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-          for (int i = 0; i < BC; ++i) rs[r][i] = fx[2 * r][i] + __shfl_up(fx[2 * r + 1][i], CXB, 64);
-      } else {
-#pragma unroll
-        for (int r = 0; r < NR; ++r)
-#pragma unroll
-          for (int i = 0; i < BC; ++i) rs[r][i] = fx[r][i];
-      }
+    if constexpr (EV) {
+      if (has) eval_cell<TL, T>(*ev, vs, ci, cj, ck, [&](int c, int i, T v2) { oc[c][i] = v2; });
     } else {
-#pragma unroll
-      for (int r = 0; r < NR; ++r)
-#pragma unroll
-        for (int i = 0; i < BC; ++i) rs[r][i] = oc[r][i];
+      if (has) cell_corner_sums(cl, cms[cl], [&](int c, int i, T v2) { oc[c][i] += v2; });
     }
-    const bool add = CMB_Y ? in && ci > 0 && cj > 0 : CMB_X ? in && ci > 0 : has;
-#pragma unroll
-    for (int r = 0; r < NR; ++r) {
-      if (r) __syncthreads();
-      if (add) {
-        const int c = r * NFOLD;
-        const int b = (ci + (c & 1)) + XB * ((cj + ((c >> 1) & 1)) + YB * (ck + ((c >> 2) & 1)));
-#pragma unroll
-        for (int i = 0; i < BC; ++i) accv[b * BC + i] += rs[r][i];
-      }
-    }
+    scatter_corners<TL, T>(oc, in, has, ci, cj, ck, accv);
   } else {
     for (int cl = threadIdx.x; cl < NCB; cl += blockDim.x) {
       T* dst = out + (size_t)cl * (NCORNER * BC);
@@ -1576,7 +1784,15 @@ __device__ __forceinline__ void tile_body(int tile, GI __restrict__ g2l, GB __re
       // vertices) into the grid-wide array, word-major:
       // val[((p*NQ + q)*NMC + n) * cells of the grid + cell]; cells outside
       // the compartment carry values that are never read
-      if constexpr (NMC > 0) {
+      if constexpr (EVAL) {
+        // (evaluated applies: the rows' linearisation point instead)
+        for (int it = threadIdx.x; it < NROW * DCG_B; it += blockDim.x) {
+          const int lr = it / DCG_B, i = it % DCG_B;
+          const int li = lr % TX, lj = DIM > 1 ? (lr / TX) % TY : 0, lk = DIM > 2 ? lr / (TX * TY) : 0;
+          const int s = sl[(li + 1) + XB * ((lj + OY) + YB * (lk + OZ))];
+          if (s >= 0) val[(size_t)s * DCG_B + i] = x[(size_t)s * DCG_B + i];
+        }
+      } else if constexpr (NMC > 0) {
         const size_t ncg = (size_t)n0 * (size_t)n1 * (size_t)n2;
         for (int k = threadIdx.x; k < OWN_WORDS; k += blockDim.x) {
           const int w = k / NOWN, o = k % NOWN;
@@ -1618,8 +1834,9 @@ __device__ __forceinline__ void tile_body(int tile, GI __restrict__ g2l, GB __re
       }
       __syncthreads();
       if constexpr (CELL_APPLY) {
-        cells_apply<ApplyTile<TX, TY, TZ>, double>(
-            [&](int cl, int wd) { return ((const double*)work)[(size_t)wd * NCB + cl]; }, xs, sl, cms, nullptr, acc4,
+        cells_apply<ApplyTile<TX, TY, TZ>, double, false>(
+            [&](int cl, int wd) { return ((const double*)work)[(size_t)wd * NCB + cl]; }, nullptr, xs, sl, cms, nullptr,
+            acc4,
             base, r, ca, dv, (GX) nullptr, (GX) nullptr, nullptr);
         return;
       }
@@ -2018,10 +2235,18 @@ __device__ __forceinline__ void tile_body(int tile, GI __restrict__ g2l, GB __re
 // and would use flat accesses)
 template <typename X>
 using dcg_gp = __attribute__((address_space(1))) X*;
+// EVAL: pc is the linearisation point itself (slot-major) and the cells
+// evaluate their coefficients there.
+template <bool E, typename A, typename B2>
+struct dcg_pick { using type = A; };
+template <typename A, typename B2>
+struct dcg_pick<false, A, B2> { using type = B2; };
+template <typename T>
+using pc_t = typename dcg_pick<EVAL, double, T>::type;
 template <typename TL, typename T>
 __device__ __forceinline__ void pc_apply(int tile, dcg_gp<const int> __restrict__ g2l,
                                          dcg_gp<const unsigned char> __restrict__ cmask,
-                                         dcg_gp<const T> __restrict__ pc, dcg_gp<const T> __restrict__ v,
+                                         dcg_gp<const pc_t<T>> __restrict__ pc, dcg_gp<const T> __restrict__ v,
                                          dcg_gp<T> __restrict__ y, dcg_gp<const double> __restrict__ tca, int n0,
                                          int n1, int n2, const double* __restrict__ prm,
                                          dcg_gp<const T> __restrict__ w1, dcg_gp<const T> __restrict__ w2,
@@ -2037,7 +2262,9 @@ __device__ __forceinline__ void pc_apply(int tile, dcg_gp<const int> __restrict_
   __shared__ T vs[NVB * BC];
   __shared__ int sl[NVB];
   __shared__ unsigned char cms[NCB];
-  __shared__ size_t coff[NCB];
+  __shared__ size_t coff[EVAL ? 1 : NCB];
+  __shared__ double xs[EVAL ? NVB * BC : 1];
+  static_assert(!EVAL || SCATTER, "evaluated applies hold one cell per thread");
   __shared__ T out[SCATTER ? 1 : NCB * NCORNER * BC];
   __shared__ T accv[SCATTER ? NVB * BC : 1];
   const int ntx = (n0 + 1 + TX - 1) / TX;
@@ -2055,6 +2282,8 @@ __device__ __forceinline__ void pc_apply(int tile, dcg_gp<const int> __restrict_
     }
     sl[b] = s;
     for (int i = 0; i < BC; ++i) vs[b * BC + i] = s >= 0 ? v[(size_t)s * DCG_B + i] : T(0);
+    if constexpr (EVAL)
+      for (int i = 0; i < BC; ++i) xs[b * BC + i] = s >= 0 ? pc[(size_t)s * DCG_B + i] : 0.0;
     if constexpr (SCATTER)
       for (int i = 0; i < BC; ++i) accv[b * BC + i] = T(0);
   }
@@ -2068,13 +2297,16 @@ __device__ __forceinline__ void pc_apply(int tile, dcg_gp<const int> __restrict_
       m = cmask[off];
     }
     cms[c] = m;
-    coff[c] = off;
+    if constexpr (!EVAL) coff[c] = off;
   }
   __syncthreads();
   double dv[NDV > 0 ? NDV : 1];
   uniform_diffusion(t, prm, dv);
-  cells_apply<TL, T>(
-      [&](int cl, int wd) -> T { return pc[coff[cl] + (size_t)wd * WS]; },
+  EvalAt ev{};
+  if constexpr (EVAL)
+    ev = EvalAt{xs, t, tca[2], ca, tca[3], tca[4], tca[5], tca[6], tca[7], tca[8], vi0, vj0, vk0, prm};
+  cells_apply<TL, T, EVAL>(
+      [&](int cl, int wd) -> T { return pc[coff[EVAL ? 0 : cl] + (size_t)wd * WS]; }, &ev,
       vs, sl, cms, out, accv, v, y, ca, dv, w1, w2, part);
 }
 
@@ -2108,8 +2340,8 @@ extern "C" __global__ void __launch_bounds__(256)
            const double* __restrict__ x, const double* __restrict__ base, double t, double cm, double ca,
            double* __restrict__ r, double* __restrict__ val, const int* __restrict__ own_start,
            const unsigned* __restrict__ own_mask, int n0, int n1, int n2, double ox, double oy, double oz, double hx,
-           double hy, double hz, int mode, const double* __restrict__ prm, const int* __restrict__ stop) {
-  (void)stop;
+           double hy, double hz, int mode, const double* __restrict__ prm, double* __restrict__ tca) {
+  if (blockIdx.x == 0 && threadIdx.x == 0) %C%::set_tca(tca, t, ca, cm, ox, oy, oz, hx, hy, hz);
   %C%::tile_body<8>(tiles[blockIdx.x], g2l, cmask, x, base, t, cm, ca, r, val, own_start, own_mask, n0, n1, n2, ox,
                     oy, oz, hx, hy, hz, mode, prm);
 }
@@ -2120,7 +2352,7 @@ extern "C" __global__ void __launch_bounds__(256)
 #define DCG_POINT_ENTRY(NAME, T, TL)                                                                              \
   extern "C" __global__ void __launch_bounds__(TL::NT, TL::MINW)                                                  \
   NAME(const int* __restrict__ tiles, int ntile, const int* __restrict__ g2l,                                     \
-       const unsigned char* __restrict__ cmask, const T* __restrict__ pc, const T* __restrict__ v,                 \
+       const unsigned char* __restrict__ cmask, const %C%::pc_t<T>* __restrict__ pc, const T* __restrict__ v,      \
        T* __restrict__ y, const double* __restrict__ tca, int n0, int n1, int n2, const double* __restrict__ prm,  \
        const int* __restrict__ stop, const T* __restrict__ w1, const T* __restrict__ w2,                          \
        double* __restrict__ part) {                                                                               \
@@ -2128,7 +2360,7 @@ extern "C" __global__ void __launch_bounds__(256)
     const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
     if (c >= ntile) return;                                                                                       \
     %C%::pc_apply<TL, T>(tiles[c], (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,          \
-                         (%C%::dcg_gp<const T>)pc, (%C%::dcg_gp<const T>)v, (%C%::dcg_gp<T>)y,                    \
+                         (%C%::dcg_gp<const %C%::pc_t<T>>)pc, (%C%::dcg_gp<const T>)v, (%C%::dcg_gp<T>)y,         \
                          (%C%::dcg_gp<const double>)tca, n0, n1, n2, prm, (%C%::dcg_gp<const T>)w1,               \
                          (%C%::dcg_gp<const T>)w2, part ? part + 2 * (size_t)c : nullptr);                        \
   }
@@ -2152,9 +2384,8 @@ extern "C" __global__ void __launch_bounds__(256)
   if (cf[3] == 0.0) return;
   const dcg_asm_member& M = mem[w.x];
   if (threadIdx.x == 0) {
-    // every workgroup of the member writes the same two values
-    M.tca[0] = cf[0];
-    M.tca[1] = cf[2];
+    // every workgroup of the member writes the same values
+    %C%::set_tca(M.tca, cf[0], cf[2], cf[1], M.origin[0], M.origin[1], M.origin[2], M.h[0], M.h[1], M.h[2]);
   }
   // (the member's pointers in the global address space: global, not flat, accesses)
   using GX = %C%::dcg_gp<const double>;
@@ -2176,7 +2407,7 @@ extern "C" __global__ void __launch_bounds__(256)
     if (skip == 1 && *M.irdone) return;                                                                           \
     using GT = %C%::dcg_gp<const T>;                                                                              \
     %C%::pc_apply<TL, T>(w.y, (%C%::dcg_gp<const int>)M.g2l, (%C%::dcg_gp<const unsigned char>)M.cmask,          \
-                         (GT)M.PC, (GT)M.VEC[xsel], (%C%::dcg_gp<T>)M.VEC[ysel],                                  \
+                         (%C%::dcg_gp<const %C%::pc_t<T>>)M.PC, (GT)M.VEC[xsel], (%C%::dcg_gp<T>)M.VEC[ysel],                                  \
                          (%C%::dcg_gp<const double>)M.tca, M.n[0], M.n[1], M.n[2], M.prm,                         \
                          w1sel >= 0 ? (GT)M.VEC[w1sel] : nullptr, w2sel >= 0 ? (GT)M.VEC[w2sel] : nullptr,        \
                          part ? part + 2 * (size_t)(part_off + c) : nullptr);                                     \
@@ -2209,6 +2440,213 @@ extern "C" __global__ void __launch_bounds__(256)
 }
 )";
 
+// The operator launch of a fused BiCGSTAB iteration over evaluated
+// coefficients (KrylovOp): the direction is formed from the iteration's
+// vectors while the vertex box is staged, so the p- and s-updates and the
+// reductions before them cost no launches and no passes of their own.  The
+// vectors are loaded before the previous launch's partials are summed.  A
+// workgroup stores the new p of its own rows; halo vertices recompute it.
+// An iteration is 3 launches (5 with the finishers of large meshes) and the
+// facets' 2, where it was 8 and up to 12 of facets.  Runs of time steps, with
+// the evaluation: 24^2 6.7 -> 4.4 ms; 47^3 mixed 35.0 -> 27.6 ms; 96^3 85 -> 70
+// ms; with an interface 300^2 mixed 17.6 -> 10.2 ms, 1024^2 167 -> 112 ms.
+const char* kEvalKrylov = R"(
+namespace %C% {
+// M^-1 q at slot s (jac 0: none, 1: a block per slot, 2: the diagonal)
+template <typename T>
+__device__ __forceinline__ void precondition(int jac, const double* __restrict__ dinv, int s, const T (&q)[BC],
+                                             T (&o)[BC]) {
+  if (jac == 2) {
+#pragma unroll
+    for (int i = 0; i < BC; ++i) o[i] = (T)(dinv[(size_t)s * DCG_B + i] * (double)q[i]);
+  } else if (jac == 1) {
+    const double* d = dinv + (size_t)s * (DCG_B * DCG_B);
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      double v = 0.0;
+#pragma unroll
+      for (int j = 0; j < BC; ++j) v += d[i * DCG_B + j] * (double)q[j];
+      o[i] = (T)v;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < BC; ++i) o[i] = q[i];
+  }
+}
+// the launch's partials of one workgroup (NT threads)
+template <int NT>
+__device__ __forceinline__ void put_partials(const KrylovOp& op, int at, double e0, double e1, double e2, double* red) {
+  double e[3] = {e0, e1, e2};
+  group_sums<NT, 3>(e, red);
+  if (threadIdx.x == 0) {
+    op.part[op.off + at] = e[0];
+    if (op.mode == 2) {
+      op.part[op.pstride + op.off + at] = e[1];
+      op.part[2 * op.pstride + op.off + at] = e[2];
+    }
+  }
+}
+)";
+const char* kEvalKrylovCells = R"(
+template <typename TL, typename T>
+__device__ __forceinline__ void eval_krylov(int tile, int at, dcg_gp<const int> __restrict__ g2l,
+                                            dcg_gp<const unsigned char> __restrict__ cmask, dcg_gp<const double> lin,
+                                            const KrylovOp& op, bool lead, dcg_gp<const double> __restrict__ tca,
+                                            int n0, int n1, int n2, const double* __restrict__ prm) {
+  constexpr int TX = TL::TX, TY = TL::TY, TZ = TL::TZ, XB = TL::XB, YB = TL::YB, CXB = TL::CXB, CYB = TL::CYB;
+  constexpr int NVB = TL::NVB, NCB = TL::NCB, NROW = TL::NROW, NT = TL::NT, IT = (NVB + NT - 1) / NT;
+  static_assert(NCB <= NT, "one cell per thread");
+  __shared__ T vs[NVB * BC], accv[NVB * BC];
+  __shared__ double xs[NVB * BC];
+  __shared__ int sl[NVB];
+  __shared__ unsigned char cms[NCB];
+  __shared__ double red[3 * (NT / 64)];
+  const auto A = (dcg_gp<const T>)(const T*)op.a;
+  const auto P = (dcg_gp<const T>)(const T*)op.b;
+  const auto C = (dcg_gp<const T>)(const T*)op.c;
+  const int mode = op.mode, tid = threadIdx.x;
+  const int ntx = (n0 + 1 + TX - 1) / TX;
+  const int nty = DIM > 1 ? (n1 + 1 + TY - 1) / TY : 1;
+  const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
+  const int vi0 = tx * TX - 1, vj0 = DIM > 1 ? ty * TY - 1 : 0, vk0 = DIM > 2 ? tz * TZ - 1 : 0;
+  T a[IT][BC], p[IT][BC], c[IT][BC];
+  int ss[IT];
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int b = tid + k * NT;
+    int s = -1;
+    if (b < NVB) {
+      const int bi = b % XB, bj = (b / XB) % YB, bk = b / (XB * YB);
+      const int gi = vi0 + bi, gj = vj0 + bj, gk = vk0 + bk;
+      if (gi >= 0 && gi <= n0 && gj >= 0 && gj <= (DIM > 1 ? n1 : 0) && gk >= 0 && gk <= (DIM > 2 ? n2 : 0)) {
+        const int vid = gi + (n0 + 1) * (gj + (n1 + 1) * gk);
+        s = g2l ? g2l[vid] : vid;
+      }
+      sl[b] = s;
+    }
+    ss[k] = s;
+    double x[BC];
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      a[k][i] = p[k][i] = c[k][i] = T(0);
+      x[i] = 0.0;
+    }
+    if (s >= 0) {
+#pragma unroll
+      for (int i = 0; i < BC; ++i) a[k][i] = A[(size_t)s * DCG_B + i];
+      if (mode)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) c[k][i] = C[(size_t)s * DCG_B + i];
+      if (mode == 1)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) p[k][i] = P[(size_t)s * DCG_B + i];
+#pragma unroll
+      for (int i = 0; i < BC; ++i) x[i] = lin[(size_t)s * DCG_B + i];
+    }
+    if (b < NVB)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        xs[b * BC + i] = x[i];
+        accv[b * BC + i] = T(0);
+      }
+  }
+  for (int cl = tid; cl < NCB; cl += NT) {
+    const int ci = cl % CXB, cj = (cl / CXB) % CYB, ck = cl / (CXB * CYB);
+    const int gi = vi0 + ci, gj = vj0 + cj, gk = vk0 + ck;
+    unsigned char m = 0;
+    if (gi >= 0 && gi < n0 && gj >= 0 && gj < (DIM > 1 ? n1 : 1) && gk >= 0 && gk < (DIM > 2 ? n2 : 1))
+      m = cmask[gi + n0 * (gj + n1 * gk)];
+    cms[cl] = m;
+  }
+  BicgScalars sc;
+  sc.alpha = sc.beta = sc.omega = 0.0;
+  if (mode == 1) {
+    if (!finish_stage<NT, 2>(sc, op.in, op.out, lead, op.fin, op.nfin, op.fstride, 4, red)) return;
+  } else if (mode == 2) {
+    if (!finish_stage<NT, 1>(sc, op.in, op.out, lead, op.fin, op.nfin, op.fstride, 1, red)) return;
+  }
+  const double alpha = sc.alpha, beta = sc.beta, omega = sc.omega;
+#pragma unroll
+  for (int k = 0; k < IT; ++k) {
+    const int b = tid + k * NT, s = ss[k];
+    if (b >= NVB) continue;
+    T q[BC], o[BC];
+#pragma unroll
+    for (int i = 0; i < BC; ++i)
+      q[i] = mode == 1   ? (T)((double)a[k][i] + beta * ((double)p[k][i] - omega * (double)c[k][i]))
+             : mode == 2 ? (T)((double)a[k][i] - alpha * (double)c[k][i])
+                         : a[k][i];
+    if (s >= 0 && mode == 1) {
+      const int bi = b % XB, bj = (b / XB) % YB, bk = b / (XB * YB);
+      if (bi >= 1 && bi <= TX && (DIM < 2 || (bj >= 1 && bj <= TY)) && (DIM < 3 || (bk >= 1 && bk <= TZ))) {
+        const auto D = (dcg_gp<T>)(T*)op.d;
+#pragma unroll
+        for (int i = 0; i < DCG_B; ++i) D[(size_t)s * DCG_B + i] = i < BC ? q[i < BC ? i : 0] : T(0);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < BC; ++i) o[i] = q[i];
+    if (s >= 0 && mode) precondition(op.jac, op.dinv, s, q, o);
+#pragma unroll
+    for (int i = 0; i < BC; ++i) vs[b * BC + i] = o[i];
+  }
+  __syncthreads();
+  const double ca = tca[1];
+  {
+    const EvalAt ev{xs, tca[0], tca[2], ca, tca[3], tca[4], tca[5], tca[6], tca[7], tca[8], vi0, vj0, vk0, prm};
+    const bool in = tid < NCB, has = in && cms[in ? tid : 0];
+    T oc[NCORNER][BC];
+#pragma unroll
+    for (int k = 0; k < NCORNER; ++k)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) oc[k][i] = T(0);
+    const int ci = tid % CXB, cj = (tid / CXB) % CYB, ck = tid / (CXB * CYB);
+    if (has) eval_cell<TL, T>(ev, vs, ci, cj, ck, [&](int k, int i, T v2) { oc[k][i] = v2; });
+    scatter_corners<TL, T>(oc, in, has, ci, cj, ck, accv);
+  }
+  __syncthreads();
+  double e0 = 0.0, e1 = 0.0, e2 = 0.0;
+  const auto Y = (dcg_gp<T>)(T*)op.y;
+  const auto W = (dcg_gp<const T>)(const T*)op.w;
+  for (int it = tid; it < NROW * DCG_B; it += NT) {
+    const int lr = it / DCG_B, i = it % DCG_B;
+    const int li = lr % TX, lj = DIM > 1 ? (lr / TX) % TY : 0, lk = DIM > 2 ? lr / (TX * TY) : 0;
+    const int vb = (li + 1) + XB * ((lj + OY) + YB * (lk + OZ));
+    const int s = sl[vb];
+    if (s < 0) continue;
+    const size_t k = (size_t)s * DCG_B + i;
+    // padding species: identity rows (their directions are zero in a solve)
+    const T acc = i < BC ? accv[vb * BC + (i < BC ? i : 0)] : mode ? T(0) : A[k];
+    Y[k] = acc;
+    if (mode == 1) {
+      e0 += (double)acc * (double)W[k];
+    } else if (mode == 2) {
+      const double sv = (double)(T)((double)A[k] - alpha * (double)C[k]);
+      e0 += (double)acc * sv;
+      e1 += (double)acc * (double)acc;
+      e2 += sv * sv;
+    }
+  }
+  if (mode) put_partials<NT>(op, at, e0, e1, e2, red);
+}
+)";
+const char* kEvalKrylovEntries = R"(
+}  // namespace %C%
+#define DCG_EVAL_ENTRY(NAME, T, TL)                                                                               \
+  extern "C" __global__ void __launch_bounds__(TL::NT, TL::MINW)                                                  \
+  NAME(const int* __restrict__ tiles, int ntile, const int* __restrict__ g2l,                                     \
+       const unsigned char* __restrict__ cmask, const double* lin, KrylovOp op, const double* __restrict__ tca,    \
+       int n0, int n1, int n2, const double* __restrict__ prm) {                                                  \
+    const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
+    if (c >= ntile) return;                                                                                       \
+    %C%::%EVAL_FN%<TL, T>(tiles[c], c, (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,      \
+                          (%C%::dcg_gp<const double>)lin, op, op.lead && blockIdx.x == 0,                         \
+                          (%C%::dcg_gp<const double>)tca, n0, n1, n2, prm);                                       \
+  }
+%EVAL_ENTRIES%
+#undef DCG_EVAL_ENTRY
+)";
+
 // Box cells with blocks of more than 4 species: one lane per (cell, corner).
 // A thread that holds all corners of a cell would need 2^DIM values per
 // species several times over; here a lane holds one corner's values, which
@@ -2239,10 +2677,9 @@ struct CornerTile {
   static constexpr int TX = X, TY = DIM > 2 ? Y : 1;           // row vertices of a layer
   static constexpr int TM = DIM > 2 ? Z : Y;                   // layers of row vertices
   static constexpr int CX = TX + 1, CY = DIM > 2 ? TY + 1 : 1;  // cells of a layer
-  static constexpr int NT = CX * CY * NCORNER, ROWS = TX * TY;
+  static constexpr int NT = CX * CY * NCORNER, ROWS = TX * TY, MINW = 1;
 };
 %CORNER_SHAPES%
-%CORNER_TABLES%
 
 // the value of the lane at the other end of the cell along axis A: lanes of a
 // cell are l = (b0 | b1 << 1) ^ (b2 ? 7 : 0), so the three axes are the lane
@@ -2273,7 +2710,8 @@ __device__ __forceinline__ void butterfly(T (&v)[N], const T (&sg)[3]) {
 }
 
 // OP 1: y = base + residual at x (T = double).  OP 4: y = J(x) v and, with
-// part, the partial dots (y.w1, y.w2).  OP 8: diagonal blocks of J(x) into y
+// part, the partial dots (y.w1, y.w2).  OP 5: a fused operator launch (op,
+// lead, its partials at `at`).  OP 8: diagonal blocks of J(x) into y
 // (all entries with `full`, else the diagonal) and the rows' x into lin.
 template <typename TL, int OP, typename T>
 __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restrict__ g2l,
@@ -2282,8 +2720,9 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
                                             dcg_gp<double> lin, double t, double cm, double ca, int n0, int n1, int n2,
                                             double ox, double oy, double oz, double hx, double hy, double hz,
                                             const double* __restrict__ prm, bool full, dcg_gp<const T> w1,
-                                            dcg_gp<const T> w2, double* __restrict__ part) {
+                                            dcg_gp<const T> w2, double* __restrict__ part%CORNER_OP_PARAMS%) {
   constexpr int TX = TL::TX, TY = TL::TY, TM = TL::TM, CX = TL::CX, NT = TL::NT;
+%CORNER_OP_BEGIN%
   constexpr int PER = (TL::ROWS * DCG_B + NT - 1) / NT;
   __shared__ T out[BC * NT];
   const int tid = threadIdx.x, l = tid % NCORNER, cell = tid / NCORNER;
@@ -2348,7 +2787,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
       if constexpr (OP == 4)
 #pragma unroll
         for (int i = 0; i < BC; ++i) vh[i] = slot >= 0 ? v[(size_t)slot * DCG_B + i] : T(0);
-      double uh[OP == 1 ? BC : 1];
+%CORNER_OP_DIRECTION%      double uh[OP == 1 ? BC : 1];
       butterfly(u, sd);
 #pragma unroll
       for (int i = 0; i < BC; ++i) {
@@ -2373,7 +2812,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
 #pragma unroll
         for (int n = 0; n < NEP; ++n) o[EPI[n]] += ca * dp[n] * (kap[EPK[n]] * uh[EPJ[n]]);
         butterfly(o, sg);
-      } else if constexpr (OP == 4) {
+      } else if constexpr (OP == 4 || OP == 5) {
         butterfly(vh, sg);
         T q[BC];
 #pragma unroll
@@ -2455,7 +2894,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
         } else if constexpr (OP == 1) {
           const T b = v ? v[at] : T(0);  // the vector passed as v is the base
           y[at] = b + (i < BC ? sum : T(0));
-        } else {
+%CORNER_OP_ROW%        } else {
           const T acc = i < BC ? sum : v[at];  // padding species: identity rows
           y[at] = acc;
           if (part) {
@@ -2467,7 +2906,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
       __syncthreads();
     }
   }
-  if constexpr (OP == 4) {
+%CORNER_OP_END%  if constexpr (OP == 4) {
     if (part) {
       // workgroup sums of the two partial dots (fixed order)
       __shared__ double red[2 * (NT / 64)];
@@ -2508,6 +2947,67 @@ extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
 }
 )";
 
+// the fused operator launch in the corner form: its reductions first, then
+// the lanes' directions, the rows and the partials
+const char* kCornerOpBegin = R"(  __shared__ double red5[OP == 5 ? 3 * (NT / 64) : 1];
+  BicgScalars sc;
+  sc.alpha = sc.beta = sc.omega = 0.0;
+  const int kmode = OP == 5 ? op->mode : 0;
+  if constexpr (OP == 5) {
+    if (kmode == 1) {
+      if (!finish_stage<NT, 2>(sc, op->in, op->out, lead, op->fin, op->nfin, op->fstride, 4, red5)) return;
+    } else if (kmode == 2) {
+      if (!finish_stage<NT, 1>(sc, op->in, op->out, lead, op->fin, op->nfin, op->fstride, 1, red5)) return;
+    }
+  }
+  const auto KA = (dcg_gp<const T>)(const T*)(OP == 5 ? op->a : nullptr);
+  const auto KP = (dcg_gp<const T>)(const T*)(OP == 5 ? op->b : nullptr);
+  const auto KC = (dcg_gp<const T>)(const T*)(OP == 5 ? op->c : nullptr);
+  // entry k of the direction before the preconditioner
+  auto kdir = [&](size_t k) -> T {
+    if (kmode == 1) return (T)((double)KA[k] + sc.beta * ((double)KP[k] - sc.omega * (double)KC[k]));
+    if (kmode == 2) return (T)((double)KA[k] - sc.alpha * (double)KC[k]);
+    return KA[k];
+  };
+  double e0 = 0.0, e1 = 0.0, e2 = 0.0;
+)";
+const char* kCornerOpDirection = R"(      if constexpr (OP == 5) {
+        T q[BC];
+#pragma unroll
+        for (int i = 0; i < BC; ++i) vh[i] = q[i] = slot >= 0 ? kdir((size_t)slot * DCG_B + i) : T(0);
+        if (slot >= 0 && kmode) precondition(op->jac, op->dinv, slot, q, vh);
+      }
+)";
+const char* kCornerOpRow = R"(        } else if constexpr (OP == 5) {
+          const T q = kdir(at);
+          // padding species: identity rows (their directions are zero in a solve)
+          const T acc = i < BC ? sum : kmode ? T(0) : q;
+          y[at] = acc;
+          if (kmode == 1) {
+            ((dcg_gp<T>)(T*)op->d)[at] = i < BC ? q : T(0);
+            e0 += (double)acc * (double)((dcg_gp<const T>)(const T*)op->w)[at];
+          } else if (kmode == 2) {
+            e0 += (double)acc * (double)q;
+            e1 += (double)acc * (double)acc;
+            e2 += (double)q * (double)q;
+          }
+)";
+const char* kCornerOpEnd = R"(  if constexpr (OP == 5) {
+    if (kmode) put_partials<NT>(*op, at0, e0, e1, e2, red5);
+  }
+)";
+const char* kCornerKrylov = R"(
+template <typename TL, typename T>
+__device__ __forceinline__ void corner_krylov(int tile, int at, dcg_gp<const int> g2l,
+                                              dcg_gp<const unsigned char> cmask, dcg_gp<const double> lin,
+                                              const KrylovOp& op, bool lead, dcg_gp<const double> tca, int n0, int n1,
+                                              int n2, const double* prm) {
+  corner_body<TL, 5, T>(tile, g2l, cmask, lin, (dcg_gp<const T>)(const T*)op.a, (dcg_gp<T>)(T*)op.y, nullptr, tca[0],
+                        tca[2], tca[1], n0, n1, n2, tca[3], tca[4], tca[5], tca[6], tca[7], tca[8], prm, false, nullptr,
+                        nullptr, nullptr, &op, lead, at);
+}
+)";
+
 // the corner form of the point-storage entry points (kTiledPoints): pc is the
 // linearisation point, tca = (t, ca, cm, origin, spacing) as the set-up left it
 const char* kCornerPoints = R"(
@@ -2523,23 +3023,6 @@ extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
       (%C%::dcg_gp<const double>)x, nullptr, (%C%::dcg_gp<double>)r, (%C%::dcg_gp<double>)lin, t, cm, ca, n0, n1, n2,
       ox, oy, oz, hx, hy, hz, prm, (mode & 16) != 0, nullptr, nullptr, nullptr);
 }
-#define DCG_CORNER_ENTRY(NAME, T, TL)                                                                             \
-  extern "C" __global__ void __launch_bounds__(TL::NT)                                                            \
-  NAME(const int* __restrict__ tiles, int ntile, const int* __restrict__ g2l,                                     \
-       const unsigned char* __restrict__ cmask, const double* __restrict__ lin, const T* __restrict__ v,           \
-       T* __restrict__ y, const double* __restrict__ tca, int n0, int n1, int n2, const double* __restrict__ prm,  \
-       const int* __restrict__ stop, const T* w1, const T* w2, double* __restrict__ part) {                       \
-    if (stop && *stop) return;                                                                                    \
-    const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
-    if (c >= ntile) return;                                                                                       \
-    %C%::corner_body<TL, 4, T>(tiles[c], (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,    \
-                               (%C%::dcg_gp<const double>)lin, (%C%::dcg_gp<const T>)v, (%C%::dcg_gp<T>)y,         \
-                               nullptr, tca[0], tca[2], tca[1], n0, n1, n2, tca[3], tca[4], tca[5], tca[6],       \
-                               tca[7], tca[8], prm, false, (%C%::dcg_gp<const T>)w1, (%C%::dcg_gp<const T>)w2,    \
-                               part ? part + 2 * (size_t)c : nullptr);                                            \
-  }
-%CORNER_ENTRIES%
-#undef DCG_CORNER_ENTRY
 )";
 
 // batched residual, set-up and apply of the corner form (as kTiledBatch and
@@ -2604,6 +3087,140 @@ extern "C" __global__ void __launch_bounds__(%C%::CornerShape0::NT)
 
 }  // namespace
 
+// The facet rows of a fused operator launch: a lane per slot on an interface
+// (or outflow boundary) adds its facets' terms to its row of y, so one launch
+// takes every facet kind and colour, and what it changes in the partial sums
+// goes into partials of its own.  Few rows, so the launch is a chain of
+// dependent loads: four waves share a row's facets (they are ordered by kind,
+// so a wave mostly runs one kind) and all slots of a facet are loaded at once.
+// 1024^2 with a circular interface, FP64: 6 launches per apply 29 us, one lane
+// per row 26 us, four waves 17 us, loads together 9.5 us.
+static const char* kFacetRows = R"(
+struct FacetRows {
+  int nslot;
+  const int *slot, *ptr;
+  const int3* ent;
+  const int* fint[%KINDS%];
+  const double* fdbl[%KINDS%];
+};
+static_assert(sizeof(FacetRows) == %FACET_ROWS_BYTES%, "facet rows layout");
+template <typename T>
+__device__ __forceinline__ void facet_rows(const FacetRows& F, const double* __restrict__ lin, const KrylovOp& op,
+                                           const double* __restrict__ tca, const double* __restrict__ prm) {
+  double alpha = 0.0;
+  if (op.mode) {
+    if (op.in->done) return;
+    alpha = op.in->alpha;
+  }
+  const T *A = (const T*)op.a, *C = (const T*)op.c, *D = (const T*)op.d, *W = (const T*)op.w;
+  T* Y = (T*)op.y;
+  auto before = [&](size_t k) -> T {
+    if (op.mode == 1) return D[k];
+    if (op.mode == 2) return (T)((double)A[k] - alpha * (double)C[k]);
+    return A[k];
+  };
+  // the direction at N slots at once, so that no load waits for another slot's
+  const T* P = op.mode == 1 ? D : A;
+  const T* S = op.mode == 2 ? C : P;
+  auto dir = [&](const int* sl, auto& o, auto count) {
+    constexpr int N = decltype(count)::value;
+    T q[N][DCG_B], c[N][DCG_B];
+#pragma unroll
+    for (int f = 0; f < N; ++f)
+#pragma unroll
+      for (int i = 0; i < DCG_B; ++i) {
+        q[f][i] = P[(size_t)sl[f] * DCG_B + i];
+        c[f][i] = S[(size_t)sl[f] * DCG_B + i];
+      }
+#pragma unroll
+    for (int f = 0; f < N; ++f)
+#pragma unroll
+      for (int i = 0; i < DCG_B; ++i) q[f][i] = op.mode == 2 ? (T)((double)q[f][i] - alpha * (double)c[f][i]) : q[f][i];
+    if (op.mode && op.jac == 2) {
+#pragma unroll
+      for (int f = 0; f < N; ++f)
+#pragma unroll
+        for (int i = 0; i < DCG_B; ++i)
+          o[f][i] = (double)(T)(op.dinv[(size_t)sl[f] * DCG_B + i] * (double)q[f][i]);
+    } else if (op.mode && op.jac == 1) {
+#pragma unroll
+      for (int f = 0; f < N; ++f)
+#pragma unroll
+        for (int i = 0; i < DCG_B; ++i) {
+          double v = 0.0;
+#pragma unroll
+          for (int j = 0; j < DCG_B; ++j) v += op.dinv[((size_t)sl[f] * DCG_B + i) * DCG_B + j] * (double)q[f][j];
+          o[f][i] = (double)(T)v;
+        }
+    } else {
+#pragma unroll
+      for (int f = 0; f < N; ++f)
+#pragma unroll
+        for (int i = 0; i < DCG_B; ++i) o[f][i] = (double)q[f][i];
+    }
+  };
+  __shared__ double red[12], part[3][DCG_B][64];
+  double e[3] = {0.0, 0.0, 0.0}, acc[DCG_B];
+  T old[DCG_B], mid[DCG_B];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n = blockIdx.x * 64 + lane;
+  const double t = tca[0], ca = tca[1];
+  const bool row = n < F.nslot && ca != 0.0;
+  const int s = row ? F.slot[n] : 0;
+#pragma unroll
+  for (int i = 0; i < DCG_B; ++i) {
+    acc[i] = 0.0;
+    old[i] = mid[i] = (T)0;
+    if (row && wave == 0) {
+      old[i] = Y[(size_t)s * DCG_B + i];
+      if (op.mode == 1) mid[i] = W[(size_t)s * DCG_B + i];
+      if (op.mode == 2) mid[i] = before((size_t)s * DCG_B + i);
+    }
+  }
+  if (row)
+    for (int k = F.ptr[n] + wave; k < F.ptr[n + 1]; k += 4) {
+      const int3 f = F.ent[k];
+%FACET_CASES%
+    }
+  if (wave)
+#pragma unroll
+    for (int i = 0; i < DCG_B; ++i) part[wave - 1][i][lane] = acc[i];
+  __syncthreads();
+  if (row && wave == 0) {
+#pragma unroll
+    for (int i = 0; i < DCG_B; ++i) {
+      const T now = (T)((double)old[i] + (((acc[i] + part[0][i][lane]) + part[1][i][lane]) + part[2][i][lane]));
+      Y[(size_t)s * DCG_B + i] = now;
+      const double d = (double)now - (double)old[i];
+      if (op.mode == 1) {
+        e[0] += d * (double)mid[i];
+      } else if (op.mode == 2) {
+        e[0] += d * (double)mid[i];
+        e[1] += d * ((double)now + (double)old[i]);
+      }
+    }
+  }
+  if (op.mode) {
+    group_sums<256, 3>(e, red);
+    if (threadIdx.x == 0) {
+      const int at = op.off + blockIdx.x;
+      op.part[at] = e[0];
+      if (op.mode == 2) {
+        op.part[op.pstride + at] = e[1];
+        op.part[2 * op.pstride + at] = e[2];
+      }
+    }
+  }
+}
+extern "C" __global__ void __launch_bounds__(256)
+dcg_facet_rows(FacetRows F, const double* lin, KrylovOp op, const double* tca, const double* prm) {
+  facet_rows<double>(F, lin, op, tca, prm);
+}
+extern "C" __global__ void __launch_bounds__(256)
+dcg_facet_rows_f(FacetRows F, const double* lin, KrylovOp op, const double* tca, const double* prm) {
+  facet_rows<float>(F, lin, op, tca, prm);
+}
+)";
+
 int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner) {
   // corner form: a lane per corner of a layer's cells
   if (corner) return (t[0] + 1) * (dim > 2 ? t[1] + 1 : 1) << dim;
@@ -2624,16 +3241,12 @@ std::vector<std::array<int, 3>> corner_tiles(int dim) {
   return {{63, 15, 1}, {31, 7, 1}};
 }
 
-// The corner form takes box cells in 2D and 3D whose equations suit the tiled
-// kernel (tile_eligible), with diffusion tensors diagonal in space (the sums
-// and differences of a cell's corners diagonalise no mixed derivatives) and
-// reactions that read no gradients, in blocks of more than 4 species: there
-// the tiled kernels keep a cell's corner values in LDS (40^3, 7 species:
-// residual 360 us, Jacobian pass 3,330 us).  Up to 4 species a thread holds a
-// whole cell in registers, without the lane exchanges.
-bool corner_eligible(const ModelSpec& m, const Grid& g, int comp) {
-  if (g.unstructured || !g.cube || g.dim < 2 || m.comp_species[comp].size() <= 4 || !tile_eligible(m, comp))
-    return false;
+// The evaluated forms take box cells whose equations suit the tiled kernel
+// (tile_eligible), with diffusion tensors diagonal in space (the sums and
+// differences of a cell's corners diagonalise no mixed derivatives) and
+// reactions that read no gradients.
+static bool box_form(const ModelSpec& m, const Grid& g, int comp) {
+  if (g.unstructured || !g.cube || !tile_eligible(m, comp)) return false;
   auto gradient_free = [](const Ex& e) {
     if (!e) return true;
     std::vector<std::string> vars;
@@ -2658,8 +3271,34 @@ bool corner_eligible(const ModelSpec& m, const Grid& g, int comp) {
   return true;
 }
 
+// The corner form is for 2D and 3D blocks of more than 4 species: there the
+// tiled kernels keep a cell's corner values in LDS (40^3, 7 species: residual
+// 360 us, Jacobian pass 3,330 us).  Up to 4 species a thread holds a whole
+// cell in registers, without the lane exchanges.
+bool corner_eligible(const ModelSpec& m, const Grid& g, int comp) {
+  return g.dim >= 2 && m.comp_species[comp].size() > 4 && box_form(m, g, comp);
+}
+
+// Point applies of up to 4 species evaluate their coefficients where that
+// costs less than reading them: a stored coefficient is 8 bytes per point of
+// every cell, which at the 3.6 TB/s of the stored apply is the time of about
+// 50 FP64 instructions per point, halo cells counted; a third of that is the
+// line, since small meshes read the stored ones from cache and the FP32
+// apply reads 4 bytes.
+bool eval_eligible(const ModelSpec& m, const Grid& g, int comp) {
+  if (m.comp_species[comp].empty() || m.comp_species[comp].size() > 4 || !box_form(m, g, comp)) return false;
+  int cost = 0;
+  for (int s : m.comp_species[comp]) {
+    const auto& sp = m.species[s];
+    cost += expr::cost(sp.storage);
+    for (const auto& pj : sp.storage_jac) cost += expr::cost(pj.e) + 1;
+    for (const auto& pj : sp.reaction_jac) cost += expr::cost(pj.e) + 1;
+  }
+  return cost <= 16 * static_cast<int>(mc_pattern(m, comp).size());
+}
+
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
-                                                      std::vector<int>* waves) {
+                                                      bool eval, std::vector<int>* waves) {
   std::vector<std::array<int, 3>> out{setup_tile};
   if (waves) waves->assign(1, 1);
   if (species > 4) return out;  // corner values in LDS: the assembly tile only
@@ -2676,6 +3315,15 @@ std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species
   } else if (g.dim == 3) {
     cand = {{8, 4, 4}, {7, 7, 3}, {6, 5, 5}, {15, 3, 3}, {7, 7, 7}, {15, 7, 3}, {15, 7, 7}, {7, 7, 7}, {8, 4, 4}};
     wv = {1, 1, 1, 1, 1, 1, 1, 6, 6};  // (8 waves spill in 3D)
+  }
+  // evaluated applies hold more (95 to 115 registers): five waves per SIMD
+  // are the most without spills
+  if (eval && g.dim == 2) {
+    cand = {{15, 15, 1}, {31, 7, 1}, {31, 15, 1}, {15, 15, 1}};
+    wv = {1, 1, 1, 5};
+  } else if (eval && g.dim == 3) {
+    cand = {{8, 4, 4}, {7, 7, 3}, {15, 3, 3}, {7, 7, 7}, {15, 7, 7}, {7, 7, 7}};
+    wv = {1, 1, 1, 1, 1, 5};
   }
   for (size_t i = 0; i < cand.size(); ++i)
     if (cand[i] != setup_tile || wv[i] != 1) {
@@ -2698,6 +3346,20 @@ bool tile_eligible(const ModelSpec& m, int comp) {
   return true;
 }
 
+bool evaluates(const ModelSpec& m, const Layout& L) {
+  if (m.jacobian == JacobianType::Numerical && !m.is_linear) return false;
+  for (size_t c = 0; c < m.comp_names.size(); ++c)
+    if (!m.comp_species[c].empty() && !corner_eligible(m, L.grid, static_cast<int>(c)) &&
+        !eval_eligible(m, L.grid, static_cast<int>(c)))
+      return false;
+  std::vector<std::tuple<int, int, bool>> kinds;
+  for (const auto& F : L.facets) {
+    const auto key = std::make_tuple(F.comp_in, F.comp_out, F.boundary);
+    if (std::find(kinds.begin(), kinds.end(), key) == kinds.end()) kinds.push_back(key);
+  }
+  return kinds.size() <= static_cast<size_t>(k::kFacetKinds);
+}
+
 std::array<int, 3> choose_tile(const Grid& g, int bc, int nmc) {
   // largest candidate whose LDS (staging + coefficient union) stays under 64 KiB
   std::vector<std::array<int, 3>> cand;
@@ -2717,7 +3379,7 @@ std::array<int, 3> choose_tile(const Grid& g, int bc, int nmc) {
 }
 
 std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::string& ns, const std::string& kname,
-                      std::array<int, 3> tile, bool geo, bool points, bool corner,
+                      std::array<int, 3> tile, bool geo, bool points, bool corner, bool eval,
                       const std::vector<std::array<int, 3>>& apply_tiles, const std::vector<int>& apply_waves) {
   const auto T = element_tables(geo ? unit_cell(g) : g);
   std::ostringstream o;
@@ -2831,33 +3493,16 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     o << "__device__ constexpr int KZJ[NKZ > 0 ? NKZ : 1] = " << arr(kzj) << ";\n";
     o << "__device__ constexpr int KZZ[NKZ > 0 ? NKZ : 1] = " << arr(kzz) << ";\n";
   }
-  o << "__device__ __forceinline__ void uniform_diffusion(double t, const double* __restrict__ prm, "
-       "double (&dv)[NDV > 0 ? NDV : 1]) {\n  (void)t; (void)prm; dv[0] = 0.0;\n";
-  for (int n = 0; n < ndv; ++n) o << "  dv[" << n << "] = " << dexpr[n] << ";\n";
-  o << "}\n";
-  o << "}  // namespace " << ns << "\n";
-  std::string body = kTiled;
-  if (geo && comp < 4) body += kTiledBatch;
-  replace_all(body, "%R_ENTRY%", corner ? "" : "DCG_TILE_ENTRY(%KERNEL%_r, 1)\n");
-  if (corner) {
-    body += kCorner;
-    if (points) body += kCornerPoints;
-    if (geo && comp < 4) body += kCornerBatch;
-    if (geo && comp < 4 && points) body += kCornerPointBatch;
-    const auto shapes = corner_tiles(d);
-    std::string cs, ce, cb;
-    for (size_t k2 = 0; k2 < shapes.size(); ++k2) {
-      const std::string id = std::to_string(k2), tl = ns + "::CornerShape" + id;
-      cs += "using CornerShape" + id + " = CornerTile<" + std::to_string(shapes[k2][0]) + ", " +
-            std::to_string(shapes[k2][1]) + ", " + std::to_string(shapes[k2][2]) + ">;\n";
-      ce += "DCG_CORNER_ENTRY(%KERNEL%_p" + id + ", double, " + tl + ")\n";
-      ce += "DCG_CORNER_ENTRY(%KERNEL%_pf" + id + ", float, " + tl + ")\n";
-      cb += "DCG_CORNER_BENTRY(%KERNEL%_pbatch" + id + ", double, v, " + tl + ")\n";
-      cb += "DCG_CORNER_BENTRY(%KERNEL%_pfbatch" + id + ", float, f, " + tl + ")\n";
-    }
+  // whether the point applies evaluate their coefficients (eval_eligible), and
+  // the tables of the evaluated forms
+  o << "constexpr bool EVAL = " << (eval ? "true" : "false") << ";\n";
+  o << "__device__ __forceinline__ void set_tca(double* tca, double t, double ca, double cm, double ox, double oy, "
+       "double oz, double hx, double hy, double hz) {\n  tca[0] = t; tca[1] = ca; tca[2] = cm; tca[3] = ox; "
+       "tca[4] = oy; tca[5] = oz; tca[6] = hx; tca[7] = hy; tca[8] = hz;\n}\n";
+  if (eval || corner) {
+    std::ostringstream ct;
     // diffusion per species pair: D_ij of an isotropic term (axis 3: all
     // axes) or of each axis; KH: the cell's sides (1: run-time spacing)
-    std::ostringstream ct;
     std::vector<int> pi, pj, pk;
     std::vector<std::string> pe;
     for (size_t i = 0; i < species.size(); ++i)
@@ -2877,6 +3522,28 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     ct << "__device__ constexpr int EPI[NEP > 0 ? NEP : 1] = " << ints(pi) << ";\n";
     ct << "__device__ constexpr int EPJ[NEP > 0 ? NEP : 1] = " << ints(pj) << ";\n";
     ct << "__device__ constexpr int EPK[NEP > 0 ? NEP : 1] = " << ints(pk) << ";\n";
+    // the point block's entries alone, as qp computes them
+    ct << "__device__ __forceinline__ void point_jacobian(const double (&u)[BC], double px, double py, double pz, "
+          "double t, double cm, double ca, double (&mc)[NMC > 0 ? NMC : 1], const double* __restrict__ prm) {\n"
+          "  (void)u; (void)px; (void)py; (void)pz; (void)t; (void)prm; mc[0] = 0.0;\n"
+          "  const double fm = FACQ(0) * cm, fa = FACQ(0) * ca;\n  (void)fm; (void)fa;\n";
+    for (size_t n = 0; n < nz.size(); ++n) {
+      ct << "  {\n    double s = 0.0;\n";
+      const int i = nz[n].first;
+      const auto& sp = m.species[species[i]];
+      auto E = [&](const Ex& e) { return expr::emit(e, vars, true); };
+      if (sp.storage && nz[n].second == i) ct << "    s += fm * " << E(sp.storage) << ";\n";
+      if (sp.storage)
+        for (const auto& pj2 : sp.storage_jac)
+          if (m.species[pj2.wrt].comp == comp && m.species[pj2.wrt].local == nz[n].second)
+            ct << "    s += fm * (" << E(pj2.e) << ") * u[" << i << "];\n";
+      if (sp.reaction)
+        for (const auto& pj2 : sp.reaction_jac)
+          if (m.species[pj2.wrt].comp == comp && m.species[pj2.wrt].local == nz[n].second)
+            ct << "    s -= fa * (" << E(pj2.e) << ");\n";
+      ct << "    mc[" << n << "] = s;\n  }\n";
+    }
+    ct << "}\n";
     // o = (point block) q, one statement per entry, in FP64 as the block is
     // (FP64 FMAs run at the FP32 rate; converting every entry would cost more)
     ct << "template <typename T>\n__device__ __forceinline__ void point_block(const double (&mc)[NMC > 0 ? NMC : 1], "
@@ -2891,27 +3558,60 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     ct << "__device__ __forceinline__ void pair_diffusion(double t, const double* __restrict__ prm, "
           "double (&dp)[NEP > 0 ? NEP : 1]) {\n  (void)t; (void)prm; dp[0] = 0.0;\n";
     for (size_t n = 0; n < pe.size(); ++n) ct << "  dp[" << n << "] = " << pe[n] << ";\n";
-    ct << "}\n__device__ __forceinline__ void set_tca(double* tca, double t, double ca, double cm, double ox, double oy, "
-          "double oz, double hx, double hy, double hz) {\n  tca[0] = t; tca[1] = ca; tca[2] = cm; tca[3] = ox; "
-          "tca[4] = oy; tca[5] = oz; tca[6] = hx; tca[7] = hy; tca[8] = hz;\n}\n";
-    replace_all(body, "%CORNER_TABLES%", ct.str());
+    ct << "}\n";
+    o << ct.str();
+  }
+  o << "__device__ __forceinline__ void uniform_diffusion(double t, const double* __restrict__ prm, "
+       "double (&dv)[NDV > 0 ? NDV : 1]) {\n  (void)t; (void)prm; dv[0] = 0.0;\n";
+  for (int n = 0; n < ndv; ++n) o << "  dv[" << n << "] = " << dexpr[n] << ";\n";
+  o << "}\n";
+  o << "}  // namespace " << ns << "\n";
+  std::string body = kTiled;
+  if (geo && comp < 4) body += kTiledBatch;
+  replace_all(body, "%EVAL_CELL%", eval ? kEvalCell : kNoEvalCell);
+  replace_all(body, "%R_ENTRY%", corner ? "" : "DCG_TILE_ENTRY(%KERNEL%_r, 1)\n");
+  if (corner) {
+    if (points) body += std::string(kEvalKrylov) + "}  // namespace %C%\n";
+    body += kCorner;
+    replace_all(body, "%CORNER_OP_PARAMS%", points ? ", const KrylovOp* op = nullptr, bool lead = false, int at0 = 0" : "");
+    replace_all(body, "%CORNER_OP_BEGIN%", points ? kCornerOpBegin : "");
+    replace_all(body, "%CORNER_OP_DIRECTION%", points ? kCornerOpDirection : "");
+    replace_all(body, "%CORNER_OP_ROW%", points ? kCornerOpRow : "");
+    replace_all(body, "%CORNER_OP_END%", points ? kCornerOpEnd : "");
+    if (points) body += std::string(kCornerPoints) + "namespace %C% {\n" + kCornerKrylov + kEvalKrylovEntries;
+    replace_all(body, "%EVAL_FN%", "corner_krylov");
+    if (geo && comp < 4) body += kCornerBatch;
+    if (geo && comp < 4 && points) body += kCornerPointBatch;
+    const auto shapes = corner_tiles(d);
+    std::string cs, ce, cb;
+    for (size_t k2 = 0; k2 < shapes.size(); ++k2) {
+      const std::string id = std::to_string(k2), tl = ns + "::CornerShape" + id;
+      cs += "using CornerShape" + id + " = CornerTile<" + std::to_string(shapes[k2][0]) + ", " +
+            std::to_string(shapes[k2][1]) + ", " + std::to_string(shapes[k2][2]) + ">;\n";
+      ce += "DCG_EVAL_ENTRY(%KERNEL%_e" + id + ", double, " + tl + ")\n";
+      ce += "DCG_EVAL_ENTRY(%KERNEL%_ef" + id + ", float, " + tl + ")\n";
+      cb += "DCG_CORNER_BENTRY(%KERNEL%_ebatch" + id + ", double, v, " + tl + ")\n";
+      cb += "DCG_CORNER_BENTRY(%KERNEL%_efbatch" + id + ", float, f, " + tl + ")\n";
+    }
     replace_all(body, "%CORNER_SHAPES%", cs);
-    replace_all(body, "%CORNER_ENTRIES%", ce);
+    replace_all(body, "%EVAL_ENTRIES%", ce);
     replace_all(body, "%CORNER_BENTRIES%", cb);
     replace_all(body, "%APPLY_SHAPES%", "");
   } else {
     if (points) body += kTiledPoints;
     if (geo && comp < 4 && points) body += kTiledPointBatch;
     // one point apply (and batched point apply) per candidate tile shape k:
-    // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k>
+    // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k> (_e.. where evaluated)
     std::string pe, pb;
+    const std::string en = eval ? "e" : "p";
     for (size_t k2 = 0; k2 < apply_tiles.size(); ++k2) {
       const std::string id = std::to_string(k2);
       const std::string tl = ns + "::ApplyShape" + id;
-      pe += "DCG_POINT_ENTRY(%KERNEL%_p" + id + ", double, " + tl + ")\n";
-      pe += "DCG_POINT_ENTRY(%KERNEL%_pf" + id + ", float, " + tl + ")\n";
-      pb += "DCG_PBATCH_ENTRY(%KERNEL%_pbatch" + id + ", double, v, pc, " + tl + ")\n";
-      pb += "DCG_PBATCH_ENTRY(%KERNEL%_pfbatch" + id + ", float, f, pc32, " + tl + ")\n";
+      const std::string entry = eval ? "DCG_EVAL_ENTRY" : "DCG_POINT_ENTRY";
+      pe += entry + "(%KERNEL%_" + en + id + ", double, " + tl + ")\n";
+      pe += entry + "(%KERNEL%_" + en + "f" + id + ", float, " + tl + ")\n";
+      pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "batch" + id + ", double, v, pc, " + tl + ")\n";
+      pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "fbatch" + id + ", float, f, " + (eval ? "pc, " : "pc32, ") + tl + ")\n";
     }
     // the candidate apply shapes as plain names (macro arguments hold no commas)
     std::string as;
@@ -2922,7 +3622,10 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
                                               false)) +
             ", " + std::to_string(k2 < apply_waves.size() ? apply_waves[k2] : 1) + ">;\n";
     replace_all(body, "%APPLY_SHAPES%", as);
-    replace_all(body, "%POINT_ENTRIES%", pe);
+    if (eval) body += std::string(kEvalKrylov) + kEvalKrylovCells + kEvalKrylovEntries;
+    replace_all(body, "%EVAL_FN%", "eval_krylov");
+    replace_all(body, "%POINT_ENTRIES%", eval ? "" : pe);
+    replace_all(body, "%EVAL_ENTRIES%", eval ? pe : "");
     replace_all(body, "%PBATCH_ENTRIES%", pb);
   }
   replace_all(body, "%C%", ns);
@@ -2938,11 +3641,19 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
   replace_all(pre, "%B%", std::to_string(L.B));
   replace_all(pre, "%GEO%", geo ? "1" : "0");
   replace_all(pre, "%UNS%", L.grid.unstructured ? "1" : "0");
+  // the fused Krylov launches' types and scalar update (bicg_scalars.hh)
+  replace_all(pre, "%KRYLOV%", points ? std::string(DCG_STR(DCG_BICG_STRUCT DCG_KRYLOV_OP_STRUCT)) +
+                                            "\nstatic_assert(sizeof(KrylovOp) == " +
+                                            std::to_string(sizeof(k::KrylovOp)) + ", \"operator arguments\");\n" +
+                                            DCG_STR(DCG_BICG_UPDATE) + "\n" + DCG_STR(DCG_KRYLOV_FINISH) + "\n"
+                                      : std::string());
+  replace_all(pre, "DCG_DEV", "__device__ __forceinline__");
   replace_all(pre, "%ASM_BYTES%", std::to_string(sizeof(k::AsmMember)));
   replace_all(pre, "%PCM_BYTES%", std::to_string(sizeof(k::PcMember)));
   std::ostringstream src;
   src << pre;
   const bool numerical = spec.jacobian == JacobianType::Numerical && !spec.is_linear;
+  const bool all_eval = evaluates(spec, L);
   for (size_t c = 0; c < spec.comp_names.size(); ++c) {
     if (spec.comp_species[c].empty()) {
       out.volume_kernel.push_back("");
@@ -2953,6 +3664,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       out.tile_dims.push_back({0, 0, 0});
       out.point_words.push_back(0);
       out.corner.push_back(0);
+      out.eval.push_back(0);
       out.apply_threads.push_back({});
       continue;
     }
@@ -2967,17 +3679,19 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       std::string tk = "dcg_tile_" + std::to_string(c);
       std::vector<int> waves, threads;
       const int nsp = static_cast<int>(spec.comp_species[c].size());
-      const bool corner = corner_eligible(spec, L.grid, static_cast<int>(c));
+      const bool corner = corner_eligible(spec, L.grid, static_cast<int>(c)) && (!points || all_eval);
+      const bool eval = points && all_eval;
       std::vector<std::array<int, 3>> shapes;
       if (points && corner) {
         shapes = corner_tiles(L.grid.dim);
         waves.assign(shapes.size(), 1);
       } else if (points) {
-        shapes = apply_tile_candidates(L.grid, nsp, tile, &waves);
+        shapes = apply_tile_candidates(L.grid, nsp, tile, eval, &waves);
       }
       for (const auto& t : shapes) threads.push_back(apply_tile_threads(L.grid.dim, t, nsp, corner));
-      src << gen_tiled(spec, L.grid, static_cast<int>(c), ns, tk, tile, geo, points, corner, shapes, waves);
+      src << gen_tiled(spec, L.grid, static_cast<int>(c), ns, tk, tile, geo, points, corner, eval && !corner, shapes, waves);
       out.corner.push_back(corner ? 1 : 0);
+      out.eval.push_back(eval ? 1 : 0);
       out.apply_threads.push_back(threads);
       out.tile_kernel.push_back(tk);
       out.apply_tiles.push_back(shapes);
@@ -2985,7 +3699,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       out.tile_batch_kernel.push_back(geo && c < 4 ? tk + "_batch" : "");
       out.tile_dims.push_back(tile);
       const int nq = static_cast<int>(element_rule(L.grid.dim, L.grid.cube).w.size());
-      out.point_words.push_back(points && !corner ? L.grid.nclass * nq *
+      out.point_words.push_back(points && !eval ? L.grid.nclass * nq *
                                                         static_cast<int>(mc_pattern(spec, static_cast<int>(c)).size())
                                                   : 0);
     } else {
@@ -2996,6 +3710,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       out.tile_dims.push_back({0, 0, 0});
       out.point_words.push_back(0);
       out.corner.push_back(0);
+      out.eval.push_back(0);
       out.apply_threads.push_back({});
     }
   }
@@ -3016,6 +3731,21 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
     std::string ns = "fac" + std::to_string(ci) + "_" + std::to_string(co) + (bnd ? "b" : "i");
     src << gen_facet(spec, L.grid, ci, co, bnd, ns, fk.name, numerical, fk);
     out.facet_kernels.push_back(fk);
+  }
+  // evaluated applies take the facets in one launch per operator
+  out.fused = points && all_eval;
+  if (out.fused && !out.facet_kernels.empty()) {
+    std::string body = kFacetRows, cases;
+    for (size_t k2 = 0; k2 < out.facet_kernels.size(); ++k2) {
+      const auto& fk = out.facet_kernels[k2];
+      cases += "      if (f.x == " + std::to_string(k2) + ") fac" + std::to_string(fk.comp_in) + "_" +
+               std::to_string(fk.comp_out) + (fk.boundary ? "b" : "i") + "::facet_row(F.fint[" + std::to_string(k2) +
+               "], F.fdbl[" + std::to_string(k2) + "], f.y, f.z, lin, t, ca, prm, dir, acc);\n";
+    }
+    replace_all(body, "%FACET_CASES%", cases);
+    replace_all(body, "%KINDS%", std::to_string(k::kFacetKinds));
+    replace_all(body, "%FACET_ROWS_BYTES%", std::to_string(sizeof(k::FacetRows)));
+    src << body;
   }
   out.source = src.str();
   return out;

@@ -37,16 +37,21 @@ struct GeneratedSource {
   // every cell of the grid, word-major: pc[word * cells + cell]
   std::vector<int> point_words;
   // candidate tile shapes of the point apply per compartment (entry points
-  // <tile_kernel>_p<k>, _pf<k> and the batched _pbatch<k>, _pfbatch<k>);
+  // <tile_kernel>_p<k>, _pf<k> and the batched _pbatch<k>, _pfbatch<k>; see
+  // eval);
   // the first is the assembly tile
   std::vector<std::vector<std::array<int, 3>>> apply_tiles;
   // per compartment and candidate: the waves per SIMD its registers are
   // bounded for (1: none), and the workgroup size
   std::vector<std::vector<int>> apply_waves, apply_threads;
-  // compartments in the corner form: the residual and the point set-up run
-  // over corner_tiles(dim).front(), and the point applies evaluate their
-  // coefficients at the linearisation point (no stored words)
-  std::vector<char> corner;
+  // compartments whose point applies evaluate their coefficients at the
+  // linearisation point (no stored words; entry points _e<k>, _ef<k>,
+  // _ebatch<k>, _efbatch<k>), and those of them in the corner form, whose
+  // residual and point set-up run over corner_tiles(dim).front()
+  std::vector<char> eval, corner;
+  // point storage evaluates everywhere and the facets have row form
+  // (dcg_facet_rows, _f): BiCGSTAB runs on fused operator launches
+  bool fused = false;
   std::vector<FacetKernel> facet_kernels;
 };
 
@@ -62,12 +67,19 @@ constexpr int kGeoWords = 8;
 bool tile_eligible(const ModelSpec& m, int comp);
 // tile shapes the point apply is generated for (the set-up tile first)
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
-                                                      std::vector<int>* waves = nullptr);
+                                                      bool eval, std::vector<int>* waves = nullptr);
 // workgroup size of the point apply with tile t (row vertices along x, y, z)
 int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner);
+// the compartment's point applies evaluate their coefficients (blocks of up
+// to 4 species)
+bool eval_eligible(const ModelSpec& m, const Grid& g, int comp);
 // the compartment's kernels take the corner form, and its tile shapes
 bool corner_eligible(const ModelSpec& m, const Grid& g, int comp);
 std::vector<std::array<int, 3>> corner_tiles(int dim);
+// every compartment with species is one or the other, and its facets' kinds
+// fit one launch: point storage then evaluates everywhere (all or nothing, as
+// the fused operator launches take the place of the whole iteration)
+bool evaluates(const ModelSpec& m, const Layout& L);
 
 // points: also emit the point-coefficient Jacobian entry points (_q, _p, _pf)
 // of every tiled compartment

@@ -490,9 +490,43 @@ static std::string num(double v) {
   return "(" + s + ")";
 }
 
-std::string emit(const Ex& e, const std::map<std::string, std::string>& map) {
+// constants, run-time parameters and time: the same at every point of a launch
+static bool uniform(const Ex& e) {
+  std::vector<std::string> vars;
+  collect_vars(e, vars);
+  for (const auto& v : vars)
+    if (v != "time" && v.rfind("$", 0) != 0) return false;
+  return true;
+}
+
+int cost(const Ex& e) {
+  if (!e) return 0;
+  int c = 0;
+  for (const auto& a : e->args) c += cost(a);
+  double p = 0.0;
+  switch (e->kind) {
+    case Kind::Const:
+    case Kind::Var: return 0;
+    case Kind::Div: return uniform(e->args[1]) ? cost(e->args[0]) + 1 : c + 14;
+    case Kind::Pow:
+      return is_const(e->args[1], &p) && (p == 2.0 || p == 3.0) ? c * static_cast<int>(p) + static_cast<int>(p) - 1
+                                                                : c + 100;
+    case Kind::Mod: return c + 40;
+    case Kind::Call: {
+      const std::string& f = e->name;
+      return c + (f == "min" || f == "max" || f == "abs" || f == "sign" ? 2 : f == "sqrt" ? 20 : 60);
+    }
+    case Kind::Neg:
+    case Kind::Add:
+    case Kind::Sub:
+    case Kind::Mul: return c + 1;
+    default: return c + 2;
+  }
+}
+
+std::string emit(const Ex& e, const std::map<std::string, std::string>& map, bool reciprocals) {
   if (!e) return "0.0";
-  auto E = [&](int i) { return emit(e->args[i], map); };
+  auto E = [&](int i) { return emit(e->args[i], map, reciprocals); };
   switch (e->kind) {
     case Kind::Const: return num(e->value);
     case Kind::Var: {
@@ -505,7 +539,9 @@ std::string emit(const Ex& e, const std::map<std::string, std::string>& map) {
     case Kind::Add: return "(" + E(0) + " + " + E(1) + ")";
     case Kind::Sub: return "(" + E(0) + " - " + E(1) + ")";
     case Kind::Mul: return "(" + E(0) + " * " + E(1) + ")";
-    case Kind::Div: return "(" + E(0) + " / " + E(1) + ")";
+    case Kind::Div:
+      if (reciprocals && uniform(e->args[1])) return "(" + E(0) + " * (1.0 / " + E(1) + "))";
+      return "(" + E(0) + " / " + E(1) + ")";
     case Kind::Mod: return "fmod(" + E(0) + ", " + E(1) + ")";
     case Kind::Pow: {
       double p;

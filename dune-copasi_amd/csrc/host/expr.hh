@@ -65,7 +65,12 @@ void collect_vars(const Ex& e, std::vector<std::string>& out);
 Ex derivative(const Ex& e, const std::string& var);
 
 // C++ source for the device; `map` renames variables to C expressions.
-std::string emit(const Ex& e, const std::map<std::string, std::string>& map);
+// reciprocals: a division by something uniform (constants, parameters, time)
+// multiplies by its reciprocal, which is computed once per thread.
+std::string emit(const Ex& e, const std::map<std::string, std::string>& map, bool reciprocals = false);
+
+// FP64 instructions of one evaluation on the device, roughly (with reciprocals)
+int cost(const Ex& e);
 
 // Host evaluation with variables looked up in `vars` (missing -> error).
 double evaluate(const Ex& e, const std::map<std::string, double>& vars);

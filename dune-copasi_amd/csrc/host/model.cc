@@ -5,6 +5,7 @@
 #include <cstdlib>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 namespace dcopasi {
 
@@ -206,13 +207,13 @@ void Model::build(const std::string& ini, const std::string& overrides) {
     else if (cfg_.precond == Preconditioner::ILU0) why = "an ILU0 preconditioner";
     else if (!all_tile_eligible()) why = "compartments outside the tiled kernel";
     if (st == "points" && !why.empty()) throw NotImplemented("linear_solver.storage = points with " + why);
-    // auto: box cells, with blocks of up to 4 species or in the corner form
-    // (40^3, 7 species, FP32 operator: apply 27 us against 83 us for the
-    // SpMV, and no Jacobian pass of 3.3 ms; larger blocks outside the corner
-    // form keep their corner sums in LDS, where the SpMV is faster)
-    bool suits = L_.grid.cube;
-    for (size_t c = 0; c < L_.comps.size(); ++c)
-      suits = suits && (L_.comps[c].b <= 4 || corner_eligible(spec_, L_.grid, static_cast<int>(c)));
+    // auto: box cells, with blocks of up to 4 species or evaluated
+    // coefficients (40^3, 7 species, FP32 operator: apply 27 us against 83 us
+    // for the SpMV, and no Jacobian pass of 3.3 ms; larger blocks outside the
+    // corner form keep their corner sums in LDS, where the SpMV is faster)
+    int bmax = 0;
+    for (const auto& C : L_.comps) bmax = std::max(bmax, C.b);
+    const bool suits = L_.grid.cube && (bmax <= 4 || evaluates(spec_, L_));
     cfg_.points = why.empty() && (st == "points" || (st == "auto" && suits));
   }
   {
@@ -263,8 +264,8 @@ bool Model::all_tile_eligible() const {
   return true;
 }
 
-bool Model::any_corner() const {
-  for (char c : gen_.corner)
+bool Model::any_eval() const {
+  for (char c : gen_.eval)
     if (c) return true;
   return false;
 }
@@ -409,6 +410,7 @@ void Model::setup_device() {
   }
   // facet records per facet kernel, grouped by colour
   facet_dev_.resize(gen_.facet_kernels.size());
+  std::map<int, std::vector<int3>> frow;  // per slot: (kind, record, row)
   for (size_t k = 0; k < gen_.facet_kernels.size(); ++k) {
     const auto& fk = gen_.facet_kernels[k];
     std::vector<int> fi;
@@ -420,6 +422,11 @@ void Model::setup_device() {
       for (int f = L_.facet_color_ptr[col]; f < L_.facet_color_ptr[col + 1]; ++f) {
         const Facet& F = L_.facets[f];
         if (F.comp_in != fk.comp_in || F.comp_out != fk.comp_out || F.boundary != fk.boundary) continue;
+        if (gen_.fused)
+          for (int v = 0; v < fk.nvf; ++v) {
+            frow[F.slot_in[v]].push_back(make_int3(static_cast<int>(k), count, v));
+            if (!F.boundary) frow[F.slot_out[v]].push_back(make_int3(static_cast<int>(k), count, fk.nvf + v));
+          }
         for (int v = 0; v < fk.nvf; ++v) fi.push_back(F.slot_in[v]);
         for (int v = 0; v < fk.nvf; ++v) fi.push_back(F.boundary ? F.slot_in[v] : F.slot_out[v]);
         auto pos = [&](int rs, int cs) -> int {
@@ -450,6 +457,27 @@ void Model::setup_device() {
     }
     dev.fint.upload(fi, stream_);
     dev.fdbl.upload(fd, stream_);
+    if (gen_.fused) {
+      frows_.fint[k] = dev.fint.get();
+      frows_.fdbl[k] = dev.fdbl.get();
+    }
+  }
+  if (!frow.empty()) {
+    std::vector<int> fslot, fptr{0};
+    std::vector<int3> fent;
+    for (const auto& [slot, ents] : frow) {
+      fslot.push_back(slot);
+      fent.insert(fent.end(), ents.begin(), ents.end());
+      fptr.push_back(static_cast<int>(fent.size()));
+    }
+    frow_slot_.upload(fslot, stream_);
+    frow_ptr_.upload(fptr, stream_);
+    frow_ent_.upload(fent, stream_);
+    frows_.nslot = static_cast<int>(fslot.size());
+    frows_.slot = frow_slot_.get();
+    frows_.ptr = frow_ptr_.get();
+    frows_.ent = frow_ent_.get();
+    synchronize();  // the host lists end here
   }
   // lumped mass weights (integral of each hat function over its compartment)
   {
@@ -511,8 +539,8 @@ void Model::setup_device() {
     }
     pdiag_.resize(static_cast<size_t>(ns) * B * B);
     pc_tca_.resize(kTca);
-    // the facet terms and the corner form apply from the linearisation point
-    if (!L_.facets.empty() || any_corner()) lin_x_.resize(nv);
+    // the facet terms and the evaluated applies read the linearisation point
+    if (!L_.facets.empty() || any_eval()) lin_x_.resize(nv);
     dinv_.resize(static_cast<size_t>(ns) * B * B);
     std::vector<int> id(ns);
     for (long i = 0; i < ns; ++i) id[i] = static_cast<int>(i);
@@ -538,8 +566,11 @@ void Model::setup_device() {
   // region: they are finalised after the next operator launch)
   spart_off_ = std::max<size_t>(std::max<size_t>(2 * nparts, 2 * ntiles_all + 16), 8 * 1024 + 64);
   part_.resize(spart_off_ + static_cast<size_t>((L_.nslot + 255) / 256) + 64);
+  if (gen_.fused)
+    kpart_.resize(4 * (ntiles_all + static_cast<size_t>(frows_.nslot + 63) / 64) +
+                  2 * static_cast<size_t>(k::bicg_fused_xr_parts(static_cast<int>(ns))) + 8);
   scalar_out_.resize(16);
-  sc_.resize(1);
+  sc_.resize(4);
   status_.resize(4);
   k::fill(u_.get(), 0.0, static_cast<long>(nv), stream_);
   k::fill(status_.get(), 0, 4, stream_);
@@ -689,7 +720,7 @@ void Model::tune_points() {
     }
   for (int i = 0; i < 4; ++i) k::fill(kv_[i].get(), 0.0, L_.nslot * L_.B, stream_);
   k::fill(pc_tca_.get(), 0.0, static_cast<long>(kTca), stream_);
-  if (any_corner()) k::fill(lin_x_.get(), 0.0, L_.nslot * L_.B, stream_);
+  if (any_eval()) k::fill(lin_x_.get(), 0.0, L_.nslot * L_.B, stream_);
   // the eviction copy: only where the coefficients could stay cached
   constexpr long kFlushBytes = 384L << 20;
   DeviceArray<char> fa, fb;
@@ -717,7 +748,8 @@ void Model::tune_points() {
         apply_shape_[c] = static_cast<int>(k2);
         if (fa.size()) k::probe_copy(fa.get(), fb.get(), kFlushBytes, stream_);
         DCG_HIP(hipEventRecord(e0, stream_));
-        launch_points_apply(kv_[0].get(), kv_[1].get(), nullptr, false, kv_[2].get(), kv_[3].get(), part_.get());
+        if (fused()) launch_points_apply(kv_[0].get(), kv_[1].get(), nullptr, false);
+        else launch_points_apply(kv_[0].get(), kv_[1].get(), nullptr, false, kv_[2].get(), kv_[3].get(), part_.get());
         DCG_HIP(hipEventRecord(e1, stream_));
         DCG_HIP(hipEventSynchronize(e1));
         float t = 0.f;
@@ -758,8 +790,9 @@ void Model::compile_and_load() {
       if (cfg_.points) {
         pc_set_fn_[c] = module_->function(gen_.tile_kernel[c] + "_q");
         for (size_t k2 = 0; k2 < gen_.apply_tiles[c].size(); ++k2) {
-          pc_app_fns_[c].push_back(module_->function(gen_.tile_kernel[c] + "_p" + std::to_string(k2)));
-          pc_appf_fns_[c].push_back(module_->function(gen_.tile_kernel[c] + "_pf" + std::to_string(k2)));
+          const std::string name = gen_.tile_kernel[c] + (gen_.eval[c] ? "_e" : "_p");
+          pc_app_fns_[c].push_back(module_->function(name + std::to_string(k2)));
+          pc_appf_fns_[c].push_back(module_->function(name + "f" + std::to_string(k2)));
         }
         pc_app_fn_[c] = pc_app_fns_[c].front();
         pc_appf_fn_[c] = pc_appf_fns_[c].front();
@@ -771,6 +804,10 @@ void Model::compile_and_load() {
   for (const auto& fk : gen_.facet_kernels) {
     facet_fn_.push_back(module_->function(fk.name));
     facetf_fn_.push_back(cfg_.points ? module_->function(fk.name + "_f") : nullptr);
+  }
+  if (gen_.fused && frows_.nslot) {
+    facet_rows_fn_ = module_->function("dcg_facet_rows");
+    facet_rows_f_fn_ = module_->function("dcg_facet_rows_f");
   }
 }
 
@@ -927,7 +964,7 @@ void Model::launch_points_setup(const double* x, double t, double cm, double ca)
         corner ? apply_tile_threads(g.dim, corner_tiles(g.dim).front(), L_.comps[c].b, true) : 256);
     const int* g2l = comp_dev_[c].g2l.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
-    double* pc = corner ? lin_x_.get() : pc_[c].get();
+    double* pc = gen_.eval[c] ? lin_x_.get() : pc_[c].get();
     void* args[] = {&tiles, &g2l, &cmask, &x, &base, &t, &cm, &ca, &diag, &pc, &own_start, &own_mask,
                     &n0, &n1, &n2, &ox, &oy, &oz, &hx, &hy, &hz, &mode, &prm, &tca};
     DCG_HIP(hipModuleLaunchKernel(pc_set_fn_[c], grid, 1, 1, block, 1, 1, 0, stream_, args, nullptr));
@@ -963,6 +1000,15 @@ void Model::launch_points_setup(const double* x, double t, double cm, double ca)
 // written (the returned count is 0: the caller forms the dots).
 int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp32, const void* w1, const void* w2,
                                double* part) {
+  if (fused()) {
+    // a plain apply of the fused launches (nothing calls it with partials)
+    if (part || stop) throw Error("internal: plain operator launch with partials");
+    k::KrylovOp op{};
+    op.a = v;
+    op.y = y;
+    launch_krylov_op(op, fp32);
+    return 0;
+  }
   const Grid& g = L_.grid;
   int n0 = static_cast<int>(g.n[0]), n1 = g.dim > 1 ? static_cast<int>(g.n[1]) : 1;
   int n2 = g.dim > 2 ? static_cast<int>(g.n[2]) : 1;
@@ -973,7 +1019,7 @@ int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp3
     if (!pc_app_fn_[c] || comp_dev_[c].ntiles <= 0) continue;
     const int* g2l = comp_dev_[c].g2l_identity ? nullptr : comp_dev_[c].g2l.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
-    const void* pc = gen_.corner[c] ? static_cast<const void*>(lin_x_.get())
+    const void* pc = gen_.eval[c] ? static_cast<const void*>(lin_x_.get())
                      : fp32         ? static_cast<const void*>(pc32_[c].get())
                                     : static_cast<const void*>(pc_[c].get());
     double* pp = part && facet_fn_.empty() ? part + 2 * static_cast<size_t>(nparts) : nullptr;
@@ -1006,6 +1052,51 @@ int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp3
     }
   }
   return 0;
+}
+
+int Model::krylov_parts() const {
+  int n = (frows_.nslot + 63) / 64;
+  for (size_t c = 0; c < L_.comps.size(); ++c)
+    if (pc_app_fn_[c] && comp_dev_[c].ntiles > 0) n += comp_dev_[c].natiles[apply_shape_[c]];
+  return n;
+}
+
+// One operator launch of the fused iteration (k::KrylovOp): the compartments'
+// tiles one after the other in the partials, then the facet rows, which take
+// the scalars that the first compartment's launch has stored.
+int Model::launch_krylov_op(k::KrylovOp op, bool fp32) {
+  const Grid& g = L_.grid;
+  int n0 = static_cast<int>(g.n[0]), n1 = g.dim > 1 ? static_cast<int>(g.n[1]) : 1;
+  int n2 = g.dim > 2 ? static_cast<int>(g.n[2]) : 1;
+  const double* prm = prm_.get();
+  const double* tca = pc_tca_.get();
+  const double* lin = lin_x_.get();
+  op.pstride = krylov_parts();
+  op.off = 0;
+  op.lead = op.in != op.out;
+  for (size_t c = 0; c < L_.comps.size(); ++c) {
+    if (!pc_app_fn_[c] || comp_dev_[c].ntiles <= 0) continue;
+    const int* g2l = comp_dev_[c].g2l_identity ? nullptr : comp_dev_[c].g2l.get();
+    const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
+    const int k2 = apply_shape_[c];
+    const int* tiles = comp_dev_[c].atiles[k2].get();
+    int ntile = comp_dev_[c].natiles[k2];
+    void* args[] = {&tiles, &ntile, &g2l, &cmask, &lin, &op, &tca, &n0, &n1, &n2, &prm};
+    const unsigned grid = static_cast<unsigned>((ntile + 7) / 8 * 8);  // the kernel maps workgroups to XCD runs
+    DCG_HIP(hipModuleLaunchKernel(fp32 ? pc_appf_fns_[c][k2] : pc_app_fns_[c][k2], grid, 1, 1,
+                                  static_cast<unsigned>(gen_.apply_threads[c][k2]), 1, 1, 0, stream_, args, nullptr));
+    op.off += ntile;
+    op.lead = 0;
+  }
+  if (frows_.nslot) {
+    if (op.mode) op.in = op.out;  // the scalars after this launch's reduction
+    k::FacetRows rows = frows_;
+    void* args[] = {&rows, &lin, &op, &tca, &prm};
+    DCG_HIP(hipModuleLaunchKernel(fp32 ? facet_rows_f_fn_ : facet_rows_fn_,
+                                  static_cast<unsigned>((frows_.nslot + 63) / 64), 1, 1, 256, 1, 1, 0, stream_, args,
+                                  nullptr));
+  }
+  return op.pstride;
 }
 
 void Model::ensure_matrix() {
@@ -1644,6 +1735,122 @@ int Model::bicgstab32(const double* b, float* x, double rtol, int maxit, int* it
   return host.done == 1 ? 0 : host.done;
 }
 
+// BiCGSTAB on fused operator launches.  An iteration is two operator launches
+// (each forms its direction while it stages it and first finishes the
+// reduction of the launch before) and the x/r update; p and v alternate
+// between two buffers, since a tile's halo reads the old ones while its
+// neighbours store the new.  The scalars pass from launch to launch through
+// three slots (sc_[0] after the x/r update, [1], [2]) and a fourth for the
+// read-back.  Launches of an iteration, one compartment: 3 in place of 8; two
+// compartments with an interface: 7 in place of 22.
+template <typename V>
+int Model::bicgstab_fused(const double* b, V* x, double rtol, double abstol, int maxit, int* its) {
+  constexpr bool fp32 = std::is_same<V, float>::value;
+  const int B = L_.B;
+  const int ns = static_cast<int>(L_.nslot);
+  const long n = static_cast<long>(ns) * B;
+  V* w[9];
+  for (int i = 0; i < 9; ++i) {
+    if constexpr (fp32) w[i] = kf_[i].get();
+    else w[i] = kv_[i].get();
+  }
+  V *r = w[0], *rh = w[1], *p[2] = {w[2], w[4]}, *v[2] = {w[3], w[6]}, *t = w[7];
+  k::BicgScalars* sc = sc_.get();
+  k::BicgScalars host{};
+  host.tol = rtol;
+  host.abstol = abstol;
+  host.maxit = maxit;
+  DCG_HIP(hipMemcpyAsync(sc, &host, sizeof host, hipMemcpyHostToDevice, stream_));
+  const int nred = std::max(1, std::min(1024, static_cast<int>((n + 255) / 256)));
+  k::bicg_init<V>(n, b, x, r, rh, p[0], v[0], part_.get(), nred, sc, stream_);
+  const int jac = cfg_.precond == Preconditioner::Jacobi ? 2 : cfg_.precond == Preconditioner::VertexBlockJacobi ? 1 : 0;
+  const int np = krylov_parts(), nx = k::bicg_fused_xr_parts(ns);
+  double *pa = kpart_.get(), *pb = pa + np, *pc = pb + 3 * static_cast<size_t>(np);
+  const int kind = fp32 ? kPointApply32 : kPointApply64;
+  int cur = 0, nfin = 0;
+  // many partials are finished once instead of by every workgroup
+  auto finish = [&](k::KrylovOp& op, int stage) {
+    if (op.nfin <= k::kFinishParts) return;
+    k::bicg_finish(op.in, op.out, op.fin, op.nfin, op.fstride, stage, stream_);
+    op.in = op.out;
+    op.nfin = 0;
+  };
+  auto iteration = [&]() {
+    k::KrylovOp op{};
+    op.jac = jac;
+    op.dinv = dinv_.get();
+    op.mode = 1;
+    op.a = r;
+    op.b = p[cur];
+    op.c = v[cur];
+    op.d = p[1 - cur];
+    op.y = v[1 - cur];
+    op.w = rh;
+    op.in = sc;
+    op.out = sc + 1;
+    op.fin = pc;
+    op.nfin = nfin;
+    op.fstride = nx;
+    op.part = pa;
+    finish(op, 4);
+    prof_begin(kind);
+    launch_krylov_op(op, fp32);
+    prof_end(kind, point_apply_bytes(sizeof(V), 4));
+    cur = 1 - cur;
+    op.mode = 2;
+    op.b = op.d = nullptr;
+    op.w = nullptr;
+    op.c = v[cur];
+    op.y = t;
+    op.in = sc + 1;
+    op.out = sc + 2;
+    op.fin = pa;
+    op.nfin = np;
+    op.fstride = np;
+    op.part = pb;
+    finish(op, 1);
+    prof_begin(kind);
+    launch_krylov_op(op, fp32);
+    prof_end(kind, point_apply_bytes(sizeof(V), 1));
+    op.in = sc + 2;
+    op.out = sc;
+    op.fin = pb;
+    op.nfin = np;
+    finish(op, 2);
+    nfin = k::bicg_fused_xr<V>(B, ns, x, p[cur], v[cur], t, r, rh, dinv_.get(), jac, op.in, op.out, pb, op.nfin, np, pc,
+                               nx, stream_);
+  };
+  // iterations run in batches between read-backs of the scalars: the first
+  // as many as this solve took in the last time step (or the last solve)
+  const int slot = solve_index_++;
+  const int guess = slot < static_cast<int>(its_hint_.size()) ? its_hint_[slot] : last_krylov_its_;
+  const size_t mark = prof_mark(kind);
+  const int fixed = cfg_.readback_iterations;
+  int done_its = 0, batch = fixed ? fixed : std::max(2, std::min(guess, 64));
+  for (;;) {
+    for (int it = 0; it < batch; ++it) iteration();
+    done_its += batch;
+    k::bicg_peek(sc, sc + 3, pc, nx, nx, stream_);
+    DCG_HIP(hipMemcpyAsync(&host, sc + 3, sizeof host, hipMemcpyDeviceToHost, stream_));
+    synchronize();
+    if (host.done) break;
+    if (done_its > maxit + 4) {
+      host.done = 2;
+      break;
+    }
+    batch = fixed ? fixed : 4;
+  }
+  // both operator launches of every iteration ran (a breakdown keeps them all)
+  if (host.done == 1 || host.done == 2) prof_keep(kind, mark, 2L * host.iter);
+  *its = host.iter;
+  last_krylov_its_ = std::max(2, host.iter);
+  if (slot < kMaxSolveHints) {
+    if (slot >= static_cast<int>(its_hint_.size())) its_hint_.resize(slot + 1, 0);
+    its_hint_[slot] = last_krylov_its_;
+  }
+  return host.done == 1 ? 0 : host.done;
+}
+
 // Solve val_ * x = b to relative tolerance rtol.  FP64: one preconditioned
 // BiCGSTAB.  Mixed: FP32 BiCGSTAB on an FP32 copy of the matrix inside FP64
 // iterative refinement; the refinement residual b - A x is FP64.
@@ -1655,7 +1862,8 @@ int Model::krylov(const double* b, double* x, double rtol, int maxit, int* its, 
   *its = 0;
   *refinements = 0;
   const long n = L_.nslot * L_.B;
-  if (cfg_.precision == Precision::FP64) return bicgstab64(b, x, rtol, 0.0, maxit, its, w);
+  if (cfg_.precision == Precision::FP64)
+    return fused() ? bicgstab_fused<double>(b, x, rtol, 0.0, maxit, its) : bicgstab64(b, x, rtol, 0.0, maxit, its, w);
   if (use_points_) {
     for (size_t c = 0; c < pc_.size(); ++c)
       if (pc_[c].size()) k::to_float(static_cast<long>(pc_[c].size()), pc_[c].get(), pc32_[c].get(), stream_);
@@ -1679,7 +1887,8 @@ int Model::krylov(const double* b, double* x, double rtol, int maxit, int* its, 
     // tighter than what reaches the outer target
     double inner = std::max(cfg_.ir_inner_rtol, 0.5 * target / rn);
     int it = 0;
-    int rc = bicgstab32(res, d, std::min(inner, 0.5), maxit, &it);
+    int rc = fused() ? bicgstab_fused<float>(res, d, std::min(inner, 0.5), 0.0, maxit, &it)
+                     : bicgstab32(res, d, std::min(inner, 0.5), maxit, &it);
     *its += it;
     *refinements += 1;
     if (rc == 3) return 3;
@@ -1998,7 +2207,7 @@ double Model::point_apply_bytes(int value_bytes, int extra_vectors) const {
   const double N = static_cast<double>(L_.nslot), B = L_.B;
   double b = (2.0 + extra_vectors) * value_bytes * B * N;
   for (size_t c = 0; c < L_.comps.size(); ++c) {
-    if (gen_.corner[c])  // the linearisation point, class masks, slots
+    if (gen_.eval[c])  // the linearisation point, class masks, slots
       b += L_.comps[c].nslot * (8.0 * B + 4.0) + static_cast<double>(L_.comps[c].cells.size());
     if (!gen_.point_words[c]) continue;
     const double cells = static_cast<double>(L_.comps[c].cells.size());
@@ -2013,7 +2222,7 @@ double Model::point_setup_bytes() const {
   const double N = static_cast<double>(L_.nslot), B = L_.B;
   double b = 8.0 * B * N + 8.0 * B * B * N;
   for (size_t c = 0; c < L_.comps.size(); ++c) {
-    if (gen_.corner[c])  // the linearisation point written, class masks, slots
+    if (gen_.eval[c])  // the linearisation point written, class masks, slots
       b += L_.comps[c].nslot * (8.0 * B + 4.0) + static_cast<double>(L_.comps[c].cells.size());
     if (!gen_.point_words[c]) continue;
     const double cells = static_cast<double>(L_.comps[c].cells.size());
@@ -2201,6 +2410,7 @@ size_t Model::device_bytes() const {
   for (const auto& c : comp_dev_)
     b += c.cells.bytes() + c.cell_slots.bytes() + c.cell_mask.bytes() + c.g2l.bytes() + c.tiles.bytes() +
          c.cell_mask_grid.bytes() + c.rtiles.bytes();
+  b += kpart_.bytes() + frow_slot_.bytes() + frow_ptr_.bytes() + frow_ent_.bytes();
   for (const auto& f : facet_dev_) b += f.fint.bytes() + f.fdbl.bytes();
   return b;
 }
@@ -2243,7 +2453,7 @@ k::MemberView Model::view() const {
         v.pc32 = c < pc32_.size() ? pc32_[c].get() : nullptr;
         v.npc = static_cast<long>(pc_[c].size());
       }
-    if (any_corner()) v.npc = -1;  // no stored coefficients to convert
+    if (any_eval()) v.npc = -1;  // no stored coefficients to convert
   }
   v.v[k::kVU] = u_.get();
   v.v[k::kVHist] = hist_.get();

@@ -219,7 +219,7 @@ class Model {
   // compartments without a batched tile kernel, or facets: per-model launches
   bool needs_own_assembly() const;
   bool all_tile_eligible() const;
-  bool any_corner() const;
+  bool any_eval() const;
   // point-coefficient Jacobian: coefficients and diagonal blocks at x, and
   // y = J v from them (v, y FP64 or FP32 as fp32 says); stop as in launch_apply
   void launch_points_setup(const double* x, double t, double cm, double ca);
@@ -250,6 +250,16 @@ class Model {
   KrylovWork own_work();
   int bicgstab64(const double* b, double* x, double rtol, double abstol, int maxit, int* its, const KrylovWork& w);
   int bicgstab32(const double* b, float* x, double rtol, int maxit, int* its);
+  // the same iteration on fused operator launches (every compartment
+  // evaluates its coefficients): three launches per iteration and compartment
+  // set instead of eight and more
+  template <typename V>
+  int bicgstab_fused(const double* b, V* x, double rtol, double abstol, int maxit, int* its);
+  bool fused() const { return use_points_ && gen_.fused; }
+  // one operator launch over all compartments and facet rows; returns its
+  // partial count
+  int launch_krylov_op(k::KrylovOp op, bool fp32);
+  int krylov_parts() const;
   void precond_setup(const KrylovWork& w);
   bool jacobi_kind() const {
     return cfg_.precond == Preconditioner::Jacobi || cfg_.precond == Preconditioner::VertexBlockJacobi;
@@ -354,7 +364,7 @@ class Model {
   DeviceArray<double> weights_;  // lumped mass per slot (mass sums)
   DeviceArray<double> prm_;      // geometry words + run-time parameters
   DeviceArray<double> u_, hist_, r_, z_, xs_, packed_;
-  // matrix-free, interface terms and the corner form: the Newton iterate the
+  // matrix-free, interface terms and evaluated applies: the Newton iterate the
   // Jacobian is applied at, and its weights
   DeviceArray<double> lin_x_;
   double lin_t_ = 0.0, lin_cm_ = 0.0, lin_ca_ = 0.0;
@@ -366,8 +376,8 @@ class Model {
   std::vector<DeviceArray<float>> pc32_;
   DeviceArray<double> pdiag_;
   DeviceArray<int> diag_id_;
-  // (t, ca) of the point coefficients, read by the applies; the corner form
-  // also reads cm and the grid's origin and spacing (kTca words)
+  // (t, ca) of the point coefficients, read by the applies; evaluated
+  // ones also read cm and the grid's origin and spacing (kTca words)
   DeviceArray<double> pc_tca_;
   static constexpr size_t kTca = 9;
   bool use_points_ = false;  // the Krylov operator is the point-coefficient one
@@ -379,6 +389,13 @@ class Model {
   DeviceArray<double> part_, scalar_out_;
   size_t spart_off_ = 0;  // offset of the s-update's partial norms in part_
   DeviceArray<k::BicgScalars> sc_;
+  // fused launches: partials (first operator, second operator's three, the
+  // x/r update's two) and the facet rows
+  DeviceArray<double> kpart_;
+  DeviceArray<int> frow_slot_, frow_ptr_;
+  DeviceArray<int3> frow_ent_;
+  k::FacetRows frows_;
+  hipFunction_t facet_rows_fn_ = nullptr, facet_rows_f_fn_ = nullptr;
   DeviceArray<int> status_;
   k::SpmvPlan plan_, plan32_;
   // ILU level schedules (host copies of the level pointers, device row lists)

@@ -52,74 +52,10 @@ __device__ __forceinline__ int xcd_chunk(int bid, int nblocks) {
 }
 
 // ----------------------------------------------------------------- BiCGSTAB scalars
-// Updates the device-resident scalars after one reduction stage; v0/v1 are the
-// two reduced sums of that stage.
-__device__ void bicg_update(BicgScalars* sc, int stage, double v0, double v1) {
-  switch (stage) {
-    case 0: {  // initial: v0 = r.r ; rho = r.r since rh = r
-      sc->r0 = sqrt(v0);
-      sc->rnorm = sc->r0;
-      sc->rho = v0;
-      sc->alpha = sc->omega = 1.0;
-      sc->beta = 0.0;
-      sc->iter = 0;
-      sc->half = 0;
-      if (!(sc->r0 > 0.0)) sc->done = isfinite(sc->r0) ? 1 : 3;
-      if (sc->r0 <= sc->abstol) sc->done = 1;
-      break;
-    }
-    case 1: {  // after v = A ph: alpha = rho / (rh.v)
-      if (v0 == 0.0 || !isfinite(v0)) {
-        sc->done = isfinite(v0) ? 4 : 3;
-        break;
-      }
-      sc->alpha = sc->rho / v0;
-      break;
-    }
-    case 2: {  // after s: half-step convergence test
-      const double ns = sqrt(v0);
-      sc->iter += 1;
-      if (!isfinite(ns)) {
-        sc->done = 3;
-        break;
-      }
-      if (ns <= sc->tol * sc->r0 || ns <= sc->abstol) {
-        sc->half = 1;
-        sc->rnorm = ns;
-      }
-      break;
-    }
-    case 3: {  // after t = A sh: omega = (t.s)/(t.t)
-      if (sc->half) break;
-      sc->omega = v1 == 0.0 ? 0.0 : v0 / v1;
-      break;
-    }
-    case 4: {  // after x, r update: convergence, beta for the next step
-      if (sc->half) {
-        sc->done = 1;
-        break;
-      }
-      const double nr = sqrt(v1);
-      sc->rnorm = nr;
-      if (!isfinite(nr)) {
-        sc->done = 3;
-        break;
-      }
-      if (nr <= sc->tol * sc->r0 || nr <= sc->abstol) {
-        sc->done = 1;
-        break;
-      }
-      if (sc->omega == 0.0 || v0 == 0.0) {
-        sc->done = 4;
-        break;
-      }
-      sc->beta = (v0 / sc->rho) * (sc->alpha / sc->omega);
-      sc->rho = v0;
-      if (sc->iter >= sc->maxit) sc->done = 2;
-      break;
-    }
-  }
-}
+#define DCG_DEV __device__ __forceinline__
+DCG_BICG_UPDATE
+DCG_KRYLOV_FINISH
+#undef DCG_DEV
 
 // out = M^-1 in at slot s: a diagonal inverse (diag: B values per slot, the
 // reference's point Jacobi) or a B x B block per slot

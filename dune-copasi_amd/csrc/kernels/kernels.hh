@@ -4,6 +4,8 @@
 
 #include <functional>
 
+#include "bicg_scalars.hh"
+
 namespace dcopasi::k {
 
 // LDS stage of the SpMV: block-row entries (blocks x B) per workgroup chunk.
@@ -26,11 +28,45 @@ struct SpmvPlan {
   int parts() const { return (variant == 0 || variant == 5) ? nchunk : row_wgs; }
 };
 
-// Device-resident BiCGSTAB state shared by its kernels.
-struct BicgScalars {
-  double rho, alpha, omega, beta, r0, rnorm, tol, abstol;
-  int iter, maxit, done, half;
+// Device-resident BiCGSTAB state shared by its kernels, and the arguments of
+// a fused operator launch (bicg_scalars.hh).
+DCG_BICG_STRUCT
+DCG_KRYLOV_OP_STRUCT
+
+// Interface facets of a fused operator, by the slots they touch: kernel kind
+// k's records at fint[k] / fdbl[k]; the entries of slot[i] are ent[ptr[i]] ..
+// ent[ptr[i + 1]] = (kind, record, row of the record's vertices: in side
+// first, then out).
+constexpr int kFacetKinds = 8;
+struct FacetRows {
+  int nslot = 0;
+  const int *slot = nullptr, *ptr = nullptr;
+  const int3* ent = nullptr;
+  const int* fint[kFacetKinds] = {};
+  const double* fdbl[kFacetKinds] = {};
 };
+
+// x += alpha M^-1 p + omega M^-1 s and r = s - omega t with s = r - alpha v,
+// after finishing the second operator's reduction (nfin partials of t.s, t.t
+// and s.s); partials (rh.r, r.r) of this launch, its workgroup count returned
+template <typename V>
+int bicg_fused_xr(int B, int nslot, V* x, const V* p, const V* v, const V* t, V* r, const V* rh, const double* dinv,
+                  int jac, const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride,
+                  double* part, int pstride, hipStream_t s);
+int bicg_fused_xr_parts(int nslot);
+// One workgroup finishes a reduction for its consumers (stage 4: rh.r and r.r,
+// 1: rh.v, 2: t.s, t.t and s.s), which then take `out` as it is (no partials,
+// in = out).  Up to kFinishParts partials each consumer workgroup sums them
+// itself, which costs no launch; above, that reading grows with the square of
+// the mesh (per iteration, FP64: 96^3, 2744 partials, 149 us without and
+// 148 us with the two launches of 4.5 and 5.9 us; 1024^2, 9,600 partials, 245
+// and 240 us)
+constexpr int kFinishParts = 2048;
+void bicg_finish(const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride, int stage,
+                 hipStream_t s);
+// the state after the x/r update's reduction, for the host to read (*in is
+// left as it is: the next iteration's first launch finishes that reduction)
+void bicg_peek(const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride, hipStream_t s);
 
 // ----------------------------------------------------------------- batches
 // A batch advances many independent models with one launch per operation:

@@ -456,6 +456,88 @@ __global__ void __launch_bounds__(kThreads) bicg_xr_k(int nslot, V* __restrict__
   }
 }
 
+// The x and r update of a fused iteration (the operator launches compute p,
+// ph, s and sh on their own boxes and store p alone): s and both
+// preconditioned directions are recomputed here.  7 vectors read, 2 written.
+template <int B, typename V>
+__global__ void __launch_bounds__(kThreads) bicg_fused_xr_k(int nslot, V* __restrict__ x, const V* __restrict__ p,
+                                                            const V* __restrict__ v, const V* __restrict__ t,
+                                                            V* __restrict__ r, const V* __restrict__ rh,
+                                                            const double* __restrict__ dinv, int jac,
+                                                            const BicgScalars* __restrict__ in,
+                                                            BicgScalars* __restrict__ out,
+                                                            const double* __restrict__ fin, int nfin, int fstride,
+                                                            double* __restrict__ part, int pstride) {
+  __shared__ double red[32];
+  BicgScalars sc;
+  if (!finish_stage<kThreads, 3>(sc, in, out, blockIdx.x == 0 && in != out, fin, nfin, fstride, 2, red)) return;
+  double acc[2] = {0.0, 0.0};
+  const bool half = sc.half != 0;
+  const double alpha = sc.alpha, omega = sc.omega;
+#pragma unroll
+  for (int u = 0; u < kXrSlots; ++u) {
+    const int s = (blockIdx.x * kXrSlots + u) * blockDim.x + threadIdx.x;
+    if (s >= nslot) continue;
+    const size_t k0 = (size_t)s * B;
+    V xv[B], pv[B], ph[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) xv[i] = x[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) ph[i] = pv[i] = p[k0 + i];
+    if (jac) dinv_apply<B>(dinv, s, pv, ph, jac == 2);
+    if (half) {
+#pragma unroll
+      for (int i = 0; i < B; ++i) x[k0 + i] = (V)((double)xv[i] + alpha * (double)ph[i]);
+      continue;
+    }
+    V rv[B], vv[B], tv[B], hv[B], sw[B], sh[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) rv[i] = r[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) vv[i] = v[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) tv[i] = t[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) hv[i] = rh[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) sh[i] = sw[i] = (V)((double)rv[i] - alpha * (double)vv[i]);
+    if (jac) dinv_apply<B>(dinv, s, sw, sh, jac == 2);
+    V xn[B], rn[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      xn[i] = (V)((double)xv[i] + alpha * (double)ph[i] + omega * (double)sh[i]);
+      rn[i] = (V)((double)sw[i] - omega * (double)tv[i]);
+      acc[0] += (double)hv[i] * (double)rn[i];
+      acc[1] += (double)rn[i] * (double)rn[i];
+    }
+#pragma unroll
+    for (int i = 0; i < B; ++i) x[k0 + i] = xn[i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) r[k0 + i] = rn[i];
+  }
+  group_sums<kThreads, 2>(acc, red);
+  if (threadIdx.x == 0) {
+    part[blockIdx.x] = acc[0];
+    part[pstride + blockIdx.x] = acc[1];
+  }
+}
+
+__global__ void __launch_bounds__(kThreads) bicg_peek_k(const BicgScalars* __restrict__ in,
+                                                        BicgScalars* __restrict__ out, const double* __restrict__ fin,
+                                                        int nfin, int fstride) {
+  __shared__ double red[32];
+  BicgScalars sc;
+  finish_stage<kThreads, 2>(sc, in, out, true, fin, nfin, fstride, 4, red);
+}
+
+template <int N>
+__global__ void __launch_bounds__(1024) bicg_finish_k(const BicgScalars* __restrict__ in, BicgScalars* __restrict__ out,
+                                                      const double* __restrict__ fin, int nfin, int fstride, int stage) {
+  __shared__ double red[16 * N];
+  BicgScalars sc;
+  finish_stage<1024, N>(sc, in, out, true, fin, nfin, fstride, stage, red);
+}
+
 // x = 0, r = rh = b, p = v = 0, partial b.b
 template <typename V, typename W>
 __global__ void __launch_bounds__(kThreads) bicg_init_k(long n, const W* __restrict__ b, V* __restrict__ x,
@@ -1377,6 +1459,34 @@ template int bicg_xr<double>(int, int, double*, const double*, const double*, co
                              const double*, const BicgScalars*, double*, hipStream_t);
 template int bicg_xr<float>(int, int, float*, const float*, const float*, const float*, const float*, float*,
                             const float*, const BicgScalars*, double*, hipStream_t);
+
+void bicg_finish(const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride, int stage,
+                 hipStream_t s) {
+  if (stage == 1) bicg_finish_k<1><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, 1);
+  else if (stage == 2) bicg_finish_k<3><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, 2);
+  else bicg_finish_k<2><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, stage);
+}
+int bicg_fused_xr_parts(int nslot) { return (nslot + kThreads * kXrSlots - 1) / (kThreads * kXrSlots); }
+template <typename V>
+int bicg_fused_xr(int B, int nslot, V* x, const V* p, const V* v, const V* t, V* r, const V* rh, const double* dinv,
+                  int jac, const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride,
+                  double* part, int pstride, hipStream_t s) {
+  const int grid = bicg_fused_xr_parts(nslot);
+  if (grid > 0)
+    DCG_DISPATCH_B(B, (bicg_fused_xr_k<BB, V><<<grid, kThreads, 0, s>>>(nslot, x, p, v, t, r, rh, dinv, jac, in, out,
+                                                                        fin, nfin, fstride, part, pstride)));
+  return grid;
+}
+template int bicg_fused_xr<double>(int, int, double*, const double*, const double*, const double*, double*,
+                                   const double*, const double*, int, const BicgScalars*, BicgScalars*, const double*,
+                                   int, int, double*, int, hipStream_t);
+template int bicg_fused_xr<float>(int, int, float*, const float*, const float*, const float*, float*, const float*,
+                                  const double*, int, const BicgScalars*, BicgScalars*, const double*, int, int,
+                                  double*, int, hipStream_t);
+
+void bicg_peek(const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride, hipStream_t s) {
+  bicg_peek_k<<<1, kThreads, 0, s>>>(in, out, fin, nfin, fstride);
+}
 
 void bicg_fin(int nparts, const double* part, int stride, int stage, BicgScalars* sc, hipStream_t s) {
   bicg_fin_k<<<1, 1024, 0, s>>>(nparts, part, stride, stage, sc);

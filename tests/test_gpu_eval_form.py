@@ -1,0 +1,110 @@
+"""Coefficients evaluated inside the apply (blocks of 1 to 4 species on box
+cells) and BiCGSTAB on fused operator launches, against the oracle: Jacobian
+apply and steps at sides around the tiles' 3, 4, 7, 15 and 31 vertices, odd
+sizes, non-square boxes, a compartment that covers a part of the grid,
+interface and boundary terms (rows with facets of several kinds), both Jacobi
+forms, FP64 and mixed; and models that keep stored coefficients because one
+compartment's expressions cost more than reading them.  Sums run in another
+order than the oracle's in FP64: 1e-12 relative for one application, the
+parity bar of 1e-8 for converged steps."""
+import numpy as np
+import pytest
+
+from tests.oracle_lib import OracleModel, rel_l2_per_species
+
+pytestmark = pytest.mark.gpu
+
+PTS = ("model.time_step_operator.linear_solver.storage = points\n"
+       "model.time_step_operator.linear_solver.preconditioner.type = {}\n"
+       "model.time_step_operator.linear_solver.precision = {}\n")
+
+# far more operations than coefficients: such a compartment stores them
+COSTLY = "1e-30*(" + "+".join(f"sin({k}*position_x)*cos({k}+time)" for k in range(1, 24)) + ")"
+
+
+def _ini(dim, cells, species, inner=0, costly=False, extensions=(1.0, 0.6, 1.7)):
+    """`species` species outside a ball, `inner` species inside it with a flux between the first ones (0: no ball)."""
+    r2 = " + ".join(f"(position_{a}-0.4)^2" for a in "xyz"[:dim])
+    comps = "domain.expression = 1" if not inner else f"domain.expression = {r2} >= 0.08\ncore.expression = {r2} < 0.08"
+    out = [f"[grid]\ndimension = {dim}\ncells = {' '.join(map(str, cells))}\n"
+           f"extensions = {' '.join(map(str, extensions[:dim]))}\ncell_type = cube", f"[compartments]\n{comps}"]
+    for comp, tag, n in (("domain", "s", species), ("core", "c", inner)):
+        for i in range(n):
+            a, b = f"{tag}{i}", f"{tag}{(i + 1) % n}"
+            extra = f" + {COSTLY}" if costly and comp == "domain" and i == 0 else ""
+            out += [f"[model.scalar_field.{a}]", f"compartment = {comp}", f"storage.expression = {1.0 + 0.1 * i}",
+                    f"initial.expression = 0.5 + 0.1*sin({i + 1}*position_x + 2*position_y)",
+                    f"cross_diffusion.{a}.expression = {0.001 * (i + 1)}"]
+            if n > 1:
+                out += [f"reaction.expression = 0.7*{b}*{b} - {a}*{b} + 0.1*position_x*{a} + 0.05*time*{b}",
+                        f"reaction.jacobian.{a}.expression = -{b} + 0.1*position_x{extra}",
+                        f"reaction.jacobian.{b}.expression = 1.4*{b} - {a} + 0.05*time"]
+            else:
+                out += [f"reaction.expression = 0.7*{a}*{a} - 0.05*time*{a}",
+                        f"reaction.jacobian.{a}.expression = 1.4*{a} - 0.05*time{extra}"]
+            if i == 0 and inner:
+                other, sign = ("core", "") if comp == "domain" else ("domain", "-")
+                out += [f"outflow.{other}.expression = {sign}0.3*(s0 - c0*c0)",
+                        f"outflow.{other}.jacobian.s0.expression = {sign}0.3",
+                        f"outflow.{other}.jacobian.c0.expression = {sign}(-0.6*c0)"]
+                if comp == "domain":  # the domain's boundary
+                    out += ["outflow.domain.expression = 0.2*s0*s0", "outflow.domain.jacobian.s0.expression = 0.4*s0"]
+    return "\n".join(out) + ("\n[model.time_step_operator]\ntype = Alexander2\nlinear_solver.type = BiCGSTAB\n"
+                             "linear_solver.convergence_condition.relative_tolerance = 1e-12\n"
+                             "linear_solver.convergence_condition.iteration_range = 1 2000\n"
+                             "linear_solver.preconditioner.type = Jacobi\n"
+                             "nonlinear_solver.convergence_condition.relative_tolerance = 1e-20\n"
+                             "nonlinear_solver.convergence_condition.absolute_tolerance = 1e-28\n"
+                             "nonlinear_solver.convergence_condition.iteration_range = 0 40\n")
+
+
+SHAPES = [(2, (1, 1)), (2, (7, 4)), (2, (15, 14)), (2, (30, 16)), (2, (47, 33)), (3, (1, 1, 1)), (3, (3, 4, 7)),
+          (3, (7, 8, 6)), (3, (8, 3, 15)), (3, (16, 5, 9))]
+
+
+@pytest.mark.parametrize("species", [1, 2, 3, 4])
+@pytest.mark.parametrize("dim,cells", SHAPES)
+def test_apply(dca, dim, cells, species):
+    print(f"case: evaluated form {dim}D {cells} {species} species", flush=True)
+    ini = _ini(dim, cells, species)
+    orc = OracleModel(ini)
+    rng = np.random.default_rng(species)
+    x = v = None
+    for tile in range(8):
+        over = f"model.time_step_operator.linear_solver.point_tile = {tile}\n"
+        gpu = dca.Model(ini, PTS.format("Jacobi", "fp64") + over, 0)
+        assert "dcg_tile_0_e0" in gpu.generated_source()
+        if x is None:
+            x, v = 0.5 + 0.2 * rng.random(gpu.n_dof), rng.standard_normal(gpu.n_dof)
+        for cm, ca in ((1.0, 0.0), (1.0, 0.3)):
+            _, vals = orc.assemble(x, 0.4, cm, ca)
+            ref = orc.csr(vals) @ v
+            y = gpu.jacobian_apply(x, 0.4, cm, ca, v)
+            assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max(), tile
+        gpu.close()
+    orc.close()
+
+
+@pytest.mark.parametrize("costly", [False, True])
+@pytest.mark.parametrize("precond", ["Jacobi", "VertexBlockJacobi"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("dim,cells,species,inner", [(2, (33, 20), 3, 2), (2, (17, 31), 1, 4), (3, (9, 8, 6), 2, 1),
+                                                     (3, (8, 7, 11), 4, 6)])
+def test_steps(dca, dim, cells, species, inner, precision, precond, costly):
+    print(f"case: evaluated form steps {dim}D {species}+{inner} {precision} {precond} costly={costly}", flush=True)
+    ini = _ini(dim, cells, species, inner, costly)
+    gpu = dca.Model(ini, PTS.format(precond, precision), 0)
+    assert ("dcg_tile_0_e0" in gpu.generated_source()) != costly
+    orc = OracleModel(ini)
+    u0 = gpu.initial_state()
+    gpu.set_state(u0, 0.0)
+    orc.set_state(u0, 0.0)
+    t = 0.0
+    for _ in range(2):
+        st = gpu.step(t, 0.1)
+        rc, newton, _ = orc.step(0.1)
+        assert st.status == 0 and rc == 0 and st.newton_iterations == newton
+        t += 0.1
+    assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], orc.get_state()[0])) < 1e-8
+    gpu.close()
+    orc.close()
