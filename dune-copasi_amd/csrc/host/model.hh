@@ -284,6 +284,9 @@ class Model {
  private:
   double assembly_bytes(bool jacobian) const;
   std::vector<ReduceKey> reduce_keys(const std::string& reduce_ini) const;
+  struct ReducePlan;
+  ReducePlan& reduce_plan(const std::string& reduce_ini);
+  std::vector<std::shared_ptr<ReducePlan>> reduce_plans_;  // the last few texts, the latest first
   double apply_bytes() const;
 
  public:

