@@ -2630,16 +2630,322 @@ __device__ __forceinline__ void eval_krylov(int tile, int at, dcg_gp<const int> 
   if (mode) put_partials<NT>(op, at, e0, e1, e2, red);
 }
 )";
+// 3D: a lane per vertex of a layer, walking along z (one workgroup: TX x TY
+// row vertices of a layer, TZ layers).  In the cell-box form above every cell
+// of a box reads its 8 corners and each box stages its own halo (8^3 cells and
+// 9^3 vertices for 7^3 rows); here a plane's vertices are loaded once per
+// chunk of layers while the layer before is computed, a plane's sums and
+// differences over x (lane exchange) and y (LDS) serve the cells below and
+// above it, and the upper half of a cell's terms stays in registers.  Layers
+// are 16 lanes wide, the width of a lane exchange row.  One barrier per layer:
+// a plane's sums are complete one layer later and stored after the next
+// barrier.
+// FP64 with the p-update, 2 species: 96^3 59 -> 42 us, 70^3 32 -> 29 us; at
+// 47^3 14.5 us against 20.7 us, too few columns: the shapes are timed at set-up
+// and the faster one is taken.  About 350 FP64 instructions per layer and
+// wave, two waves per SIMD (218 registers; bounded for three it spills: 102
+// us); bound by their issue and by what two waves leave of the latency.
+const char* kEvalMarch = R"(
+template <int A>
+__device__ __forceinline__ double lane_next(double v) {  // A 0: of lane + 1, 1: of lane - 1 (of 16)
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), A == 0 ? 0x101 : 0x111, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), A == 0 ? 0x101 : 0x111, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+template <int A>
+__device__ __forceinline__ float lane_next(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), A == 0 ? 0x101 : 0x111, 0xF, 0xF, true));
+}
+// the z points' weights 0.5 + G2 and 0.5 - G2 as 1 and Z10 times the former,
+// which goes with the weights of the modes of x and y
+constexpr double Z1 = 0.5 + G2, Z0 = 0.5 - G2, Z10 = Z0 / Z1;
+__device__ constexpr double plane_weight(int a) { return Z1 * ((a & 1) ? G2 : 0.5) * ((a & 2) ? G2 : 0.5); }
+template <typename T>
+__device__ __forceinline__ void plane_modes(T (&v)[4][BC]) {
+#pragma unroll
+  for (int i = 0; i < BC; ++i) {
+    const T a = v[0][i] + v[1][i], b = v[0][i] - v[1][i], c = v[2][i] + v[3][i], d = v[2][i] - v[3][i];
+    v[0][i] = a + c;
+    v[1][i] = b + d;
+    v[2][i] = a - c;
+    v[3][i] = b - d;
+  }
+}
+template <typename TL, typename T>
+__device__ __forceinline__ void eval_march(int tile, int at, dcg_gp<const int> __restrict__ g2l,
+                                           dcg_gp<const unsigned char> __restrict__ cmask, dcg_gp<const double> lin,
+                                           const KrylovOp& op, bool lead, dcg_gp<const double> __restrict__ tca,
+                                           int n0, int n1, int n2, const double* __restrict__ prm) {
+  constexpr int TX = TL::TX, TY = TL::TY, TZ = TL::TZ, YB = TY + 2, NT = 16 * YB;
+  static_assert(DIM == 3 && TX == 14 && NT == TL::NT && NT % 64 == 0, "a layer of 16 lanes per row");
+  __shared__ double sx[2][2 * BC][NT];
+  __shared__ T sv[2][2 * BC][NT], sy[2][BC][NT];
+  __shared__ double red[3 * (NT / 64)];
+  const auto A = (dcg_gp<const T>)(const T*)op.a;
+  const auto P = (dcg_gp<const T>)(const T*)op.b;
+  const auto C = (dcg_gp<const T>)(const T*)op.c;
+  const auto W = (dcg_gp<const T>)(const T*)op.w;
+  const auto D = (dcg_gp<T>)(T*)op.d;
+  const auto Y = (dcg_gp<T>)(T*)op.y;
+  const auto DI = (dcg_gp<const double>)op.dinv;
+  const int mode = op.mode, tid = threadIdx.x, bi = tid & 15, bj = tid >> 4;
+  const int ntx = (n0 + 1 + TX - 1) / TX, nty = (n1 + 1 + TY - 1) / TY;
+  const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);
+  const int gi = tx * TX - 1 + bi, gj = ty * TY - 1 + bj;
+  const int z0 = tz * TZ, z1 = z0 + TZ - 1 < n2 ? z0 + TZ - 1 : n2;  // row planes
+  const int p0 = z0 > 0 ? z0 - 1 : 0, p1 = z1 < n2 ? z1 + 1 : n2;     // planes of their cells
+  const bool vin = gi >= 0 && gi <= n0 && gj >= 0 && gj <= n1;
+  const bool row = vin && bi >= 1 && bi <= TX && bj >= 1 && bj <= TY;
+  const bool col = bi < 15 && bj < YB - 1 && gi >= 0 && gi < n0 && gj >= 0 && gj < n1;
+  const int up = bj < YB - 1 ? tid + 16 : tid, down = bj > 0 ? tid - 16 : tid;
+  T la[BC], lp[BC], lc[BC];
+  double lx[BC];
+  int ls = -1;
+  auto slot_of = [&](int k) -> int {
+    if (!vin || k > n2) return -1;
+    const int vid = gi + (n0 + 1) * (gj + (n1 + 1) * k);
+    return g2l ? g2l[vid] : vid;
+  };
+  auto load = [&](int s) {
+    ls = s;
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      la[i] = lp[i] = lc[i] = T(0);
+      lx[i] = 0.0;
+    }
+    if (s < 0) return;
+#pragma unroll
+    for (int i = 0; i < BC; ++i) la[i] = A[(size_t)s * DCG_B + i];
+    if (mode)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) lc[i] = C[(size_t)s * DCG_B + i];
+    if (mode == 1)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) lp[i] = P[(size_t)s * DCG_B + i];
+#pragma unroll
+    for (int i = 0; i < BC; ++i) lx[i] = lin[(size_t)s * DCG_B + i];
+  };
+  load(slot_of(p0));
+  int nexts = slot_of(p0 + 1);
+  BicgScalars sc;
+  sc.alpha = sc.beta = sc.omega = 0.0;
+  if (mode == 1) {
+    if (!finish_stage<NT, 2>(sc, op.in, op.out, lead, op.fin, op.nfin, op.fstride, 4, red)) return;
+  } else if (mode == 2) {
+    if (!finish_stage<NT, 1>(sc, op.in, op.out, lead, op.fin, op.nfin, op.fstride, 1, red)) return;
+  }
+  const double alpha = sc.alpha, beta = sc.beta, omega = sc.omega;
+  const double t = tca[0], ca = tca[1], cm = tca[2], ox = tca[3], oy = tca[4], oz = tca[5], hx = tca[6], hy = tca[7],
+               hz = tca[8];
+  double dp[NEP > 0 ? NEP : 1];
+  pair_diffusion(t, prm, dp);
+  // of the plane below: the values over it at the layer's points (x and y),
+  // the direction's modes, and what the layer below adds to its sums (at the
+  // points, and in modes)
+  double xg[4][BC], e0 = 0.0, e1 = 0.0, e2 = 0.0;
+  T vg[4][BC], vm[4][BC], cg[4][BC], cs[4][BC], own[BC];
+  T q1[BC], q2[BC];                                 // the direction before M^-1, one and two planes back
+  int s1 = -1, s2 = -1;
+#pragma unroll
+  for (int i = 0; i < BC; ++i) {
+    own[i] = q1[i] = q2[i] = T(0);
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      xg[a][i] = 0.0;
+      vg[a][i] = vm[a][i] = cg[a][i] = cs[a][i] = T(0);
+    }
+  }
+  for (int k = p0; k <= z1 + 2; ++k) {
+    const int buf = k & 1;
+    const bool plane = k <= p1;
+    const int s = ls;
+    T q0[BC], o[BC];
+    double x0[BC];
+    bool has = false;
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      q0[i] = o[i] = T(0);
+      x0[i] = 0.0;
+    }
+    if (plane) {
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        q0[i] = mode == 1   ? (T)((double)la[i] + beta * ((double)lp[i] - omega * (double)lc[i]))
+                : mode == 2 ? (T)((double)la[i] - alpha * (double)lc[i])
+                            : la[i];
+        o[i] = q0[i];
+        x0[i] = lx[i];
+      }
+      if (s >= 0 && mode) precondition(op.jac, op.dinv, s, q0, o);
+      if (mode == 1 && row && s >= 0 && k >= z0 && k <= z1)
+#pragma unroll
+        for (int i = 0; i < DCG_B; ++i) D[(size_t)s * DCG_B + i] = i < BC ? q0[i < BC ? i : 0] : T(0);
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        const double xn = lane_next<0>(x0[i]);
+        const T vn = lane_next<0>(o[i]);
+        sx[buf][2 * i][tid] = x0[i] + xn;
+        sx[buf][2 * i + 1][tid] = x0[i] - xn;
+        sv[buf][2 * i][tid] = o[i] + vn;
+        sv[buf][2 * i + 1][tid] = o[i] - vn;
+      }
+      if (k > p0 && col) has = cmask[gi + n0 * (gj + n1 * (k - 1))] != 0;
+      if (k < p1) {
+        load(nexts);
+        nexts = slot_of(k + 2);
+      } else {
+        ls = -1;
+      }
+    }
+    const bool store = row && s2 >= 0 && k - 2 >= z0;
+    T w2[BC];
+#pragma unroll
+    for (int i = 0; i < BC; ++i) w2[i] = store && mode == 1 ? W[(size_t)s2 * DCG_B + i] : T(0);
+    __syncthreads();
+    T y2[BC];
+#pragma unroll
+    for (int i = 0; i < BC; ++i) y2[i] = own[i] + sy[buf ^ 1][i][down];
+    double xc[4][BC];
+    T vc[4][BC], vp[4][BC];
+    if (plane) {
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        const double xa = sx[buf][2 * i][tid], xb = sx[buf][2 * i + 1][tid], xu = sx[buf][2 * i][up],
+                     xw = sx[buf][2 * i + 1][up];
+        xc[0][i] = (xa + xu) * plane_weight(0);
+        xc[1][i] = (xb + xw) * plane_weight(1);
+        xc[2][i] = (xa - xu) * plane_weight(2);
+        xc[3][i] = (xb - xw) * plane_weight(3);
+        const T va = sv[buf][2 * i][tid], vb = sv[buf][2 * i + 1][tid], vu = sv[buf][2 * i][up],
+                vw = sv[buf][2 * i + 1][up];
+        vc[0][i] = va + vu;
+        vc[1][i] = vb + vw;
+        vc[2][i] = va - vu;
+        vc[3][i] = vb - vw;
+      }
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) vp[a][i] = vc[a][i] * T(plane_weight(a));
+      plane_modes(xc);
+      plane_modes(vp);
+    }
+    // the sums of plane k - 1: at the points from both layers, then modes
+    T lo[4][BC], ls4[4][BC];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        lo[a][i] = cg[a][i];
+        ls4[a][i] = cs[a][i];
+        cg[a][i] = cs[a][i] = T(0);
+      }
+    if (has) {
+      const double pza = oz + (k - 1 + Z0) * hz, pzb = oz + (k - 1 + Z1) * hz;
+#pragma unroll
+      for (int a = 0; a < 4; ++a) {
+        const double px = ox + (gi + ((a & 1) ? Z1 : Z0)) * hx, py = oy + (gj + ((a & 2) ? Z1 : Z0)) * hy;
+        double mc[NMC > 0 ? NMC : 1], u[BC];
+        T q[BC], wa[BC], wb[BC];
+#pragma unroll
+        for (int i = 0; i < BC; ++i) {
+          u[i] = xg[a][i] + Z10 * xc[a][i];
+          q[i] = vg[a][i] + T(Z10) * vp[a][i];
+        }
+        point_jacobian(u, px, py, pza, t, cm, ca, mc, prm);
+        point_block(mc, q, wa);
+#pragma unroll
+        for (int i = 0; i < BC; ++i) {
+          u[i] = Z10 * xg[a][i] + xc[a][i];
+          q[i] = T(Z10) * vg[a][i] + vp[a][i];
+        }
+        point_jacobian(u, px, py, pzb, t, cm, ca, mc, prm);
+        point_block(mc, q, wb);
+#pragma unroll
+        for (int i = 0; i < BC; ++i) {
+          lo[a][i] += wa[i] + T(Z10) * wb[i];
+          cg[a][i] = T(Z10) * wa[i] + wb[i];
+        }
+      }
+#pragma unroll
+      for (int n = 0; n < NEP; ++n) {
+        const double cd = ca * dp[n];
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+          double ks = 0.0, kd = 0.0;
+#pragma unroll
+          for (int d = 0; d < DIM; ++d)
+            if (EPK[n] == 3 || EPK[n] == d) {
+              ks += mode_kap(a, d);
+              kd += mode_kap(a + 4, d);
+            }
+          const T zs = T(cd) * (T(ks) * (vm[a][EPJ[n]] + vc[a][EPJ[n]]));
+          const T zd = T(cd) * (T(kd) * (vm[a][EPJ[n]] - vc[a][EPJ[n]]));
+          ls4[a][EPI[n]] += zs + zd;
+          cs[a][EPI[n]] += zs - zd;
+        }
+      }
+    }
+    plane_modes(lo);
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int i = 0; i < BC; ++i) lo[a][i] = T(plane_weight(a)) * lo[a][i] + ls4[a][i];
+    plane_modes(lo);
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      own[i] = lo[0][i] + lane_next<1>(lo[1][i]);
+      sy[buf][i][tid] = lo[2][i] + lane_next<1>(lo[3][i]);
+    }
+    if (plane)
+#pragma unroll
+      for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int i = 0; i < BC; ++i) {
+          xg[a][i] = xc[a][i];
+          vg[a][i] = vp[a][i];
+          vm[a][i] = vc[a][i];
+        }
+    // plane k - 2 is complete
+    if (store) {
+#pragma unroll
+      for (int i = 0; i < DCG_B; ++i) {
+        const T y = i < BC ? y2[i < BC ? i : 0] : mode ? T(0) : A[(size_t)s2 * DCG_B + i];
+        Y[(size_t)s2 * DCG_B + i] = y;
+      }
+#pragma unroll
+      for (int i = 0; i < BC; ++i) {
+        const double y = (double)y2[i];
+        if (mode == 1) {
+          e0 += y * (double)w2[i];
+        } else {
+          e0 += y * (double)q2[i];
+          e1 += y * y;
+          e2 += (double)q2[i] * (double)q2[i];
+        }
+      }
+    }
+    s2 = s1;
+    s1 = plane ? s : -1;
+#pragma unroll
+    for (int i = 0; i < BC; ++i) {
+      q2[i] = q1[i];
+      q1[i] = q0[i];
+    }
+  }
+  if (mode) put_partials<NT>(op, at, e0, e1, e2, red);
+}
+)";
 const char* kEvalKrylovEntries = R"(
 }  // namespace %C%
-#define DCG_EVAL_ENTRY(NAME, T, TL)                                                                               \
+#define DCG_EVAL_ENTRY(NAME, T, TL, FN)                                                                           \
   extern "C" __global__ void __launch_bounds__(TL::NT, TL::MINW)                                                  \
   NAME(const int* __restrict__ tiles, int ntile, const int* __restrict__ g2l,                                     \
        const unsigned char* __restrict__ cmask, const double* lin, KrylovOp op, const double* __restrict__ tca,    \
        int n0, int n1, int n2, const double* __restrict__ prm) {                                                  \
     const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
     if (c >= ntile) return;                                                                                       \
-    %C%::%EVAL_FN%<TL, T>(tiles[c], c, (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,      \
+    %C%::FN<TL, T>(tiles[c], c, (%C%::dcg_gp<const int>)g2l, (%C%::dcg_gp<const unsigned char>)cmask,      \
                           (%C%::dcg_gp<const double>)lin, op, op.lead && blockIdx.x == 0,                         \
                           (%C%::dcg_gp<const double>)tca, n0, n1, n2, prm);                                       \
   }
@@ -3221,9 +3527,16 @@ dcg_facet_rows_f(FacetRows F, const double* lin, KrylovOp op, const double* tca,
 }
 )";
 
+// boxes of more cells than a workgroup's threads are walked layer by layer
+// (eval_march)
+static bool march_tile(int dim, std::array<int, 3> t) {
+  return dim == 3 && (t[0] + 1) * (t[1] + 1) * (t[2] + 1) > 1024;
+}
+
 int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner) {
   // corner form: a lane per corner of a layer's cells
   if (corner) return (t[0] + 1) * (dim > 2 ? t[1] + 1 : 1) << dim;
+  if (march_tile(dim, t)) return 16 * (t[1] + 2);  // a lane per vertex of a layer
   // one cell of the cell box per thread (corner sums scattered in LDS) for
   // blocks of up to 4 species; larger blocks loop over the cells
   int ncb = t[0] + 1;
@@ -3298,7 +3611,7 @@ bool eval_eligible(const ModelSpec& m, const Grid& g, int comp) {
 }
 
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
-                                                      bool eval, std::vector<int>* waves) {
+                                                      bool eval, bool geo, std::vector<int>* waves) {
   std::vector<std::array<int, 3>> out{setup_tile};
   if (waves) waves->assign(1, 1);
   if (species > 4) return out;  // corner values in LDS: the assembly tile only
@@ -3324,6 +3637,13 @@ std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species
   } else if (eval && g.dim == 3) {
     cand = {{8, 4, 4}, {7, 7, 3}, {15, 3, 3}, {7, 7, 7}, {15, 7, 7}, {7, 7, 7}};
     wv = {1, 1, 1, 1, 1, 5};
+    // larger meshes walk layers (not in batches, whose members' geometry is a
+    // run time value); short walks fill the chip, long ones load fewer halo
+    // planes
+    if (!geo) {
+      cand = {{8, 4, 4}, {7, 7, 3}, {7, 7, 7}, {14, 14, 6}, {14, 14, 10}, {14, 14, 20}};
+      wv = {1, 1, 1, 1, 1, 1};
+    }
   }
   for (size_t i = 0; i < cand.size(); ++i)
     if (cand[i] != setup_tile || wv[i] != 1) {
@@ -3579,7 +3899,6 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     replace_all(body, "%CORNER_OP_ROW%", points ? kCornerOpRow : "");
     replace_all(body, "%CORNER_OP_END%", points ? kCornerOpEnd : "");
     if (points) body += std::string(kCornerPoints) + "namespace %C% {\n" + kCornerKrylov + kEvalKrylovEntries;
-    replace_all(body, "%EVAL_FN%", "corner_krylov");
     if (geo && comp < 4) body += kCornerBatch;
     if (geo && comp < 4 && points) body += kCornerPointBatch;
     const auto shapes = corner_tiles(d);
@@ -3588,8 +3907,8 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
       const std::string id = std::to_string(k2), tl = ns + "::CornerShape" + id;
       cs += "using CornerShape" + id + " = CornerTile<" + std::to_string(shapes[k2][0]) + ", " +
             std::to_string(shapes[k2][1]) + ", " + std::to_string(shapes[k2][2]) + ">;\n";
-      ce += "DCG_EVAL_ENTRY(%KERNEL%_e" + id + ", double, " + tl + ")\n";
-      ce += "DCG_EVAL_ENTRY(%KERNEL%_ef" + id + ", float, " + tl + ")\n";
+      ce += "DCG_EVAL_ENTRY(%KERNEL%_e" + id + ", double, " + tl + ", corner_krylov)\n";
+      ce += "DCG_EVAL_ENTRY(%KERNEL%_ef" + id + ", float, " + tl + ", corner_krylov)\n";
       cb += "DCG_CORNER_BENTRY(%KERNEL%_ebatch" + id + ", double, v, " + tl + ")\n";
       cb += "DCG_CORNER_BENTRY(%KERNEL%_efbatch" + id + ", float, f, " + tl + ")\n";
     }
@@ -3603,13 +3922,17 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     // one point apply (and batched point apply) per candidate tile shape k:
     // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k> (_e.. where evaluated)
     std::string pe, pb;
+    bool any_march = false;
     const std::string en = eval ? "e" : "p";
     for (size_t k2 = 0; k2 < apply_tiles.size(); ++k2) {
       const std::string id = std::to_string(k2);
       const std::string tl = ns + "::ApplyShape" + id;
       const std::string entry = eval ? "DCG_EVAL_ENTRY" : "DCG_POINT_ENTRY";
-      pe += entry + "(%KERNEL%_" + en + id + ", double, " + tl + ")\n";
-      pe += entry + "(%KERNEL%_" + en + "f" + id + ", float, " + tl + ")\n";
+      const bool march = eval && march_tile(g.dim, apply_tiles[k2]);
+      const std::string fn = !eval ? "" : march ? ", eval_march" : ", eval_krylov";
+      pe += entry + "(%KERNEL%_" + en + id + ", double, " + tl + fn + ")\n";
+      pe += entry + "(%KERNEL%_" + en + "f" + id + ", float, " + tl + fn + ")\n";
+      any_march = any_march || march;
       pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "batch" + id + ", double, v, pc, " + tl + ")\n";
       pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "fbatch" + id + ", float, f, " + (eval ? "pc, " : "pc32, ") + tl + ")\n";
     }
@@ -3622,8 +3945,7 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
                                               false)) +
             ", " + std::to_string(k2 < apply_waves.size() ? apply_waves[k2] : 1) + ">;\n";
     replace_all(body, "%APPLY_SHAPES%", as);
-    if (eval) body += std::string(kEvalKrylov) + kEvalKrylovCells + kEvalKrylovEntries;
-    replace_all(body, "%EVAL_FN%", "eval_krylov");
+    if (eval) body += std::string(kEvalKrylov) + kEvalKrylovCells + (any_march ? kEvalMarch : "") + kEvalKrylovEntries;
     replace_all(body, "%POINT_ENTRIES%", eval ? "" : pe);
     replace_all(body, "%EVAL_ENTRIES%", eval ? pe : "");
     replace_all(body, "%PBATCH_ENTRIES%", pb);
@@ -3686,7 +4008,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
         shapes = corner_tiles(L.grid.dim);
         waves.assign(shapes.size(), 1);
       } else if (points) {
-        shapes = apply_tile_candidates(L.grid, nsp, tile, eval, &waves);
+        shapes = apply_tile_candidates(L.grid, nsp, tile, eval, geo, &waves);
       }
       for (const auto& t : shapes) threads.push_back(apply_tile_threads(L.grid.dim, t, nsp, corner));
       src << gen_tiled(spec, L.grid, static_cast<int>(c), ns, tk, tile, geo, points, corner, eval && !corner, shapes, waves);

@@ -67,7 +67,7 @@ constexpr int kGeoWords = 8;
 bool tile_eligible(const ModelSpec& m, int comp);
 // tile shapes the point apply is generated for (the set-up tile first)
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
-                                                      bool eval, std::vector<int>* waves = nullptr);
+                                                      bool eval, bool geo, std::vector<int>* waves = nullptr);
 // workgroup size of the point apply with tile t (row vertices along x, y, z)
 int apply_tile_threads(int dim, std::array<int, 3> t, int species, bool corner);
 // the compartment's point applies evaluate their coefficients (blocks of up

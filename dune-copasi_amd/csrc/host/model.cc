@@ -735,6 +735,27 @@ void Model::tune_points() {
       fb = DeviceArray<char>();
     }
   }
+  // evaluated applies: the launch with the p-update of a solve under way
+  // (the scalars are zero: not done)
+  const k::BicgScalars going{};
+  DCG_HIP(hipMemcpyAsync(sc_.get(), &going, sizeof going, hipMemcpyHostToDevice, stream_));
+  k::KrylovOp op{};
+  op.mode = 1;
+  // in the precision of the solver's iteration
+  const bool op32 = fused() && cfg_.precision == Precision::Mixed;
+  void* vec[5];
+  for (int i = 0; i < 5; ++i) {
+    vec[i] = op32 ? static_cast<void*>(kf_[i].get()) : static_cast<void*>(kv_[i].get());
+    if (fused()) DCG_HIP(hipMemsetAsync(vec[i], 0, (op32 ? sizeof(float) : sizeof(double)) * L_.nslot * L_.B, stream_));
+  }
+  op.a = op.w = vec[0];
+  op.b = vec[1];
+  op.c = vec[2];
+  op.d = vec[3];
+  op.y = vec[4];
+  op.in = sc_.get();
+  op.out = sc_.get() + 1;
+  op.part = kpart_.get();
   hipEvent_t e0, e1;
   DCG_HIP(hipEventCreate(&e0));
   DCG_HIP(hipEventCreate(&e1));
@@ -748,7 +769,7 @@ void Model::tune_points() {
         apply_shape_[c] = static_cast<int>(k2);
         if (fa.size()) k::probe_copy(fa.get(), fb.get(), kFlushBytes, stream_);
         DCG_HIP(hipEventRecord(e0, stream_));
-        if (fused()) launch_points_apply(kv_[0].get(), kv_[1].get(), nullptr, false);
+        if (fused()) launch_krylov_op(op, op32);
         else launch_points_apply(kv_[0].get(), kv_[1].get(), nullptr, false, kv_[2].get(), kv_[3].get(), part_.get());
         DCG_HIP(hipEventRecord(e1, stream_));
         DCG_HIP(hipEventSynchronize(e1));

@@ -59,7 +59,7 @@ def _ini(dim, cells, species, inner=0, costly=False, extensions=(1.0, 0.6, 1.7))
 
 
 SHAPES = [(2, (1, 1)), (2, (7, 4)), (2, (15, 14)), (2, (30, 16)), (2, (47, 33)), (3, (1, 1, 1)), (3, (3, 4, 7)),
-          (3, (7, 8, 6)), (3, (8, 3, 15)), (3, (16, 5, 9))]
+          (3, (7, 8, 6)), (3, (8, 3, 15)), (3, (16, 5, 9)), (3, (13, 6, 18)), (3, (28, 14, 34))]
 
 
 @pytest.mark.parametrize("species", [1, 2, 3, 4])
