@@ -1,6 +1,7 @@
 #include "batch.hh"
 
 #include <algorithm>
+#include <tuple>
 #include <cstddef>
 #include <cstdlib>
 #include <cmath>
@@ -177,17 +178,19 @@ void Batch::rebuild() {
   sgroups_.clear();
   agroups_.clear();
   // solver groups by block size and Jacobian storage
-  std::map<std::pair<int, bool>, int> by_b;
+  std::map<std::tuple<int, bool, bool>, int> by_b;
   for (size_t i = 0; i < members_.size(); ++i) {
     Entry& e = members_[i];
     const int B = e.m->layout().B;
     const bool pts = e.m->point_storage();
-    auto it = by_b.find({B, pts});
+    const bool fused = pts && e.m->gen_.fused;
+    auto it = by_b.find({B, pts, fused});
     if (it == by_b.end()) {
-      it = by_b.emplace(std::make_pair(B, pts), static_cast<int>(sgroups_.size())).first;
+      it = by_b.emplace(std::make_tuple(B, pts, fused), static_cast<int>(sgroups_.size())).first;
       sgroups_.emplace_back();
       sgroups_.back().B = B;
       sgroups_.back().points = pts;
+      sgroups_.back().fused = fused;
     }
     e.sg = it->second;
     e.si = static_cast<int>(sgroups_[e.sg].mem.size());
@@ -268,6 +271,7 @@ void Batch::rebuild() {
         pm.pc32 = c0 < m.pc32_.size() ? m.pc32_[c0].get() : nullptr;
         pm.tca = m.pc_tca_.get();
         pm.prm = m.prm_.get();
+        pm.dinv = mv[j].dinv;
         const Grid& gr = m.L_.grid;
         pm.n[0] = static_cast<int>(gr.n[0]);
         pm.n[1] = gr.dim > 1 ? static_cast<int>(gr.n[1]) : 1;
@@ -289,8 +293,11 @@ void Batch::rebuild() {
           for (size_t k2 = 0; k2 < nk; ++k2) {
             const std::string id = std::to_string(k2);
             pl.f64s.push_back(m.module_->function(name + "batch" + id));
-            pl.f32s.push_back(opt_.precision == Precision::Mixed ? m.module_->function(name + "fbatch" + id)
-                                                                 : nullptr);
+            const bool mixed = opt_.precision == Precision::Mixed;
+            pl.f32s.push_back(mixed && !g.fused ? m.module_->function(name + "fbatch" + id) : nullptr);
+            const std::string kname = m.gen_.tile_kernel[c0];
+            pl.k64s.push_back(g.fused && !mixed ? m.module_->function(kname + "_kbatch" + id) : nullptr);
+            pl.k32s.push_back(g.fused && mixed ? m.module_->function(kname + "_kfbatch" + id) : nullptr);
             pl.tiles.push_back(m.gen_.apply_tiles[c0][k2]);
             pl.nts.push_back(m.gen_.apply_threads[c0][k2]);
           }
@@ -342,6 +349,31 @@ void Batch::rebuild() {
           for (size_t k2 = 0; k2 < nk; ++k2) dw[k2].upload(items[l][k2], stream_);
           std::vector<double> ms(nk, 0.0);
           const k::PcMember* mem = g.pcm.get();
+          // (fused groups: the launch and precision of their iterations)
+          DeviceArray<k::BicgScalars> tsc;
+          DeviceArray<double> tpart;
+          DeviceArray<int2> trange;
+          k::BatchOp op{};
+          if (g.fused) {
+            size_t most = 0;
+            for (const auto& it2 : items[l]) most = std::max(most, it2.size());
+            tpart.resize(3 * most + 8);
+            tsc.upload(std::vector<k::BicgScalars>(2 * static_cast<size_t>(M)), stream_);
+            trange.upload(std::vector<int2>(M, make_int2(-1, -1)), stream_);
+            const int base = opt_.precision == Precision::Mixed ? 0 : k::kVKry;
+            op.mode = 1;
+            op.jac = jacobi_kind();
+            op.a = base;
+            op.b = base + 2;
+            op.c = base + 3;
+            op.d = base + 4;
+            op.y = base + 6;
+            op.w = base + 1;
+            op.in = tsc.get();
+            op.out = tsc.get() + M;
+            op.range = trange.get();
+            op.part = tpart.get();
+          }
           for (int round = 0; round < 4; ++round)
             for (size_t k2 = 0; k2 < nk; ++k2) {
               const int2* work = dw[k2].get();
@@ -349,12 +381,16 @@ void Batch::rebuild() {
                   a2 = -1, sk = -1;
               double* part = nullptr;
               void* args[] = {&work, &nwork, &o0, &mem, &xs, &ys, &a1, &a2, &sk, &part};
+              void* fargs[] = {&work, &nwork, &mem, &op};
               const unsigned grid = static_cast<unsigned>((nwork + 7) / 8 * 8);
               if (nwork <= 0) continue;
               DCG_HIP(hipEventRecord(e0, stream_));
               for (int rep = 0; rep < 2; ++rep)
-                DCG_HIP(hipModuleLaunchKernel(pl.f64s[k2], grid, 1, 1, static_cast<unsigned>(pl.nts[k2]), 1, 1, 0,
-                                              stream_, args, nullptr));
+                DCG_HIP(hipModuleLaunchKernel(!g.fused                               ? pl.f64s[k2]
+                                              : opt_.precision == Precision::Mixed ? pl.k32s[k2]
+                                                                                   : pl.k64s[k2],
+                                              grid, 1, 1, static_cast<unsigned>(pl.nts[k2]), 1, 1, 0, stream_,
+                                              g.fused ? fargs : args, nullptr));
               DCG_HIP(hipEventRecord(e1, stream_));
               DCG_HIP(hipEventSynchronize(e1));
               float t = 0.f;
@@ -367,6 +403,8 @@ void Batch::rebuild() {
         }
         pl.f64 = pl.f64s[best];
         pl.f32 = pl.f32s[best];
+        pl.k64 = pl.k64s[best];
+        pl.k32 = pl.k32s[best];
         pl.tile = pl.tiles[best];
         pl.nt = pl.nts[best];
         pl.work.upload(items[l][best], stream_);
@@ -383,6 +421,10 @@ void Batch::rebuild() {
       g.nitems = off;
       g.prange.upload(prange, stream_);
       g.part.resize(2 * std::max<size_t>(std::max(vwork.size(), static_cast<size_t>(g.nitems)), 1) + 64);
+      if (g.fused) {
+        g.sck.resize(3 * static_cast<size_t>(M));
+        g.kpart.resize(4 * static_cast<size_t>(g.nitems) + 2 * static_cast<size_t>(g.w.nvwork4) + 64);
+      }
       const int gi = static_cast<int>(&g - sgroups_.data());
       g.op64.range = g.prange.get();
       g.op64.apply = [this, gi](int x, int y, int w1, int w2, double* part, int skip) {
@@ -525,10 +567,87 @@ void Batch::tune(SolverGroup& g) {
   (void)hipEventDestroy(e1);
 }
 
+// Fused BiCGSTAB iterations: both operator launches form their direction and
+// finish the reductions before them (k::BatchOp), so an iteration is 3
+// launches where it was 8; one more per call leaves the scalars in g.sc.
+void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* ev) {
+  const size_t M = g.mem.size();
+  const int np = g.nitems, nx = g.w.nvwork4;
+  double *pa = g.kpart.get(), *pb = pa + np, *pc = pb + 3 * static_cast<size_t>(np);
+  k::BicgScalars* s[3] = {g.sck.get(), g.sck.get() + M, g.sck.get() + 2 * M};
+  const int base = fp32 ? 0 : k::kVKry;
+  const k::PcMember* mem = g.pcm.get();
+  auto mark = [&](int i) {
+    if (ev) DCG_HIP(hipEventRecord(ev[i], stream_));
+  };
+  auto launch = [&](k::BatchOp op) {
+    for (int* v : {&op.a, &op.b, &op.c, &op.d, &op.y, &op.w}) *v += base;
+    for (auto& pl : g.plaunch) {
+      if (pl.nwork <= 0) continue;
+      const int2* work = pl.work.get();
+      int nwork = pl.nwork;
+      op.off = pl.off;
+      void* args[] = {&work, &nwork, &mem, &op};
+      const unsigned grid = static_cast<unsigned>((pl.nwork + 7) / 8 * 8);
+      DCG_HIP(hipModuleLaunchKernel(fp32 ? pl.k32 : pl.k64, grid, 1, 1, static_cast<unsigned>(pl.nt), 1, 1, 0, stream_,
+                                    args, nullptr));
+    }
+  };
+  const int p[2] = {2, 4}, v[2] = {3, 6}, t = 7;
+  for (int it = 0; it < count; ++it) {
+    const int cur = g.parity, nxt = 1 - cur;
+    k::BatchOp op{};
+    op.jac = jacobi_kind();
+    op.mode = 1;
+    op.b = p[cur];
+    op.c = v[cur];
+    op.d = p[nxt];
+    op.y = v[nxt];
+    op.w = 1;
+    op.in = it ? s[0] : g.sc.get();
+    op.out = s[1];
+    op.fin = pc;
+    op.frange = it ? g.w.vrange4 : nullptr;
+    op.fstride = nx;
+    op.range = g.prange.get();
+    op.part = pa;
+    op.pstride = np;
+    mark(0);
+    launch(op);
+    mark(1);
+    op.mode = 2;
+    op.b = op.d = op.w = 0;
+    op.c = v[nxt];
+    op.y = t;
+    op.in = s[1];
+    op.out = s[2];
+    op.fin = pa;
+    op.frange = g.prange.get();
+    op.fstride = np;
+    op.part = pb;
+    mark(2);
+    launch(op);
+    mark(3);
+    op.a = p[nxt];
+    op.in = s[2];
+    op.out = s[0];
+    op.fin = pb;
+    op.range = g.w.vrange4;
+    op.part = pc;
+    op.pstride = nx;
+    if (fp32) k::b_bicg_fused_xr<float>(g.B, g.w, g.mv.get(), k::kVKry + 9, op, stream_);
+    else k::b_bicg_fused_xr<double>(g.B, g.w, g.mv.get(), k::kVZ, op, stream_);
+    g.parity = nxt;
+  }
+  k::b_bicg_finish(g.w, s[0], g.sc.get(), pc, stream_);
+}
+
 void Batch::capture(SolverGroup& g, bool fp32) {
   hipGraph_t graph;
   DCG_HIP(hipStreamBeginCapture(stream_, hipStreamCaptureModeThreadLocal));
-  for (int it = 0; it < opt_.graph_iterations; ++it) {
+  // (an even number of fused iterations: p and v are where they were)
+  if (g.fused) fused_iterations(g, fp32, opt_.graph_iterations * (1 + opt_.graph_iterations % 2), nullptr);
+  for (int it = 0; it < opt_.graph_iterations && !g.fused; ++it) {
     if (fp32)
       k::b_bicg_iteration<float>(g.B, g.variant32, g.w, g.mv.get(), k::kVKry + 9, jacobi_kind(), g.part.get(),
                                  g.sc.get(), stream_, nullptr, g.points ? &g.op32 : nullptr);
@@ -724,7 +843,8 @@ void Batch::norms(const std::vector<char>& on, int x, std::vector<double>& out) 
 // iterations (captured graphs or plain launches), then one read-back of the
 // per-member scalars.
 void Batch::iterate(SolverGroup& g, bool fp32) {
-  const int K = std::max(1, opt_.graph_iterations);
+  const int K = std::max(1, opt_.graph_iterations) * (g.fused && opt_.graph_iterations % 2 ? 2 : 1);
+  g.parity = 0;
   const size_t M = g.mem.size();
   std::vector<k::BicgScalars> sc(M);
   int done_its = 0;
@@ -752,7 +872,9 @@ void Batch::iterate(SolverGroup& g, bool fp32) {
         bytes += mj.point_storage() ? mj.point_apply_bytes(fp32 ? 4 : 8, 1) : mj.spmv_bytes(fp32 ? 4 : 8, fp32 ? 4 : 8, 1);
       }
       if (all || done_its > opt_.lin_maxit + 4) break;
-      if (fp32)
+      if (g.fused)
+        fused_iterations(g, fp32, 1, ev_);
+      else if (fp32)
         k::b_bicg_iteration<float>(g.B, g.variant32, g.w, g.mv.get(), k::kVKry + 9, jacobi_kind(), g.part.get(),
                                    g.sc.get(), stream_, ev_, g.points ? &g.op32 : nullptr);
       else
@@ -777,6 +899,8 @@ void Batch::iterate(SolverGroup& g, bool fp32) {
       if (opt_.graph_iterations > 0) {
         if (!g.graph[fp32 ? 1 : 0]) capture(g, fp32);
         DCG_HIP(hipGraphLaunch(g.graph[fp32 ? 1 : 0], stream_));
+      } else if (g.fused) {
+        fused_iterations(g, fp32, 1, nullptr);
       } else if (fp32) {
         k::b_bicg_iteration<float>(g.B, g.variant32, g.w, g.mv.get(), k::kVKry + 9, jacobi_kind(), g.part.get(),
                                    g.sc.get(), stream_, nullptr, g.points ? &g.op32 : nullptr);

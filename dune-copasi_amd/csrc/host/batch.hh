@@ -130,10 +130,11 @@ class Batch {
       // the kernels and tile shape in use, chosen by timing among the
       // module's candidate tile shapes
       hipFunction_t f64 = nullptr, f32 = nullptr;
+      hipFunction_t k64 = nullptr, k32 = nullptr;  // of fused iterations
       std::shared_ptr<RtcModule> module;
       std::array<int, 3> tile{};
       int nt = 256;  // workgroup size
-      std::vector<hipFunction_t> f64s, f32s;
+      std::vector<hipFunction_t> f64s, f32s, k64s, k32s;
       std::vector<std::array<int, 3>> tiles;
       std::vector<int> nts;
       DeviceArray<int2> work;
@@ -144,7 +145,16 @@ class Batch {
     DeviceArray<int2> prange;
     int nitems = 0;
     k::BatchOperator op64, op32;
+    // members that evaluate their coefficients: fused iterations (3 launches
+    // per module, 2 of them operators), with the scalars handed from launch to
+    // launch in sck (M each) and partials of their own
+    bool fused = false;
+    int parity = 0;  // which of the two p and v a fused iteration reads
+    DeviceArray<k::BicgScalars> sck;
+    DeviceArray<double> kpart;
   };
+  // `count` iterations from the scalars in g.sc and back to them
+  void fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* ev);
   struct AsmGroup {
     std::shared_ptr<RtcModule> module;
     std::vector<hipFunction_t> fn;  // batched tile kernel per compartment (or null)

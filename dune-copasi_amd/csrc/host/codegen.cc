@@ -258,6 +258,7 @@ struct dcg_pc_member {
   float* f[10];
   const int* done;
   const int* irdone;
+  const double* dinv;
 };
 static_assert(sizeof(dcg_asm_member) == %ASM_BYTES%, "batch member descriptor layout");
 static_assert(sizeof(dcg_pc_member) == %PCM_BYTES%, "point member descriptor layout");
@@ -2953,6 +2954,42 @@ const char* kEvalKrylovEntries = R"(
 #undef DCG_EVAL_ENTRY
 )";
 
+// One operator launch of a fused iteration over (member, tile) items (BatchOp)
+const char* kEvalBatch = R"(
+#define DCG_KBATCH_ENTRY(NAME, T, VEC, TL, FN)                                                                    \
+  extern "C" __global__ void __launch_bounds__(TL::NT, TL::MINW)                                                  \
+  NAME(const int2* __restrict__ work, int nwork, const dcg_pc_member* __restrict__ mem, BatchOp bo) {             \
+    const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
+    if (c >= nwork) return;                                                                                       \
+    const int2 w = work[c];                                                                                       \
+    const dcg_pc_member& M = mem[w.x];                                                                            \
+    KrylovOp op;                                                                                                  \
+    op.mode = bo.mode;                                                                                            \
+    op.jac = bo.jac;                                                                                              \
+    op.a = M.VEC[bo.a];                                                                                           \
+    op.b = M.VEC[bo.b];                                                                                           \
+    op.c = M.VEC[bo.c];                                                                                           \
+    op.d = M.VEC[bo.d];                                                                                           \
+    op.y = M.VEC[bo.y];                                                                                           \
+    op.w = M.VEC[bo.w];                                                                                           \
+    op.dinv = M.dinv;                                                                                             \
+    op.in = bo.in + w.x;                                                                                          \
+    op.out = bo.out + w.x;                                                                                        \
+    const int2 fr = bo.frange ? bo.frange[w.x] : make_int2(0, 0);                                                 \
+    op.fin = bo.fin + fr.x;                                                                                       \
+    op.nfin = fr.y - fr.x;                                                                                        \
+    op.fstride = bo.fstride;                                                                                      \
+    op.pstride = bo.pstride;                                                                                      \
+    op.off = bo.off;                                                                                              \
+    op.part = bo.part;                                                                                            \
+    %C%::FN<TL, T>(w.y, c, (%C%::dcg_gp<const int>)M.g2l, (%C%::dcg_gp<const unsigned char>)M.cmask,              \
+                   (%C%::dcg_gp<const double>)M.pc, op, bo.off + c == bo.range[w.x].x,                            \
+                   (%C%::dcg_gp<const double>)M.tca, M.n[0], M.n[1], M.n[2], M.prm);                              \
+  }
+%KBATCH_ENTRIES%
+#undef DCG_KBATCH_ENTRY
+)";
+
 // Box cells with blocks of more than 4 species: one lane per (cell, corner).
 // A thread that holds all corners of a cell would need 2^DIM values per
 // species several times over; here a lane holds one corner's values, which
@@ -3902,7 +3939,7 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     if (geo && comp < 4) body += kCornerBatch;
     if (geo && comp < 4 && points) body += kCornerPointBatch;
     const auto shapes = corner_tiles(d);
-    std::string cs, ce, cb;
+    std::string cs, ce, cb, kb;
     for (size_t k2 = 0; k2 < shapes.size(); ++k2) {
       const std::string id = std::to_string(k2), tl = ns + "::CornerShape" + id;
       cs += "using CornerShape" + id + " = CornerTile<" + std::to_string(shapes[k2][0]) + ", " +
@@ -3910,8 +3947,12 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
       ce += "DCG_EVAL_ENTRY(%KERNEL%_e" + id + ", double, " + tl + ", corner_krylov)\n";
       ce += "DCG_EVAL_ENTRY(%KERNEL%_ef" + id + ", float, " + tl + ", corner_krylov)\n";
       cb += "DCG_CORNER_BENTRY(%KERNEL%_ebatch" + id + ", double, v, " + tl + ")\n";
-      cb += "DCG_CORNER_BENTRY(%KERNEL%_efbatch" + id + ", float, f, " + tl + ")\n";
+      if (!(geo && comp < 4 && points)) continue;
+      kb += "DCG_KBATCH_ENTRY(%KERNEL%_kbatch" + id + ", double, v, " + tl + ", corner_krylov)\n";
+      kb += "DCG_KBATCH_ENTRY(%KERNEL%_kfbatch" + id + ", float, f, " + tl + ", corner_krylov)\n";
     }
+    if (!kb.empty()) body += kEvalBatch;
+    replace_all(body, "%KBATCH_ENTRIES%", kb);
     replace_all(body, "%CORNER_SHAPES%", cs);
     replace_all(body, "%EVAL_ENTRIES%", ce);
     replace_all(body, "%CORNER_BENTRIES%", cb);
@@ -3920,8 +3961,10 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
     if (points) body += kTiledPoints;
     if (geo && comp < 4 && points) body += kTiledPointBatch;
     // one point apply (and batched point apply) per candidate tile shape k:
-    // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k> (_e.. where evaluated)
-    std::string pe, pb;
+    // %KERNEL%_p<k>, _pf<k>, _pbatch<k>, _pfbatch<k>; where evaluated _e<k>,
+    // _ef<k>, _ebatch<k> and the fused iteration's _kbatch<k>, _kfbatch<k>
+    std::string pe, pb, kb;
+    std::string en2;
     bool any_march = false;
     const std::string en = eval ? "e" : "p";
     for (size_t k2 = 0; k2 < apply_tiles.size(); ++k2) {
@@ -3934,7 +3977,12 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
       pe += entry + "(%KERNEL%_" + en + "f" + id + ", float, " + tl + fn + ")\n";
       any_march = any_march || march;
       pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "batch" + id + ", double, v, pc, " + tl + ")\n";
-      pb += "DCG_PBATCH_ENTRY(%KERNEL%_" + en + "fbatch" + id + ", float, f, " + (eval ? "pc, " : "pc32, ") + tl + ")\n";
+      if (!eval) {
+        pb += "DCG_PBATCH_ENTRY(%KERNEL%_pfbatch" + id + ", float, f, pc32, " + tl + ")\n";
+      } else if (geo && comp < 4) {
+        kb += "DCG_KBATCH_ENTRY(%KERNEL%_kbatch" + id + ", double, v, " + tl + ", eval_krylov)\n";
+        kb += "DCG_KBATCH_ENTRY(%KERNEL%_kfbatch" + id + ", float, f, " + tl + ", eval_krylov)\n";
+      }
     }
     // the candidate apply shapes as plain names (macro arguments hold no commas)
     std::string as;
@@ -3945,7 +3993,9 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
                                               false)) +
             ", " + std::to_string(k2 < apply_waves.size() ? apply_waves[k2] : 1) + ">;\n";
     replace_all(body, "%APPLY_SHAPES%", as);
-    if (eval) body += std::string(kEvalKrylov) + kEvalKrylovCells + (any_march ? kEvalMarch : "") + kEvalKrylovEntries;
+    if (!kb.empty()) en2 = kEvalBatch;
+    if (eval) body += std::string(kEvalKrylov) + kEvalKrylovCells + (any_march ? kEvalMarch : "") + kEvalKrylovEntries + en2;
+    replace_all(body, "%KBATCH_ENTRIES%", kb);
     replace_all(body, "%POINT_ENTRIES%", eval ? "" : pe);
     replace_all(body, "%EVAL_ENTRIES%", eval ? pe : "");
     replace_all(body, "%PBATCH_ENTRIES%", pb);
@@ -3964,7 +4014,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
   replace_all(pre, "%GEO%", geo ? "1" : "0");
   replace_all(pre, "%UNS%", L.grid.unstructured ? "1" : "0");
   // the fused Krylov launches' types and scalar update (bicg_scalars.hh)
-  replace_all(pre, "%KRYLOV%", points ? std::string(DCG_STR(DCG_BICG_STRUCT DCG_KRYLOV_OP_STRUCT)) +
+  replace_all(pre, "%KRYLOV%", points ? std::string(DCG_STR(DCG_BICG_STRUCT DCG_KRYLOV_OP_STRUCT DCG_BATCH_OP_STRUCT)) +
                                             "\nstatic_assert(sizeof(KrylovOp) == " +
                                             std::to_string(sizeof(k::KrylovOp)) + ", \"operator arguments\");\n" +
                                             DCG_STR(DCG_BICG_UPDATE) + "\n" + DCG_STR(DCG_KRYLOV_FINISH) + "\n"

@@ -446,6 +446,82 @@ __global__ void __launch_bounds__(kThreads) bfin_k(const int2* __restrict__ rang
   if (threadIdx.x == 0) bicg_update(sc + m, stage, v[0], v[1]);
 }
 
+// The x and r update of a fused iteration, as bicg_fused_xr_k: s and both
+// preconditioned directions are recomputed from p and v.
+template <int B, typename V>
+__global__ void __launch_bounds__(kThreads) bfused_xr_k(const int2* __restrict__ work,
+                                                        const MemberView* __restrict__ mv, int x, BatchOp op) {
+  __shared__ double red[32];
+  const int2 w = work[blockIdx.x];
+  const int2 fr = op.frange[w.x];
+  BicgScalars sc;
+  if (!finish_stage<kThreads, 3>(sc, op.in + w.x, op.out + w.x, (int)blockIdx.x == op.range[w.x].x, op.fin + fr.x,
+                                 fr.y - fr.x, op.fstride, 2, red))
+    return;
+  const MemberView& m = mv[w.x];
+  double acc[2] = {0.0, 0.0};
+  const bool half = sc.half != 0;
+  const auto xv = in_global(vsel<V>(m, x));
+  const auto r = in_global(vsel<V>(m, kVKry + 0));
+  const auto rh = in_global(vsel<V>(m, kVKry + 1));
+  const auto p = in_global(vsel<V>(m, kVKry + op.a));
+  const auto v = in_global(vsel<V>(m, kVKry + op.c));
+  const auto t = in_global(vsel<V>(m, kVKry + op.y));
+  const double* dinv = (const double*)in_global(m.dinv);
+  const double alpha = sc.alpha, omega = sc.omega;
+#pragma unroll
+  for (int u = 0; u < kBVecSlots; ++u) {
+    const int s = (w.y * kBVecSlots + u) * kThreads + threadIdx.x;
+    if (s >= m.nslot) break;
+    const size_t k0 = (size_t)s * B;
+    V x0[B], pv[B], ph[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) x0[i] = xv[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) ph[i] = pv[i] = p[k0 + i];
+    if (op.jac) dinv_apply<B>(dinv, s, pv, ph, op.jac == 2);
+    if (half) {
+#pragma unroll
+      for (int i = 0; i < B; ++i) xv[k0 + i] = (V)((double)x0[i] + alpha * (double)ph[i]);
+      continue;
+    }
+    V rv[B], vv[B], tv[B], hv[B], sw[B], sh[B];
+#pragma unroll
+    for (int i = 0; i < B; ++i) rv[i] = r[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) vv[i] = v[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) tv[i] = t[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) hv[i] = rh[k0 + i];
+#pragma unroll
+    for (int i = 0; i < B; ++i) sh[i] = sw[i] = (V)((double)rv[i] - alpha * (double)vv[i]);
+    if (op.jac) dinv_apply<B>(dinv, s, sw, sh, op.jac == 2);
+#pragma unroll
+    for (int i = 0; i < B; ++i) {
+      xv[k0 + i] = (V)((double)x0[i] + alpha * (double)ph[i] + omega * (double)sh[i]);
+      const V rn = (V)((double)sw[i] - omega * (double)tv[i]);
+      r[k0 + i] = rn;
+      acc[0] += (double)hv[i] * (double)rn;
+      acc[1] += (double)rn * (double)rn;
+    }
+  }
+  group_sums<kThreads, 2>(acc, red);
+  if (threadIdx.x == 0) {
+    op.part[blockIdx.x] = acc[0];
+    op.part[op.pstride + blockIdx.x] = acc[1];
+  }
+}
+__global__ void __launch_bounds__(kThreads) bfinish_k(const int2* __restrict__ range, const BicgScalars* __restrict__ in,
+                                                      BicgScalars* __restrict__ out, const double* __restrict__ fin,
+                                                      int fstride) {
+  __shared__ double red[32];
+  const int m = blockIdx.x;
+  const int2 r = range[m];
+  BicgScalars sc;
+  finish_stage<kThreads, 2>(sc, in + m, out + m, true, fin + r.x, r.y - r.x, fstride, 4, red);
+}
+
 // ----------------------------------------------------------------- refinement
 __global__ void birbegin_k(int members, Skip sk, const double* __restrict__ rtol, const double* __restrict__ sums,
                            IrState* __restrict__ ir) {
@@ -632,6 +708,17 @@ template void b_bicg_iteration<double>(int, int, const BatchWork&, const MemberV
                                        BicgScalars*, hipStream_t, hipEvent_t*, const BatchOperator*);
 template void b_bicg_iteration<float>(int, int, const BatchWork&, const MemberView*, int, int, double*,
                                       BicgScalars*, hipStream_t, hipEvent_t*, const BatchOperator*);
+
+template <typename V>
+void b_bicg_fused_xr(int B, const BatchWork& w, const MemberView* mv, int x, const BatchOp& op, hipStream_t st) {
+  if (w.nvwork4 <= 0) return;
+  DCG_BATCH_B(B, (bfused_xr_k<BB, V><<<w.nvwork4, kThreads, 0, st>>>(w.vwork4, mv, x, op)));
+}
+template void b_bicg_fused_xr<double>(int, const BatchWork&, const MemberView*, int, const BatchOp&, hipStream_t);
+template void b_bicg_fused_xr<float>(int, const BatchWork&, const MemberView*, int, const BatchOp&, hipStream_t);
+void b_bicg_finish(const BatchWork& w, const BicgScalars* in, BicgScalars* out, const double* fin, hipStream_t st) {
+  if (w.members > 0) bfinish_k<<<w.members, kThreads, 0, st>>>(w.vrange4, in, out, fin, w.nvwork4);
+}
 
 void b_spmv64(int B, int variant, const BatchWork& w, const MemberView* mv, Skip sk, int x, int y, hipStream_t st) {
   DCG_BATCH_B(B, (bspmv_launch<BB, double, double>(variant, w, mv, sk, nullptr, x, y, -1, -1, nullptr, st)));

@@ -33,6 +33,21 @@
     double* part;                                                \
   };
 
+// The same launch over the members of a batch: vectors by index, the scalars
+// one per member (in[m], out[m]), frange[m] = member m's partials of the
+// previous launch (null: none to finish) and range[m] of this one, whose work
+// items are numbered from off.
+#define DCG_BATCH_OP_STRUCT                                      \
+  struct BatchOp {                                               \
+    int mode, jac, fstride, pstride, off;                        \
+    int a, b, c, d, y, w;                                        \
+    const int2 *frange, *range;                                  \
+    const BicgScalars* in;                                       \
+    BicgScalars* out;                                            \
+    const double* fin;                                           \
+    double* part;                                                \
+  };
+
 // Updates the scalars after one reduction stage; v0/v1 are its reduced sums.
 // 0: v0 = r.r at the start (rho = r.r since rh = r).  1: after v = A ph,
 // alpha = rho / (rh.v).  2: after s, half-step convergence test.  3: after

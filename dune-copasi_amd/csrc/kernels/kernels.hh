@@ -32,6 +32,7 @@ struct SpmvPlan {
 // a fused operator launch (bicg_scalars.hh).
 DCG_BICG_STRUCT
 DCG_KRYLOV_OP_STRUCT
+DCG_BATCH_OP_STRUCT
 
 // Interface facets of a fused operator, by the slots they touch: kernel kind
 // k's records at fint[k] / fdbl[k]; the entries of slot[i] are ent[ptr[i]] ..
@@ -122,6 +123,7 @@ struct PcMember {
   float* f[kBatchVecF] = {};
   const int* done = nullptr;    // BicgScalars::done of the member's Krylov solve
   const int* irdone = nullptr;  // IrState::done of its refinement
+  const double* dinv = nullptr;
 };
 
 // The operator of a batched Krylov solve when it is not the members' BCSR
@@ -206,6 +208,13 @@ void b_bicg_init(int B, const BatchWork& w, const MemberView* mv, int b, int x, 
                  hipStream_t st);
 // one BiCGSTAB iteration on every unfinished member (jacobi: apply dinv)
 // ev (optional, 4 events): recorded before and after each of the two SpMVs
+// A fused iteration's x and r update over the members (after its second
+// operator launch, op: the finish of that launch's partials, and where this
+// one's scalars and partials go; vectors p = op.a, v = op.c), and the finish of
+// its reductions into out for the host and the next block of iterations.
+template <typename V>
+void b_bicg_fused_xr(int B, const BatchWork& w, const MemberView* mv, int x, const BatchOp& op, hipStream_t s);
+void b_bicg_finish(const BatchWork& w, const BicgScalars* in, BicgScalars* out, const double* fin, hipStream_t s);
 template <typename V>
 void b_bicg_iteration(int B, int variant, const BatchWork& w, const MemberView* mv, int x, int jacobi,
                       double* part, BicgScalars* sc, hipStream_t st, hipEvent_t* ev = nullptr,

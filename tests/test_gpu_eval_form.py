@@ -108,3 +108,32 @@ def test_steps(dca, dim, cells, species, inner, precision, precond, costly):
     assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], orc.get_state()[0])) < 1e-8
     gpu.close()
     orc.close()
+
+
+@pytest.mark.parametrize("graph", [0, 3, 4])
+@pytest.mark.parametrize("precision,precond", [("fp64", "Jacobi"), ("mixed", "Jacobi"), ("fp64", "VertexBlockJacobi"),
+                                               ("mixed", "None")])
+def test_batch(dca, precision, precond, graph):
+    """Members of several modules, sizes and block sizes (one with stored coefficients) on fused iterations, as
+    plain launches and captured in odd and even numbers."""
+    print(f"case: evaluated form batch {precision} {precond} graph_iterations={graph}", flush=True)
+    inis = [_ini(2, (33, 20), 2), _ini(2, (7, 50), 2, extensions=(0.5, 2.0, 1.0)), _ini(2, (16, 9), 2, costly=True),
+            _ini(3, (9, 8, 6), 3), _ini(2, (1, 1), 4), _ini(3, (4, 5, 7), 6)]
+    batch = dca.Batch(f"precision = {precision}\npreconditioner = {precond}\ngraph_iterations = {graph}\n"
+                      "iteration_limit = 2000\n", 0)
+    members, oracles = [], []
+    for ini in inis:
+        i = batch.add(ini)
+        batch.set_time_step(i, 0.1)
+        m, o = batch.member(i), OracleModel(ini)
+        u0 = 0.5 + 0.2 * np.random.default_rng(i).random(m.n_dof)
+        m.set_state(u0, 0.0)
+        o.set_state(u0, 0.0)
+        members.append(m)
+        oracles.append(o)
+    for _ in range(3):
+        assert all(s.status == 0 for s in batch.step())
+        for o in oracles:
+            assert o.step(0.1)[0] == 0
+        for m, o in zip(members, oracles):
+            assert max(rel_l2_per_species(m.compartments(), m.get_state()[0], o.get_state()[0])) < 1e-8
