@@ -387,6 +387,7 @@ __global__ void __launch_bounds__(kThreads) dot_parts_k(long n, const V* __restr
 // workgroup is contiguous): more bytes in flight per thread and a quarter of
 // the workgroup reductions of one slot per thread.
 constexpr int kXrSlots = 4;
+constexpr int kFusedXrWide = 512 * 256;
 template <int B, typename V>
 __global__ void __launch_bounds__(kThreads) bicg_xr_k(int nslot, V* __restrict__ x, const V* __restrict__ ph,
                                                       const V* __restrict__ sh, const V* __restrict__ sv,
@@ -459,7 +460,7 @@ __global__ void __launch_bounds__(kThreads) bicg_xr_k(int nslot, V* __restrict__
 // The x and r update of a fused iteration (the operator launches compute p,
 // ph, s and sh on their own boxes and store p alone): s and both
 // preconditioned directions are recomputed here.  7 vectors read, 2 written.
-template <int B, typename V>
+template <int B, typename V, int U>
 __global__ void __launch_bounds__(kThreads) bicg_fused_xr_k(int nslot, V* __restrict__ x, const V* __restrict__ p,
                                                             const V* __restrict__ v, const V* __restrict__ t,
                                                             V* __restrict__ r, const V* __restrict__ rh,
@@ -475,8 +476,8 @@ __global__ void __launch_bounds__(kThreads) bicg_fused_xr_k(int nslot, V* __rest
   const bool half = sc.half != 0;
   const double alpha = sc.alpha, omega = sc.omega;
 #pragma unroll
-  for (int u = 0; u < kXrSlots; ++u) {
-    const int s = (blockIdx.x * kXrSlots + u) * blockDim.x + threadIdx.x;
+  for (int u = 0; u < U; ++u) {
+    const int s = (blockIdx.x * U + u) * blockDim.x + threadIdx.x;
     if (s >= nslot) continue;
     const size_t k0 = (size_t)s * B;
     V xv[B], pv[B], ph[B];
@@ -1466,15 +1467,28 @@ void bicg_finish(const BicgScalars* in, BicgScalars* out, const double* fin, int
   else if (stage == 2) bicg_finish_k<3><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, 2);
   else bicg_finish_k<2><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, stage);
 }
-int bicg_fused_xr_parts(int nslot) { return (nslot + kThreads * kXrSlots - 1) / (kThreads * kXrSlots); }
+// Slots per thread of the x and r update: 4 for meshes whose workgroups fill
+// the chip twice over, 1 below, where four times the workgroups load at once
+// (4 slots -> 1: 25^2 FP64 4.7 -> 3.6 us, 48^3 FP32 7.3 -> 5.8 us, 41^3 with 7
+// species FP32 9.2 -> 6.6 us, 301^2 with 4 species FP32 8.7 -> 6.2 us)
+static int fused_xr_slots(int nslot) { return nslot > kFusedXrWide ? kXrSlots : 1; }
+int bicg_fused_xr_parts(int nslot) {
+  const int per = kThreads * fused_xr_slots(nslot);
+  return (nslot + per - 1) / per;
+}
 template <typename V>
 int bicg_fused_xr(int B, int nslot, V* x, const V* p, const V* v, const V* t, V* r, const V* rh, const double* dinv,
                   int jac, const BicgScalars* in, BicgScalars* out, const double* fin, int nfin, int fstride,
                   double* part, int pstride, hipStream_t s) {
   const int grid = bicg_fused_xr_parts(nslot);
-  if (grid > 0)
-    DCG_DISPATCH_B(B, (bicg_fused_xr_k<BB, V><<<grid, kThreads, 0, s>>>(nslot, x, p, v, t, r, rh, dinv, jac, in, out,
-                                                                        fin, nfin, fstride, part, pstride)));
+  if (grid <= 0) return grid;
+  if (fused_xr_slots(nslot) == 1) {
+    DCG_DISPATCH_B(B, (bicg_fused_xr_k<BB, V, 1><<<grid, kThreads, 0, s>>>(nslot, x, p, v, t, r, rh, dinv, jac, in, out,
+                                                                           fin, nfin, fstride, part, pstride)));
+  } else {
+    DCG_DISPATCH_B(B, (bicg_fused_xr_k<BB, V, kXrSlots><<<grid, kThreads, 0, s>>>(
+                          nslot, x, p, v, t, r, rh, dinv, jac, in, out, fin, nfin, fstride, part, pstride)));
+  }
   return grid;
 }
 template int bicg_fused_xr<double>(int, int, double*, const double*, const double*, const double*, double*,

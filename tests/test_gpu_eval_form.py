@@ -110,6 +110,21 @@ def test_steps(dca, dim, cells, species, inner, precision, precond, costly):
     orc.close()
 
 
+@pytest.mark.parametrize("cells", [(361, 361), (362, 362)])
+def test_step_slots_per_thread(dca, cells):
+    """Meshes just below and above the 131,072 vertices where the x and r update takes four slots per thread."""
+    print(f"case: evaluated form slots {cells}", flush=True)
+    ini = _ini(2, cells, 1)
+    gpu, orc = dca.Model(ini, PTS.format("Jacobi", "fp64"), 0), OracleModel(ini)
+    u0 = gpu.initial_state()
+    gpu.set_state(u0, 0.0)
+    orc.set_state(u0, 0.0)
+    assert gpu.step(0.0, 0.1).status == 0 and orc.step(0.1)[0] == 0
+    assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], orc.get_state()[0])) < 1e-8
+    gpu.close()
+    orc.close()
+
+
 @pytest.mark.parametrize("graph", [0, 3, 4])
 @pytest.mark.parametrize("precision,precond", [("fp64", "Jacobi"), ("mixed", "Jacobi"), ("fp64", "VertexBlockJacobi"),
                                                ("mixed", "None")])
