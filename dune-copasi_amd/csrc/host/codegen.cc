@@ -2449,8 +2449,9 @@ extern "C" __global__ void __launch_bounds__(256)
 // workgroup stores the new p of its own rows; halo vertices recompute it.
 // An iteration is 3 launches (5 with the finishers of large meshes) and the
 // facets' 2, where it was 8 and up to 12 of facets.  Runs of time steps, with
-// the evaluation: 24^2 6.7 -> 4.4 ms; 47^3 mixed 35.0 -> 27.6 ms; 96^3 85 -> 70
-// ms; with an interface 300^2 mixed 17.6 -> 10.2 ms, 1024^2 167 -> 112 ms.
+// the evaluation and the walked layers below: 24^2 6.4 -> 4.0 ms; 47^3 mixed
+// 34.0 -> 26.4 ms; 96^3 85 -> 49 ms; with an interface 300^2 mixed 17.2 -> 9.8
+// ms, 1024^2 160 -> 96 ms.
 const char* kEvalKrylov = R"(
 namespace %C% {
 // M^-1 q at slot s (jac 0: none, 1: a block per slot, 2: the diagonal)
