@@ -1083,8 +1083,9 @@ int Model::krylov_parts() const {
 }
 
 // One operator launch of the fused iteration (k::KrylovOp): the compartments'
-// tiles one after the other in the partials, then the facet rows, which take
-// the scalars that the first compartment's launch has stored.
+// tiles one after the other in the partials, then the facet rows.  The first
+// launch finishes the reduction before it, the others take the scalars it
+// has stored.
 int Model::launch_krylov_op(k::KrylovOp op, bool fp32) {
   const Grid& g = L_.grid;
   int n0 = static_cast<int>(g.n[0]), n1 = g.dim > 1 ? static_cast<int>(g.n[1]) : 1;
@@ -1107,10 +1108,14 @@ int Model::launch_krylov_op(k::KrylovOp op, bool fp32) {
     DCG_HIP(hipModuleLaunchKernel(fp32 ? pc_appf_fns_[c][k2] : pc_app_fns_[c][k2], grid, 1, 1,
                                   static_cast<unsigned>(gen_.apply_threads[c][k2]), 1, 1, 0, stream_, args, nullptr));
     op.off += ntile;
+    // one set of scalars per operator: the launches that follow take what the
+    // first one has stored (a sum of their own would run in their workgroup's
+    // order and differ in the last bits, in the convergence tests too)
     op.lead = 0;
+    op.nfin = 0;
+    op.in = op.out;
   }
   if (frows_.nslot) {
-    if (op.mode) op.in = op.out;  // the scalars after this launch's reduction
     k::FacetRows rows = frows_;
     void* args[] = {&rows, &lin, &op, &tca, &prm};
     DCG_HIP(hipModuleLaunchKernel(fp32 ? facet_rows_f_fn_ : facet_rows_fn_,

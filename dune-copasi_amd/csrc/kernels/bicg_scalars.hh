@@ -15,10 +15,11 @@
 // Arguments of one operator launch of a fused BiCGSTAB iteration.  mode 0:
 // y = J a.  mode 1: p = a + beta (b - omega c) into d, y = J M^-1 p, partial
 // y.w.  mode 2: s = a - alpha c, y = J M^-1 s, partials y.s, y.y, s.s.  Modes
-// 1 and 2 first finish the previous launch's reduction: every workgroup sums
-// the same partials (fin[j * fstride + i], i < nfin) in the same order and
-// updates its copy of *in; the leading launch's first workgroup stores it to
-// *out.  part[j * pstride + off + workgroup] gets this launch's partials.
+// 1 and 2 first finish the previous launch's reduction: every workgroup of the
+// leading launch sums the same partials (fin[j * fstride + i], i < nfin) in the
+// same order and updates its copy of *in; its first workgroup stores it to
+// *out, which the launches of further compartments and of the facet rows take
+// as it is (in = out, nfin = 0).  part[j * pstride + off + workgroup] gets this launch's partials.
 // jac: 0 no preconditioner, 1 a block per slot, 2 the diagonal (in dinv).
 #define DCG_KRYLOV_OP_STRUCT                                     \
   struct KrylovOp {                                              \

@@ -152,3 +152,59 @@ def test_batch(dca, precision, precond, graph):
             assert o.step(0.1)[0] == 0
         for m, o in zip(members, oracles):
             assert max(rel_l2_per_species(m.compartments(), m.get_state()[0], o.get_state()[0])) < 1e-8
+
+
+def test_compartments_share_scalars(dca):
+    """Two compartments whose forced tiles have 256 and 512 threads, about 400 partials: every launch of an iteration
+    works with one set of scalars.  The initial state makes r.(J r) cancel to 1e-6 of its terms, so alpha is 1e6 with a
+    relative rounding of about 1e-10: compartments with an alpha each leave parts of the right-hand side unsolved (4e-6
+    where it happened); with one alpha the true residual is the recursion's (1e-8) up to 1e6 roundings: 1e-7.  The
+    state comes from a linear step, which has no later defect test."""
+    print("case: evaluated form, scalars of two compartments", flush=True)
+    n, off = 40, 41 * 41 * 21 * 4
+    out = [f"[grid]\ndimension = 3\ncells = {n} {n} {n}\nextensions = 1 1 1\ncell_type = cube",
+           "[compartments]\nlow.expression = position_z < 0.5\nhigh.expression = position_z >= 0.5"]
+    for comp, names in (("low", ["a0", "a1", "a2", "a3"]), ("high", ["b0", "b1"])):
+        for i, s in enumerate(names):
+            jac = {s: "-1"}
+            if i % 2 == 0:
+                jac[names[i + 1]] = "8"
+            if comp == "low":  # a full block, so that the compartments' candidate tiles differ
+                jac.update({o: "1e-30" for o in names if o not in jac})
+            out += [f"[model.scalar_field.{s}]", f"compartment = {comp}", "storage.expression = 1",
+                    "reaction.expression = " + " + ".join(f"{c}*{o}" for o, c in jac.items())]
+            out += [f"reaction.jacobian.{o}.expression = {c}" for o, c in jac.items()]
+    ini = "\n".join(out) + ("\n[model]\nis_linear = true\n[model.time_step_operator]\ntype = ImplicitEuler\n"
+                            "linear_solver.type = BiCGSTAB\n"
+                            "linear_solver.convergence_condition.relative_tolerance = 1e-8\n"
+                            "linear_solver.convergence_condition.iteration_range = 1 500\n"
+                            "linear_solver.preconditioner.type = None\n")
+    orc = OracleModel(ini)
+    _, vals = orc.assemble(np.zeros(orc.n_dof), 1.0, 1.0, 1.0)
+    A = orc.csr(vals)
+    x = [np.tile(np.arange(n + 1) / n, 41 * 21) for _ in range(2)]
+
+    def state(inside, sign):  # whose reaction is (1, sign) per pair of species at the vertices inside, else 0
+        u = np.zeros(orc.n_dof)
+        for part, xs, b in ((u[:off], x[0], 4), (u[off:], x[1], 2)):
+            g = inside(xs)[:, None]
+            part.reshape(-1, b)[:, 1::2] = -sign * g
+            part.reshape(-1, b)[:, 0::2] = -(8 * sign + 1) * g
+        return u
+
+    P, Q = state(lambda s: 1.0 * (s < 0.75), 1.0), state(lambda s: 1.0 * (s >= 0.75), -1.0)
+    rP, rQ = orc.assemble(P, 1.0, 0.0, 1.0)[0], orc.assemble(Q, 1.0, 0.0, 1.0)[0]
+    pp, pq, qq = rP @ (A @ rP), rP @ (A @ rQ) + rQ @ (A @ rP), rQ @ (A @ rQ)
+    assert pp < 0 < qq
+    a = max(np.roots([qq, pq, pp - 1e-6 * (qq - pp)]).real)
+    b = rP + a * rQ
+    gpu = dca.Model(ini, PTS.format("None", "fp64") + "model.time_step_operator.linear_solver.point_tile = 2\n", 0)
+    src = gpu.generated_source()
+    assert "ApplyShape2 = ApplyTile<7, 7, 3, 256" in src and "ApplyShape2 = ApplyTile<7, 7, 7, 512" in src
+    gpu.set_state(P + a * Q, 0.0)
+    st = gpu.step(0.0, 1.0)
+    assert st.status == 0
+    z = P + a * Q - gpu.get_state()[0]
+    assert np.linalg.norm(b - A @ z) <= 1e-7 * np.linalg.norm(b)
+    gpu.close()
+    orc.close()
