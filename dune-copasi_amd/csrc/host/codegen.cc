@@ -3005,6 +3005,9 @@ const char* kEvalBatch = R"(
 // is one lane exchange per axis (DPP, no LDS) and one FMA.  The coefficients
 // of the Jacobian are evaluated at the linearisation point inside the apply,
 // so an apply reads two vectors instead of a matrix or stored coefficients.
+// The FP32 apply reads and stores FP32 vectors and sums a row's terms in FP64
+// (40^3 with 7 species, mixed steps: 1.8% slower than with FP32 sums, 1% over
+// a batch of networks), as the SpMV on the FP32 matrix does.
 // A workgroup takes the cells around TX x TY row vertices of a layer and walks
 // TM layers along the last axis; a layer's corner sums meet in LDS, and what
 // it adds to the next layer's vertices stays in a register.
@@ -3033,18 +3036,14 @@ __device__ __forceinline__ int corner_dpp(int v) {
   return __builtin_amdgcn_mov_dpp(v, A == 0 ? 0xB1 : A == 1 ? 0x4E : 0x141, 0xF, 0xF, true);
 }
 template <int A>
-__device__ __forceinline__ float other_end(float v) {
-  return __int_as_float(corner_dpp<A>(__float_as_int(v)));
-}
-template <int A>
 __device__ __forceinline__ double other_end(double v) {
   const long long u = __double_as_longlong(v);
   const int lo = corner_dpp<A>((int)u), hi = corner_dpp<A>((int)(u >> 32));
   return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 // sums (bit 0) and differences (bit 1) over the corners along every axis
-template <typename T, int N>
-__device__ __forceinline__ void butterfly(T (&v)[N], const T (&sg)[3]) {
+template <int N>
+__device__ __forceinline__ void butterfly(double (&v)[N], const double (&sg)[3]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     v[i] = fma(v[i], sg[0], other_end<0>(v[i]));
@@ -3068,12 +3067,11 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
   constexpr int TX = TL::TX, TY = TL::TY, TM = TL::TM, CX = TL::CX, NT = TL::NT;
 %CORNER_OP_BEGIN%
   constexpr int PER = (TL::ROWS * DCG_B + NT - 1) / NT;
-  __shared__ T out[BC * NT];
+  __shared__ double out[BC * NT];
   const int tid = threadIdx.x, l = tid % NCORNER, cell = tid / NCORNER;
   const int cx = cell % CX, cy = cell / CX;
   const int b2 = DIM > 2 ? l >> 2 : 0, la = l ^ (b2 ? 7 : 0), b0 = la & 1, b1 = (la >> 1) & 1;
   const int mb = DIM > 2 ? b2 : b1;  // the lane's end along the last axis
-  const T sg[3] = {b0 ? T(-1) : T(1), b1 ? T(-1) : T(1), b2 ? T(-1) : T(1)};
   const double sd[3] = {b0 ? -1.0 : 1.0, b1 ? -1.0 : 1.0, b2 ? -1.0 : 1.0};
   constexpr double G2 = 0.28867513459481288225;  // 1 / (2 sqrt 3)
   const double S = (b0 ? G2 : 0.5) * (b1 ? G2 : 0.5) * (DIM > 2 ? (b2 ? G2 : 0.5) : 1.0);
@@ -3110,9 +3108,9 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
   double d1 = 0.0, d2 = 0.0;
   const int chunks = OP == 8 && full ? BC : 1;
   for (int ch = 0; ch < chunks; ++ch) {
-    T carry[PER];
+    double carry[PER];
 #pragma unroll
-    for (int p = 0; p < PER; ++p) carry[p] = T(0);
+    for (int p = 0; p < PER; ++p) carry[p] = 0.0;
     for (int s = 0; s <= TM; ++s) {
       const int k = vm0 + s;
       if (k > nm) break;  // no vertex at or above this layer (uniform)
@@ -3127,10 +3125,10 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
       double u[BC];
 #pragma unroll
       for (int i = 0; i < BC; ++i) u[i] = slot >= 0 ? x[(size_t)slot * DCG_B + i] : 0.0;
-      T vh[BC];
+      double vh[BC];
       if constexpr (OP == 4)
 #pragma unroll
-        for (int i = 0; i < BC; ++i) vh[i] = slot >= 0 ? v[(size_t)slot * DCG_B + i] : T(0);
+        for (int i = 0; i < BC; ++i) vh[i] = slot >= 0 ? (double)v[(size_t)slot * DCG_B + i] : 0.0;
 %CORNER_OP_DIRECTION%      double uh[OP == 1 ? BC : 1];
       butterfly(u, sd);
 #pragma unroll
@@ -3146,42 +3144,42 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
       for (int i = 0; i < BC; ++i) g[i][0] = g[i][1] = g[i][2] = 0.0;
       if constexpr (OP == 1) qp(0, u, g, px, py, pz, t, cm, ca, rs, rf, nullptr, nullptr, nullptr, prm, nullptr);
       else qp(0, u, g, px, py, pz, t, cm, ca, rs, rf, mc, nullptr, nullptr, prm, nullptr);
-      T o[BC];
+      double o[BC];
       if constexpr (OP == 1) {
 #pragma unroll
         for (int i = 0; i < BC; ++i) o[i] = rs[i];
-        butterfly(o, sg);
+        butterfly(o, sd);
 #pragma unroll
         for (int i = 0; i < BC; ++i) o[i] *= S;
 #pragma unroll
         for (int n = 0; n < NEP; ++n) o[EPI[n]] += ca * dp[n] * (kap[EPK[n]] * uh[EPJ[n]]);
-        butterfly(o, sg);
+        butterfly(o, sd);
       } else if constexpr (OP == 4 || OP == 5) {
-        butterfly(vh, sg);
-        T q[BC];
+        butterfly(vh, sd);
+        double q[BC];
 #pragma unroll
-        for (int i = 0; i < BC; ++i) q[i] = T(S) * vh[i];
-        butterfly(q, sg);
+        for (int i = 0; i < BC; ++i) q[i] = S * vh[i];
+        butterfly(q, sd);
         point_block(mc, q, o);
-        butterfly(o, sg);
+        butterfly(o, sd);
 #pragma unroll
-        for (int i = 0; i < BC; ++i) o[i] *= T(S);
+        for (int i = 0; i < BC; ++i) o[i] *= S;
 #pragma unroll
-        for (int n = 0; n < NEP; ++n) o[EPI[n]] += T(ca * dp[n] * kap[EPK[n]]) * vh[EPJ[n]];
-        butterfly(o, sg);
+        for (int n = 0; n < NEP; ++n) o[EPI[n]] += ca * dp[n] * kap[EPK[n]] * vh[EPJ[n]];
+        butterfly(o, sd);
       } else {
         // entries (j, j), or row ch of the block; the squared basis functions
         // have weights 1/3 and 1/(2 sqrt 3) in sums and differences
 #pragma unroll
-        for (int j = 0; j < BC; ++j) o[j] = T(0);
+        for (int j = 0; j < BC; ++j) o[j] = 0.0;
 #pragma unroll
         for (int n = 0; n < NMC; ++n)
           if (full ? MCI[n] == ch : MCI[n] == MCJ[n]) o[MCJ[n]] += mc[n];
-        butterfly(o, sg);
+        butterfly(o, sd);
         const double S2 = (b0 ? G2 : 1.0 / 3.0) * (b1 ? G2 : 1.0 / 3.0) * (DIM > 2 ? (b2 ? G2 : 1.0 / 3.0) : 1.0);
 #pragma unroll
         for (int j = 0; j < BC; ++j) o[j] *= S2;
-        butterfly(o, sg);
+        butterfly(o, sd);
         double kd[4];
         kd[0] = KH[1] * (DIM > 2 ? KH[2] / 3.0 : 1.0) / (3.0 * KH[0]);
         kd[1] = KH[0] * (DIM > 2 ? KH[2] / 3.0 : 1.0) / (3.0 * KH[1]);
@@ -3196,7 +3194,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
           if (full ? EPI[n] == ch : EPI[n] == EPJ[n]) o[EPJ[n]] += ca * dp[n] * kd[EPK[n]];
       }
 #pragma unroll
-      for (int i = 0; i < BC; ++i) out[i * NT + tid] = on ? o[i] : T(0);
+      for (int i = 0; i < BC; ++i) out[i * NT + tid] = on ? o[i] : 0.0;
       __syncthreads();
 #pragma unroll
       for (int p = 0; p < PER; ++p) {
@@ -3204,7 +3202,7 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
         const int rx = row % TX, ry = row / TX;
         const int wx = vi0 + 1 + rx, wy = DIM > 2 ? vj0 + 1 + ry : 0;
         if (row >= TL::ROWS || wx > n0 || wy > (DIM > 2 ? n1 : 0)) continue;
-        T low = T(0), up = T(0);
+        double low = 0.0, up = 0.0;
         if (i < BC) {
 #pragma unroll
           for (int ey = 0; ey < (DIM > 2 ? 2 : 1); ++ey)
@@ -3212,12 +3210,12 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
             for (int ex = 0; ex < 2; ++ex) {
               const int c = (rx + ex) + CX * (ry + ey);
               const int e = (1 - ex) | (DIM > 2 ? (1 - ey) << 1 : 0);  // the vertex's corner, lower layer end
-              const T* oc = out + i * NT + c * NCORNER;
+              const double* oc = out + i * NT + c * NCORNER;
               low += oc[e];
               up += oc[DIM > 2 ? e ^ 7 : e | 2];
             }
         }
-        const T sum = carry[p] + low;
+        const double sum = carry[p] + low;
         carry[p] = up;
         if (s == 0) continue;  // the layer below the tile's rows
         const int vid = wx + (DIM > 2 ? (n0 + 1) * wy : 0) + vstep * k;
@@ -3227,19 +3225,19 @@ __device__ __forceinline__ void corner_body(int tile, dcg_gp<const int> __restri
         if constexpr (OP == 8) {
           auto blk = y + (size_t)sr * (DCG_B * DCG_B);
           if (full) {
-            if (i < BC) blk[ch * DCG_B + i] = sum;
+            if (i < BC) blk[ch * DCG_B + i] = T(sum);
             else blk[ch * DCG_B + i] = T(0);
             if (ch == 0 && i >= BC)
               for (int j = 0; j < DCG_B; ++j) blk[i * DCG_B + j] = i == j ? T(1) : T(0);
           } else {
-            for (int j = 0; j < DCG_B; ++j) blk[i * DCG_B + j] = i == j ? (i < BC ? sum : T(1)) : T(0);
+            for (int j = 0; j < DCG_B; ++j) blk[i * DCG_B + j] = i == j ? (i < BC ? T(sum) : T(1)) : T(0);
           }
           if (ch == 0) lin[at] = x[at];
         } else if constexpr (OP == 1) {
-          const T b = v ? v[at] : T(0);  // the vector passed as v is the base
-          y[at] = b + (i < BC ? sum : T(0));
+          const double b = v ? (double)v[at] : 0.0;  // the vector passed as v is the base
+          y[at] = T(b + (i < BC ? sum : 0.0));
 %CORNER_OP_ROW%        } else {
-          const T acc = i < BC ? sum : v[at];  // padding species: identity rows
+          const T acc = i < BC ? T(sum) : v[at];  // padding species: identity rows
           y[at] = acc;
           if (part) {
             d1 += (double)acc * (double)(w1 == y ? acc : w1[at]);
@@ -3316,16 +3314,18 @@ const char* kCornerOpBegin = R"(  __shared__ double red5[OP == 5 ? 3 * (NT / 64)
   double e0 = 0.0, e1 = 0.0, e2 = 0.0;
 )";
 const char* kCornerOpDirection = R"(      if constexpr (OP == 5) {
-        T q[BC];
+        T q[BC], h[BC];
 #pragma unroll
-        for (int i = 0; i < BC; ++i) vh[i] = q[i] = slot >= 0 ? kdir((size_t)slot * DCG_B + i) : T(0);
-        if (slot >= 0 && kmode) precondition(op->jac, op->dinv, slot, q, vh);
+        for (int i = 0; i < BC; ++i) h[i] = q[i] = slot >= 0 ? kdir((size_t)slot * DCG_B + i) : T(0);
+        if (slot >= 0 && kmode) precondition(op->jac, op->dinv, slot, q, h);
+#pragma unroll
+        for (int i = 0; i < BC; ++i) vh[i] = (double)h[i];
       }
 )";
 const char* kCornerOpRow = R"(        } else if constexpr (OP == 5) {
           const T q = kdir(at);
           // padding species: identity rows (their directions are zero in a solve)
-          const T acc = i < BC ? sum : kmode ? T(0) : q;
+          const T acc = i < BC ? T(sum) : kmode ? T(0) : q;
           y[at] = acc;
           if (kmode == 1) {
             ((dcg_gp<T>)(T*)op->d)[at] = i < BC ? q : T(0);

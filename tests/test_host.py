@@ -294,6 +294,18 @@ def test_large_block_kernel_source_compiles(dca, wl):
     assert rc == 0, log
 
 
+def test_corner_form_sums_in_64_bits(dca, wl):
+    """Blocks of more than 4 species on box cells: the FP32 apply reads and stores FP32 vectors, but a row's terms are
+    summed in FP64, as the SpMV on the FP32 matrix sums them."""
+    m = dca.Model(wl.random_request(18, precision="mixed", side3=(5, 6)).ini, "", -1)
+    src = m.generated_source()
+    m.close()
+    body = src[src.index("void corner_body("):src.index("DCG_EVAL_ENTRY(dcg_tile_0_e0")]
+    for sums in (r"out\[", r"carry\[", r"vh\[BC\]", r"o\[BC\]", r"low\b", r"sum\b"):
+        decl = re.findall(r"\b(double|T|float) " + sums, body)
+        assert decl and set(decl) == {"double"}, sums
+
+
 def test_coloured_kernel_source_compiles(dca):
     """A model with advection needs the coloured kernel; it is generated and compiles."""
     ini = """[grid]
