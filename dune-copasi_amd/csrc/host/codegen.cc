@@ -3636,8 +3636,7 @@ bool corner_eligible(const ModelSpec& m, const Grid& g, int comp) {
 // 50 FP64 instructions per point, halo cells counted; a third of that is the
 // line, since small meshes read the stored ones from cache and the FP32
 // apply reads 4 bytes.
-bool eval_eligible(const ModelSpec& m, const Grid& g, int comp) {
-  if (m.comp_species[comp].empty() || m.comp_species[comp].size() > 4 || !box_form(m, g, comp)) return false;
+static int jacobian_cost(const ModelSpec& m, int comp) {
   int cost = 0;
   for (int s : m.comp_species[comp]) {
     const auto& sp = m.species[s];
@@ -3645,7 +3644,56 @@ bool eval_eligible(const ModelSpec& m, const Grid& g, int comp) {
     for (const auto& pj : sp.storage_jac) cost += expr::cost(pj.e) + 1;
     for (const auto& pj : sp.reaction_jac) cost += expr::cost(pj.e) + 1;
   }
-  return cost <= 16 * static_cast<int>(mc_pattern(m, comp).size());
+  return cost;
+}
+bool eval_eligible(const ModelSpec& m, const Grid& g, int comp) {
+  if (m.comp_species[comp].empty() || m.comp_species[comp].size() > 4 || !box_form(m, g, comp)) return false;
+  return jacobian_cost(m, comp) <= 16 * static_cast<int>(mc_pattern(m, comp).size());
+}
+
+// The lines were measured as times of Newton steps, the evaluated form against
+// the matrix (auto) and the stored coefficients (chosen), with 5 to 8 species,
+// kinetics of 30 to 2,600 instructions per point (mass action, Michaelis-
+// Menten, exponentials, Hill terms) and meshes of 16^2 to 400^2 and 6^3 to
+// 40^3 cells.  Gains (time of the other form over the evaluated one's):
+//   - interface and outflow terms: the facet rows hold a facet's whole
+//     Jacobian per lane, 0.2 to 0.8 of the matrix' speed at 10^3 to 28^3 and
+//     at 32^2 and 100^2; against stored coefficients, which launch six facet
+//     kernels per apply, 2 to 3.5 in 3D and 0.6 to 1 in 2D.
+//   - kinetics of more than 20 instructions per block entry (Hill terms):
+//     bound by their evaluation while the matrix streams from the last-level
+//     cache: 2D 0.6 to 0.9 below 256 MB of matrix, 1.3 to 2.2 above in FP64
+//     (mixed 1.0 at 350 MB); 3D 0.5 to 0.8 below 60 MB, 1.0 to 2.3 above 100.
+//   - lighter kinetics: a small mesh's launch takes the time of one lane's
+//     chain, its kinetics and about 60 instructions per species.  Up to 480
+//     (6 species of mass action) 0.95 to 1.3 on the smallest meshes against
+//     the matrix; above, 0.8 to 1 below the vertices stated here and 1 to 4.2
+//     past them (8 species, mixed: 2D 1.0 at 64^2, 1.3 at 256^2; 3D 0.9 at
+//     14^3, 1.1 at 20^3, 2.6 at 36^3).
+//   - chosen storage: in 2D the stored coefficients are the faster form, 0.7
+//     to 1 with mass action and 0.4 to 0.6 with Hill terms (8 species in FP64
+//     alone: 1.3 at 300^2); in 3D 0.7 to 0.9 at 14^3 and 1.3 to 6.9 at 40^3.
+//   - members of a batch share their launches; 8 of them move the lines to
+//     about an eighth of the mesh (Hill terms, 8 species, mixed: 2D 0.8 at
+//     128^2, 1.1 at 200^2; 3D 0.7 at 10^3, 1.2 at 16^3).
+bool corner_pays(const ModelSpec& m, const Layout& L, bool mixed, bool member, bool chosen) {
+  const int dim = L.grid.dim;
+  int cost = 0;
+  double rows = 0.0;
+  for (size_t c = 0; c < L.comps.size(); ++c) {
+    if (!L.comps[c].b) continue;
+    cost = std::max(cost, jacobian_cost(m, static_cast<int>(c)));
+    rows += L.comps[c].nslot;
+  }
+  if (!L.facets.empty()) return chosen && dim == 3;
+  if (chosen && dim == 2) return false;
+  if (member) rows *= 8.0;
+  if (cost > 20 * L.B * L.B)
+    return rows * (dim == 3 ? 27 : 9) * L.B * L.B * (mixed ? 4 : 8) >= (dim == 3 ? 100e6 : 256e6);
+  const double chain = cost + 60.0 * L.B;
+  if (chosen) return rows >= (mixed ? 30.0 : 15.0) * chain;
+  if (chain <= 480.0) return true;
+  return dim == 3 ? rows >= (mixed ? 7.0 : 1.2) * chain : rows >= (mixed ? 60.0 : 2.0) * (chain - 480.0);
 }
 
 std::vector<std::array<int, 3>> apply_tile_candidates(const Grid& g, int species, std::array<int, 3> setup_tile,
@@ -4007,7 +4055,8 @@ std::string gen_tiled(const ModelSpec& m, const Grid& g, int comp, const std::st
   return o.str() + body;
 }
 
-GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool runtime_geometry, bool points) {
+GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool runtime_geometry, bool points,
+                                  bool evaluate) {
   GeneratedSource out;
   const bool geo = runtime_geometry;
   std::string pre = kPrelude;
@@ -4026,7 +4075,7 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
   std::ostringstream src;
   src << pre;
   const bool numerical = spec.jacobian == JacobianType::Numerical && !spec.is_linear;
-  const bool all_eval = evaluates(spec, L);
+  const bool all_eval = evaluate;
   for (size_t c = 0; c < spec.comp_names.size(); ++c) {
     if (spec.comp_species[c].empty()) {
       out.volume_kernel.push_back("");
@@ -4052,7 +4101,9 @@ GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& L, bool r
       std::string tk = "dcg_tile_" + std::to_string(c);
       std::vector<int> waves, threads;
       const int nsp = static_cast<int>(spec.comp_species[c].size());
-      const bool corner = corner_eligible(spec, L.grid, static_cast<int>(c)) && (!points || all_eval);
+      // (2D models on the matrix keep the tiled residual: the corner form's is 0.98 to 1.05 of its speed with mass
+      // action at 20^2 and 100^2 and 0.86 to 0.97 with Hill terms; 40^3 with 7 species: 360 -> 28 us)
+      const bool corner = corner_eligible(spec, L.grid, static_cast<int>(c)) && (points ? all_eval : L.grid.dim == 3);
       const bool eval = points && all_eval;
       std::vector<std::array<int, 3>> shapes;
       if (points && corner) {

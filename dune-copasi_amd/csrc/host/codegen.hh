@@ -80,11 +80,15 @@ std::vector<std::array<int, 3>> corner_tiles(int dim);
 // fit one launch: point storage then evaluates everywhere (all or nothing, as
 // the fused operator launches take the place of the whole iteration)
 bool evaluates(const ModelSpec& m, const Layout& L);
+// with a block of more than 4 species: whether that is the faster form for
+// this mesh and these kinetics (mixed: FP32 operator; member: of a batch;
+// chosen: against stored point coefficients, else against the matrix)
+bool corner_pays(const ModelSpec& m, const Layout& L, bool mixed, bool member, bool chosen);
 
 // points: also emit the point-coefficient Jacobian entry points (_q, _p, _pf)
-// of every tiled compartment
+// of every tiled compartment; evaluate: in the evaluated forms
 GeneratedSource generate_assembly(const ModelSpec& spec, const Layout& layout, bool runtime_geometry = false,
-                                  bool points = false);
+                                  bool points = false, bool evaluate = false);
 
 // Geometry words of unstructured cells, in the order of `cells`, as the
 // generated cell kernels read them: the gradients of the element's basis

@@ -190,7 +190,7 @@ void Model::build(const std::string& ini, const std::string& overrides) {
   // keeps only the coefficient blocks of every cell's quadrature points and
   // applies them (with the uniform diffusion) to each Krylov direction, which
   // is the same operator in fewer bytes; "auto" takes points on box grids
-  // with blocks of up to 4 species where the model allows it.  Points need
+  // where the model allows it and they are the faster form.  Points need
   // compartments on the tiled kernel and a preconditioner built from diagonal
   // blocks (Jacobi, vertex-block Jacobi or none); interface and outflow terms
   // are applied from the linearisation point by the facet kernels.
@@ -207,13 +207,14 @@ void Model::build(const std::string& ini, const std::string& overrides) {
     else if (cfg_.precond == Preconditioner::ILU0) why = "an ILU0 preconditioner";
     else if (!all_tile_eligible()) why = "compartments outside the tiled kernel";
     if (st == "points" && !why.empty()) throw NotImplemented("linear_solver.storage = points with " + why);
-    // auto: box cells, with blocks of up to 4 species or evaluated
-    // coefficients (40^3, 7 species, FP32 operator: apply 27 us against 83 us
-    // for the SpMV, and no Jacobian pass of 3.3 ms; larger blocks outside the
-    // corner form keep their corner sums in LDS, where the SpMV is faster)
+    // auto: box cells, with blocks of up to 4 species or with larger ones that
+    // gain from evaluated coefficients (corner_pays); else larger blocks keep
+    // their corner sums in LDS, where the SpMV is faster
     int bmax = 0;
     for (const auto& C : L_.comps) bmax = std::max(bmax, C.b);
-    const bool suits = L_.grid.cube && (bmax <= 4 || evaluates(spec_, L_));
+    cfg_.evaluate = evaluates(spec_, L_) && (bmax <= 4 || corner_pays(spec_, L_, cfg_.precision == Precision::Mixed,
+                                                                      opt_.batch_member, st == "points"));
+    const bool suits = L_.grid.cube && (bmax <= 4 || cfg_.evaluate);
     cfg_.points = why.empty() && (st == "points" || (st == "auto" && suits));
   }
   {
@@ -254,7 +255,7 @@ void Model::build(const std::string& ini, const std::string& overrides) {
   time_ = c.get(p + "time_begin", 0.0);
   t_end_ = c.get(p + "time_end", 1.0);
   dt_initial_ = c.get(p + "time_step_initial", c.get(p + "time_step_max", 0.1));
-  gen_ = generate_assembly(spec_, L_, opt_.runtime_parameters, cfg_.points);
+  gen_ = generate_assembly(spec_, L_, opt_.runtime_parameters, cfg_.points, cfg_.evaluate);
 }
 
 bool Model::all_tile_eligible() const {

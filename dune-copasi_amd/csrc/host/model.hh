@@ -65,6 +65,7 @@ struct SolverConfig {
   // linear_solver.storage: the Jacobian as point coefficients per cell (the
   // BiCGSTAB operator applies them) instead of an assembled BCSR matrix
   bool points = false;
+  bool evaluate = false;  // the coefficients are evaluated in the operator, not stored
   // linear_solver.readback_iterations: BiCGSTAB iterations launched between
   // read-backs of its scalars (0: as many as the same solve took in the last
   // time step, then 4); 1 launches none past convergence (for profilers)

@@ -76,6 +76,31 @@ def test_residual_and_apply(dca, dim, cells, species):
     orc.close()
 
 
+@pytest.mark.parametrize("dim,cells,species", [(d, c, b) for d, c in SHAPES for b in (5, 6)] +
+                         [(2, (30, 31), 8), (2, (70, 33), 8), (3, (15, 4, 9), 8)])
+def test_default_storage(dca, dim, cells, species):
+    """The same on the storage that a model takes by itself, which is the evaluated form at these sizes."""
+    print(f"case: corner form by default {dim}D {cells} {species} species", flush=True)
+    ini = _ini(dim, cells, species, extensions=(1.0, 0.6, 1.7))
+    orc = OracleModel(ini)
+    rng = np.random.default_rng(species)
+    x = v = None
+    for tile in ("0", "1"):
+        gpu = dca.Model(ini, f"model.time_step_operator.linear_solver.point_tile = {tile}\n", 0)
+        assert "dcg_tile_0_e0" in gpu.generated_source()
+        if x is None:
+            x, v = 0.5 + 0.2 * rng.random(gpu.n_dof), rng.standard_normal(gpu.n_dof)
+        for cm, ca in ((1.0, 0.0), (0.0, 0.7), (1.0, 0.3)):
+            ro, vals = orc.assemble(x, 0.4, cm, ca)
+            r, _ = gpu.assemble(x, 0.4, cm, ca, jacobian=False)
+            assert np.abs(r - ro).max() <= 1e-12 * np.abs(ro).max()
+            ref = orc.csr(vals) @ v
+            y = gpu.jacobian_apply(x, 0.4, cm, ca, v)
+            assert np.abs(y - ref).max() <= 1e-12 * np.abs(ref).max()
+        gpu.close()
+    orc.close()
+
+
 @pytest.mark.parametrize("runtime", [False, True])
 @pytest.mark.parametrize("precond", ["Jacobi", "VertexBlockJacobi"])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])

@@ -297,13 +297,69 @@ def test_large_block_kernel_source_compiles(dca, wl):
 def test_corner_form_sums_in_64_bits(dca, wl):
     """Blocks of more than 4 species on box cells: the FP32 apply reads and stores FP32 vectors, but a row's terms are
     summed in FP64, as the SpMV on the FP32 matrix sums them."""
-    m = dca.Model(wl.random_request(18, precision="mixed", side3=(5, 6)).ini, "", -1)
+    m = dca.Model(wl.random_request(18, precision="mixed", side3=(32, 33)).ini, "", -1)
     src = m.generated_source()
     m.close()
     body = src[src.index("void corner_body("):src.index("DCG_EVAL_ENTRY(dcg_tile_0_e0")]
     for sums in (r"out\[", r"carry\[", r"vh\[BC\]", r"o\[BC\]", r"low\b", r"sum\b"):
         decl = re.findall(r"\b(double|T|float) " + sums, body)
         assert decl and set(decl) == {"double"}, sums
+
+
+_KINETICS = {  # per species: reaction by its neighbour, and its Jacobian entry
+    "mass": ("0.9*{b}*{b} - 0.7*{a}*{b}", "-0.7*{b}", "1.8*{b} - 0.7*{a}"),
+    "hill": ("{b}^2.5/(0.4+{b}^2.5) - 0.3*{a}", "-0.3",
+             "2.5*{b}^1.5/(0.4+{b}^2.5) - 2.5*{b}^2.5*{b}^1.5/((0.4+{b}^2.5)*(0.4+{b}^2.5))"),
+}
+
+
+def _chain_ini(dim, n, species, kinetics, inner=0):
+    """`species` species in a chain; `inner` more of them in the half x < 0.5, with a flux of the first ones."""
+    comps = "domain.expression = 1" if not inner else "domain.expression = position_x >= 0.5\n" \
+        "core.expression = position_x < 0.5"
+    out = [f"[grid]\ndimension = {dim}\ncells = {' '.join([str(n)] * dim)}\nextensions = {' '.join(['1'] * dim)}\n"
+           f"cell_type = cube\n[compartments]\n{comps}"]
+    for comp, tag, m in (("domain", "s", species), ("core", "c", inner)):
+        for i in range(m):
+            a, b = f"{tag}{i}", f"{tag}{(i + 1) % m}"
+            r, ja, jb = (e.format(a=a, b=b) for e in _KINETICS[kinetics])
+            out.append(f"[model.scalar_field.{a}]\ncompartment = {comp}\nstorage.expression = 1\n"
+                       f"cross_diffusion.{a}.expression = 0.01\nreaction.expression = {r}\n"
+                       f"reaction.jacobian.{a}.expression = {ja}\nreaction.jacobian.{b}.expression = {jb}")
+            if i == 0 and inner:
+                other, s = ("core", "") if comp == "domain" else ("domain", "-")
+                out.append(f"outflow.{other}.expression = {s}0.3*(s0 - c0)\noutflow.{other}.jacobian.s0.expression = "
+                           f"{s}0.3\noutflow.{other}.jacobian.c0.expression = {'' if s else '-'}0.3")
+    return "\n".join(out) + "\n[model.time_step_operator]\ntype = ImplicitEuler\nlinear_solver.type = BiCGSTAB\n" \
+        "linear_solver.preconditioner.type = Jacobi\n"
+
+
+@pytest.mark.parametrize("dim,n,species,inner,kinetics,precision,storage,form", [
+    # auto: evaluated coefficients against the matrix
+    (2, 16, 6, 0, "mass", "mixed", "auto", "evaluated"), (3, 6, 6, 0, "mass", "mixed", "auto", "evaluated"),
+    (2, 48, 8, 0, "mass", "mixed", "auto", "matrix"), (2, 48, 8, 0, "mass", "fp64", "auto", "evaluated"),
+    (2, 100, 8, 0, "mass", "mixed", "auto", "evaluated"), (3, 14, 8, 0, "mass", "mixed", "auto", "matrix"),
+    (3, 14, 8, 0, "mass", "fp64", "auto", "evaluated"), (3, 20, 8, 0, "mass", "mixed", "auto", "evaluated"),
+    (2, 128, 8, 0, "hill", "fp64", "auto", "matrix"), (2, 256, 8, 0, "hill", "fp64", "auto", "evaluated"),
+    (2, 256, 8, 0, "hill", "mixed", "auto", "matrix"), (3, 14, 6, 0, "hill", "mixed", "auto", "matrix"),
+    (3, 40, 6, 0, "hill", "mixed", "auto", "evaluated"),
+    # interface terms
+    (2, 32, 5, 5, "mass", "fp64", "auto", "matrix"), (3, 16, 6, 2, "mass", "mixed", "auto", "matrix"),
+    (3, 16, 4, 4, "mass", "mixed", "auto", "evaluated"),
+    # points asked for: evaluated against stored coefficients
+    (2, 64, 8, 0, "mass", "mixed", "points", "stored"), (2, 64, 5, 5, "mass", "fp64", "points", "stored"),
+    (3, 10, 6, 0, "mass", "fp64", "points", "stored"), (3, 10, 6, 0, "hill", "fp64", "points", "stored"),
+    (3, 32, 6, 0, "mass", "mixed", "points", "evaluated"),
+    (3, 10, 5, 5, "hill", "fp64", "points", "evaluated")])
+def test_storage_above_four_species(dca, dim, n, species, inner, kinetics, precision, storage, form):
+    """Blocks of more than 4 species take the evaluated form where it is the faster one (corner_pays)."""
+    p = "model.time_step_operator.linear_solver."
+    m = dca.Model(_chain_ini(dim, n, species, kinetics, inner), f"{p}storage = {storage}\n{p}precision = {precision}\n",
+                  -1)
+    src = m.generated_source()
+    m.close()
+    got = "evaluated" if "dcg_tile_0_e0" in src else "stored" if "dcg_tile_0_p0" in src else "matrix"
+    assert got == form
 
 
 def test_coloured_kernel_source_compiles(dca):
