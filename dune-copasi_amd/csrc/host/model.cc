@@ -614,8 +614,12 @@ void Model::setup_device() {
     lo_lev_.upload(lo_ptr_, stream_);
     up_lev_.upload(up_ptr_, stream_);
     ilu_stencil_ = build_ilu_stencil(rows, rows_u);
-    if (ilu_sweep_ && !ilu_stencil_) build_ilu_sweep_tables(rows, rows_u);
-    lu_.resize(static_cast<size_t>(matrix_values()));
+    // (beside the stencil form the sweeps serve the allocation-free solve
+    // alone, where only their buffers fit its work space)
+    ilu_sweep_ = ilu_sweep_ && (!ilu_stencil_ || (cfg_.precision == Precision::FP64 && !noalloc_fits(true) &&
+                                                  noalloc_fits(false)));
+    if (ilu_sweep_) build_ilu_sweep_tables(rows, rows_u);
+    if (!ilu_stencil_) lu_.resize(static_cast<size_t>(matrix_values()));
   }
   {
     // geometry words (spacing, reciprocals, cell measure) + parameters
@@ -1131,7 +1135,8 @@ void Model::ensure_matrix() {
   val_.resize(static_cast<size_t>(matrix_values()));
   if (cfg_.precision == Precision::Mixed) val32_.resize(static_cast<size_t>(matrix_values()));
   if (!dinv_.size()) dinv_.resize(static_cast<size_t>(L_.nslot) * L_.B * L_.B);
-  if (cfg_.precond == Preconditioner::ILU0 && !lu_.size()) lu_.resize(static_cast<size_t>(matrix_values()));
+  if (cfg_.precond == Preconditioner::ILU0 && !ilu_stencil_ && !lu_.size())
+    lu_.resize(static_cast<size_t>(matrix_values()));
   plan32_ = plan_;
 }
 
@@ -1154,6 +1159,9 @@ Model::KrylovWork Model::own_work() {
   w.val = val_.get();
   w.dinv = dinv_.get();
   w.lu = lu_.get();
+  w.st_pack = st_pack_.get();
+  w.st_lower = st_lower_.get();
+  w.st_upper = st_upper_.get();
   w.status = status_.get();
   return w;
 }
@@ -1472,7 +1480,7 @@ bool Model::build_ilu_stencil(const std::vector<int>& lrows, const std::vector<i
       lds = std::max(lds, std::min(v, 160 * 1024));
   }
   if (!k::ilu_stencil_fits(t, L_.B, static_cast<size_t>(lds))) return false;
-  const int LW = k::ilu_stencil_lower_words(L_.B), UW = k::ilu_stencil_upper_words(L_.B);
+  const int UW = k::ilu_stencil_upper_words(L_.B);
   if (ns * UW > 0x7fffffffL) return false;
   const int zero = t.ring * t.width;
   std::vector<int4> frow(ns);
@@ -1516,12 +1524,11 @@ bool Model::build_ilu_stencil(const std::vector<int>& lrows, const std::vector<i
   st_lsrc_.upload(lsrc, stream_);
   st_usrc_.upload(usrc, stream_);
   st_upos_.upload(up, stream_);
-  const size_t N = static_cast<size_t>(ns);
-  st_pack_.resize(N * (2 * NP + 1) * L_.B * L_.B);
-  st_lower_.resize(N * LW * 2);
-  st_upper_.resize(N * UW * 2);
-  k::fill(st_lower_.get(), 0.0, static_cast<long>(N) * LW * 2, stream_);
-  k::fill(st_upper_.get(), 0.0, static_cast<long>(N) * UW * 2, stream_);
+  st_pack_.resize(stencil_words(0));
+  st_lower_.resize(stencil_words(1));
+  st_upper_.resize(stencil_words(2));
+  k::fill(st_lower_.get(), 0.0, static_cast<long>(st_lower_.size()), stream_);
+  k::fill(st_upper_.get(), 0.0, static_cast<long>(st_upper_.size()), stream_);
   t.frow = st_frow_.get();
   t.first = st_first_.get();
   t.lo_src = st_lsrc_.get();
@@ -1541,8 +1548,8 @@ void Model::precond_setup(const KrylovWork& w) {
   } else if (jacobi_kind()) {
     k::block_inverse(B, ns, w.val, diag_pos_.get(), w.dinv, w.status, cfg_.precond == Preconditioner::Jacobi, stream_);
   } else if (cfg_.precond == Preconditioner::ILU0) {
-    if (ilu_stencil_) {
-      k::ilu_stencil_factor(B, ilu_st_, w.val, st_pack_.get(), st_lower_.get(), st_upper_.get(), w.status, stream_);
+    if (w.st_pack) {
+      k::ilu_stencil_factor(B, ilu_st_, w.val, w.st_pack, w.st_lower, w.st_upper, w.status, stream_);
       return;
     }
     DCG_HIP(hipMemcpyAsync(w.lu, w.val, matrix_values() * sizeof(double), hipMemcpyDeviceToDevice, stream_));
@@ -1577,8 +1584,8 @@ int Model::bicgstab64(const double* b, double* x, double rtol, double abstol, in
   const bool point_jacobi = cfg_.precond == Preconditioner::Jacobi;
   const bool ilu = cfg_.precond == Preconditioner::ILU0;
   auto apply_ilu = [&](const double* in, double* out) {
-    if (ilu_stencil_) {
-      k::ilu_stencil_apply<double>(B, ilu_st_, st_lower_.get(), st_upper_.get(), in, tmp, out, sc, stream_);
+    if (w.st_pack) {
+      k::ilu_stencil_apply<double>(B, ilu_st_, w.st_lower, w.st_upper, in, tmp, out, sc, stream_);
       return;
     }
     if (ilu_sweep_) {
@@ -2335,6 +2342,33 @@ int Model::linear_solve(const double* jac, const double* b_packed, double* x_pac
   return rc;
 }
 
+size_t Model::stencil_words(int which) const {
+  const size_t n = static_cast<size_t>(L_.nslot);
+  if (which == 0) return n * (2 * k::kIluPlaces + 1) * L_.B * L_.B;
+  return n * 2 * static_cast<size_t>(which == 1 ? k::ilu_stencil_lower_words(L_.B) : k::ilu_stencil_upper_words(L_.B));
+}
+
+// every region of the fixed work space starts on 256 bytes
+static size_t noalloc_round(size_t words) { return (words + 31) / 32 * 32; }
+static constexpr size_t kNoallocScalarWords = (sizeof(k::BicgScalars) + sizeof(double) - 1) / sizeof(double);
+
+size_t Model::noalloc_words(bool stencil) const {
+  const size_t nv = static_cast<size_t>(L_.nslot) * L_.B;
+  size_t w = 11 * noalloc_round(nv) + noalloc_round(part_.size()) + noalloc_round(kNoallocScalarWords) +
+             noalloc_round(2);
+  if (stencil) {
+    for (int i = 0; i < 3; ++i) w += noalloc_round(stencil_words(i));
+    return w;
+  }
+  w += noalloc_round(nv * L_.B);
+  if (cfg_.precond == Preconditioner::ILU0) w += noalloc_round(static_cast<size_t>(matrix_values()));
+  return w;
+}
+
+bool Model::noalloc_fits(bool stencil) const {
+  return noalloc_words(stencil) <= k::kNoallocScratchBytes / sizeof(double);
+}
+
 // dcg_linear_solve without device allocations: J, b and x are the caller's
 // device buffers (BCSR values, packed state layout), every other buffer the
 // FP64 solve needs (Krylov vectors, the unpacked right-hand side and
@@ -2349,35 +2383,35 @@ int Model::linear_solve_noalloc(const double* jac, const double* b_packed, doubl
     throw NotImplemented("the allocation-free linear solve runs FP64 models only (linear_solver.precision = fp64)");
   if (!jac || !b_packed || !x_packed) throw Error("null device buffer");
   const size_t nv = static_cast<size_t>(L_.nslot) * L_.B;
-  const size_t align = 32;  // doubles: every region starts on 256 bytes
-  auto round = [&](size_t w) { return (w + align - 1) / align * align; };
   const bool ilu = cfg_.precond == Preconditioner::ILU0;
-  const size_t sc_words = round((sizeof(k::BicgScalars) + sizeof(double) - 1) / sizeof(double));
-  const size_t words = 11 * round(nv) + round(static_cast<size_t>(L_.nslot) * L_.B * L_.B) +
-                       (ilu ? round(static_cast<size_t>(matrix_values())) : 0) + round(part_.size()) + sc_words +
-                       round(2);
-  const size_t limit = k::kNoallocScratchBytes / sizeof(double);
-  if (words > limit)
-    throw Error("the allocation-free linear solve needs " + std::to_string(words * sizeof(double)) +
+  // ILU0's stencil form where its buffers fit, else the factors' in matrix order
+  const bool stencil = ilu_stencil_ && noalloc_fits(true);
+  if (!stencil && !noalloc_fits(false))
+    throw Error("the allocation-free linear solve needs " + std::to_string(noalloc_words(false) * sizeof(double)) +
                 " bytes of work space for this model; the fixed work space holds " +
                 std::to_string(k::kNoallocScratchBytes) + " bytes");
   double* base = k::noalloc_scratch(device_);
   size_t off = 0;
   auto take = [&](size_t w) {
     double* q = base + off;
-    off += round(w);
+    off += noalloc_round(w);
     return q;
   };
   KrylovWork w;
   for (auto& v : w.kv) v = take(nv);
   double* rhs = take(nv);
   double* sol = take(nv);
-  w.dinv = take(static_cast<size_t>(L_.nslot) * L_.B * L_.B);
-  w.lu = ilu ? take(static_cast<size_t>(matrix_values())) : nullptr;
+  if (stencil) {
+    w.st_pack = take(stencil_words(0));
+    w.st_lower = take(stencil_words(1));
+    w.st_upper = take(stencil_words(2));
+  } else {
+    w.dinv = take(nv * L_.B);
+    w.lu = ilu ? take(static_cast<size_t>(matrix_values())) : nullptr;
+  }
   w.part = take(part_.size());
   w.spart = w.part + spart_off_;
-  w.sc = reinterpret_cast<k::BicgScalars*>(base + off);
-  off += sc_words;
+  w.sc = reinterpret_cast<k::BicgScalars*>(take(kNoallocScalarWords));
   w.status = reinterpret_cast<int*>(take(2));
   w.val = jac;
   // the given matrix is the operator; the solve keeps no per-step hint

@@ -246,9 +246,15 @@ class Model {
     const double* val = nullptr;  // the assembled operator
     double* dinv = nullptr;
     double* lu = nullptr;
+    double *st_pack = nullptr, *st_lower = nullptr, *st_upper = nullptr;  // ILU0's stencil form (null: lu and dinv)
     int* status = nullptr;
   };
   KrylovWork own_work();
+  // doubles that linear_solve_noalloc takes of the fixed work space, with the
+  // stencil form's buffers or with lu and dinv, and whether they fit
+  size_t noalloc_words(bool stencil) const;
+  bool noalloc_fits(bool stencil) const;
+  size_t stencil_words(int which) const;  // 0: pack, 1: lower, 2: upper stream
   int bicgstab64(const double* b, double* x, double rtol, double abstol, int maxit, int* its, const KrylovWork& w);
   int bicgstab32(const double* b, float* x, double rtol, int maxit, int* its);
   // the same iteration on fused operator launches (every compartment

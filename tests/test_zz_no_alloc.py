@@ -101,3 +101,44 @@ def test_noalloc_solve_rejects_what_it_cannot_hold(dca, wl):
     rc, _, _, err = _solve_noalloc(dca, hip, mixed, J, np.zeros(mixed.n_dof), 1e-8, 10)
     assert rc < 0 and "fp64" in err
     mixed.close()
+
+
+def test_noalloc_ilu0_works_in_the_fixed_space(dca, wl):
+    """The factors of ILU0's stencil form (9 blocks per vertex in packed order, 9 in the solves' streams) lie in the
+    fixed work space beside the 11 work vectors: a marked array has lost its mark at as many words."""
+    print("case: no-alloc ILU0 in the work space", flush=True)
+    hip = _Hip()
+    lib = dca.load_library()
+    space = lib._ZN7dcopasi1k15noalloc_scratchEi  # dcopasi::k::noalloc_scratch(int)
+    space.restype, space.argtypes = ctypes.c_void_p, [ctypes.c_int]
+    w = _case(wl, 48, "ILU")
+    m = dca.Model(w.ini, "", 0)
+    _, J = m.assemble(w.initial_state(m), 0.0, 1.0, 1.0)
+    b = np.random.default_rng(5).standard_normal(m.n_dof)
+    x_ref, rc_ref, its_ref = m.linear_solve(J, b, rtol=1e-10, maxit=500)
+    words, mark = (64 << 20) // 8, 1.25e300
+    marked = np.full(words, mark)
+    base = space(0)
+    assert hip.L.hipMemcpy(ctypes.c_void_p(base), marked.ctypes.data, marked.nbytes, H2D) == 0
+    rc, x, its, err = _solve_noalloc(dca, hip, m, J, b, 1e-10, 500)
+    assert (rc, its) == (0, its_ref), err
+    assert np.array_equal(x, x_ref)
+    used = int((hip.to_host(ctypes.c_void_p(base), words) != mark).sum())
+    assert used >= 11 * m.n_dof + 18 * m.n_slots * m.block_size ** 2
+    m.close()
+
+
+def test_noalloc_ilu0_where_the_stencil_form_does_not_fit(dca, wl):
+    """331^2 vertices: the factors in matrix order fit the work space, the stencil form's buffers do not."""
+    print("case: no-alloc ILU0 on the sweeps", flush=True)
+    hip = _Hip()
+    w = _case(wl, 330, "ILU")
+    m = dca.Model(w.ini, "", 0)
+    _, J = m.assemble(w.initial_state(m), 0.0, 1.0, 1.0)
+    b = np.random.default_rng(6).standard_normal(m.n_dof)
+    x_ref, rc_ref, its_ref = m.linear_solve(J, b, rtol=1e-8, maxit=500)
+    rc, x, its, err = _solve_noalloc(dca, hip, m, J, b, 1e-8, 500)
+    assert (rc_ref, rc) == (0, 0), err
+    assert its == its_ref
+    assert np.abs(x - x_ref).max() <= 1e-12 * np.abs(x_ref).max()
+    m.close()
