@@ -2471,7 +2471,7 @@ size_t Model::device_bytes() const {
   for (const auto& c : comp_dev_)
     b += c.cells.bytes() + c.cell_slots.bytes() + c.cell_mask.bytes() + c.g2l.bytes() + c.tiles.bytes() +
          c.cell_mask_grid.bytes() + c.rtiles.bytes();
-  b += kpart_.bytes() + frow_slot_.bytes() + frow_ptr_.bytes() + frow_ent_.bytes();
+  b += kpart_.bytes() + frow_slot_.bytes() + frow_ptr_.bytes() + frow_ent_.bytes() + reduce_bytes();
   for (const auto& f : facet_dev_) b += f.fint.bytes() + f.fdbl.bytes();
   return b;
 }

@@ -293,6 +293,7 @@ class Model {
   std::vector<ReduceKey> reduce_keys(const std::string& reduce_ini) const;
   struct ReducePlan;
   ReducePlan& reduce_plan(const std::string& reduce_ini);
+  size_t reduce_bytes() const;  // device arrays of the kept plans
   std::vector<std::shared_ptr<ReducePlan>> reduce_plans_;  // the last few texts, the latest first
   double apply_bytes() const;
 

@@ -98,6 +98,15 @@ struct Model::ReducePlan {
   std::vector<DeviceArray<double>> rgeo;
 };
 
+size_t Model::reduce_bytes() const {
+  size_t b = 0;
+  for (const auto& p : reduce_plans_) {
+    b += p->part.bytes() + p->out.bytes();
+    for (const auto& g : p->rgeo) b += g.bytes();
+  }
+  return b;
+}
+
 Model::ReducePlan& Model::reduce_plan(const std::string& reduce_ini) {
   constexpr size_t kept = 4;
   for (size_t i = 0; i < reduce_plans_.size(); ++i)

@@ -50,3 +50,21 @@ def test_reduce_levels(dca, cells, split):
                    - 6.0 * (i + 1)) <= 1e-11
     assert abs(m.reduce(KEYS)["moment"] - 18.0) <= 1e-10
     m.close()
+
+
+def test_kept_plans_count_as_footprint(dca):
+    """A plan holds (value, defined) pairs per key: one per workgroup of 256 cells and one result."""
+    print("case: reduce plans in the footprint", flush=True)
+    m = dca.Model("[grid]\ndimension = 2\ncells = 100 100\nextensions = 1 1\ncell_type = cube\n[compartments]\n"
+                  "domain.expression = 1\n[model.scalar_field.u]\ncompartment = domain\nstorage.expression = 1\n"
+                  "cross_diffusion.u.expression = 0.1\ninitial.expression = position_x\n[model.time_step_operator]\n"
+                  "type = ImplicitEuler\n", "", 0)
+    m.set_state(m.initial_state(), 0.0)
+    before = m.device_bytes()
+    m.reduce(KEYS)
+    plan = 4 * 16 * (-(-100 * 100 // 256) + 1)
+    assert m.device_bytes() == before + plan
+    for i in range(6):  # four are kept
+        m.reduce(f"[v{i}]\nevaluation.expression = {i + 1}*integration_factor\n")
+    assert m.device_bytes() == before + 4 * plan // 4
+    m.close()
