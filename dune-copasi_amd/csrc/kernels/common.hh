@@ -4,8 +4,10 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <type_traits>
 
+#include "../host/error.hh"
 #include "kernels.hh"
 
 namespace dcopasi::k {
@@ -49,6 +51,21 @@ __device__ __forceinline__ int xcd_chunk(int bid, int nblocks) {
   const int per = (nblocks + 7) / 8;
   const int c = (bid % 8) * per + bid / 8;
   return c;
+}
+
+// Before a launch with more than 64 KiB of dynamic LDS: the kernel's limit on
+// the current device becomes the device's own, once per device (raised: a bit
+// per device; the same value whoever comes first, so threads that launch
+// different sizes do not lower each other's).
+inline void raise_lds(const void* kernel, size_t lds, std::atomic<unsigned long long>& raised) {
+  if (lds <= 64 * 1024) return;
+  int dev = 0, most = 0;
+  DCG_HIP(hipGetDevice(&dev));
+  const unsigned long long bit = 1ull << (dev & 63);
+  if (raised.load() & bit) return;
+  DCG_HIP(hipDeviceGetAttribute(&most, hipDeviceAttributeMaxSharedMemoryPerBlock, dev));
+  DCG_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, most));
+  raised.fetch_or(bit);
 }
 
 // ----------------------------------------------------------------- BiCGSTAB scalars

@@ -28,9 +28,6 @@
 // the ~300 FP64 instructions of a lane's row.
 #include <hip/hip_runtime.h>
 
-#include <atomic>
-
-#include "../host/error.hh"
 #include "common.hh"
 #include "kernels.hh"
 
@@ -441,22 +438,13 @@ bool ilu_stencil_fits(const IluStencil& t, int B, size_t lds) {
          ilu_stencil_factor_lds(t, B) <= lds && apply_lds(t, B, sizeof(double)) <= lds;
 }
 
-// dynamic LDS above 64 KiB: raise the kernel's limit first
-static void raise_lds(const void* f, size_t lds, std::atomic<size_t>& raised) {
-  if (lds <= raised.load()) return;
-  DCG_HIP(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-  size_t cur = raised.load();
-  while (lds > cur && !raised.compare_exchange_weak(cur, lds)) {
-  }
-}
-
 template <int B>
 static void factor_t(const IluStencil& t, const double* val, double* pack, double* ls, double* us, int* status,
                      hipStream_t s) {
   const long n = (long)t.nrows * NO;
   ilu_stencil_pack_k<B><<<(unsigned)((n + kThreads - 1) / kThreads), kThreads, 0, s>>>(t.nrows, t, val, pack);
   const size_t lds = ilu_stencil_factor_lds(t, B);
-  static std::atomic<size_t> raised{64 * 1024};
+  static std::atomic<unsigned long long> raised{0};
   raise_lds(reinterpret_cast<const void*>(&ilu_stencil_factor_k<B>), lds, raised);
   const int G = (t.width * B + kWave - 1) / kWave;
   ilu_stencil_factor_k<B><<<1, kIluBlock, lds, s>>>(t, G, pack, ls, us, status);
@@ -473,7 +461,7 @@ template <int B, typename V>
 static void apply_t(const IluStencil& t, const double* ls, const double* us, const V* in, V* tmp, V* out,
                     const BicgScalars* sc, hipStream_t s) {
   const size_t lds = apply_lds(t, B, sizeof(V));
-  static std::atomic<size_t> raised{64 * 1024};
+  static std::atomic<unsigned long long> raised{0};
   raise_lds(reinterpret_cast<const void*>(&ilu_stencil_apply_k<B, V>), lds, raised);
   const int G = (t.width + kWave - 1) / kWave;
   ilu_stencil_apply_k<B, V><<<1, kIluBlock, lds, s>>>(t, G, ls, us, in, tmp, out, sc);

@@ -1537,18 +1537,12 @@ void ilu_factor_sweep(int B, const IluSweep& t, const int* rp, const int* col, c
 }
 
 // the chunked apply with `lds` bytes of dynamic LDS; above 64 KiB the
-// kernel's limit is raised first (once per instantiation and size)
+// kernel's limit is raised first
 template <int BB, typename V, int K>
 void launch_ilu_chunk_k(size_t lds, const IluSweep& t, const double* lu, const double* dinv, const V* in, V* tmp,
                         V* out, const BicgScalars* sc, hipStream_t s) {
-  static std::atomic<size_t> raised{64 * 1024};
-  if (lds > raised.load()) {
-    DCG_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&ilu_apply_chunk_k<BB, V, K>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds)));
-    size_t cur = raised.load();
-    while (lds > cur && !raised.compare_exchange_weak(cur, lds)) {
-    }
-  }
+  static std::atomic<unsigned long long> raised{0};
+  raise_lds(reinterpret_cast<const void*>(&ilu_apply_chunk_k<BB, V, K>), lds, raised);
   ilu_apply_chunk_k<BB, V, K><<<1, kIluThreads, lds, s>>>(t, lu, dinv, in, tmp, out, sc);
 }
 template <int BB, typename V>

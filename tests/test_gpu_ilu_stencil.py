@@ -1,10 +1,14 @@
 """The stencil form of ILU0 (1D and 2D structured grids, blocks of 1 and 2
 species) against the oracle at the sizes where its level schedule changes
-shape: single-cell grids, levels of 63 to 65 rows (one and two waves), of 128
-and more (the widest it takes), odd sizes, boxes and triangles, a compartment
-that covers a part of the grid.  The preconditioner is the same ILU0, so the
+shape: single-cell grids, levels of 63 to 66 rows (one and two waves) and of
+101 to 241 (501 with one species: nearly the widest it takes, with rings beyond
+64 KiB of LDS), odd sizes, boxes and triangles, a compartment that covers a
+part of the grid.  The preconditioner is the same ILU0, so the
 Newton iterations are equal, the BiCGSTAB iterations equal within one and the
 states equal to the parity bar of the other sweeps (1e-8)."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 
@@ -123,3 +127,61 @@ def test_partial_compartment(dca, wl):
     ini = w.ini.replace("domain.expression = 1", "domain.expression = (position_x-0.5)^2 + (position_y-0.45)^2 < 0.16")
     w.ini = ini
     _compare(dca, w, state=lambda m: 0.5 + 0.1 * np.random.default_rng(2).random(m.n_dof))
+
+
+def _wide(dca, wl, species, n, cell):
+    """A model, its matrix at a random state, a right-hand side, and the oracle's x after one BiCGSTAB iteration."""
+    w = (wl.exponential_decay(dim=2, n=n, cell_type=cell, D=0.02) if species == 1 else _gray_scott(wl, n, cell))
+    m, o = dca.Model(w.ini, "", 0), OracleModel(w.ini)
+    rng = np.random.default_rng(n)
+    x = 0.5 + 0.3 * rng.random(m.n_dof)
+    _, J = m.assemble(x, 0.0, 1.0, 0.1)
+    _, vals = o.assemble(x, 0.0, 1.0, 0.1)
+    b = rng.standard_normal(m.n_dof)
+    ref, its = np.zeros(m.n_dof), ctypes.c_int()
+    ptr = [ctypes.c_void_p(a.ctypes.data) for a in (vals, b, ref)]
+    o._L.orc_solve(o._h, *ptr, 1e-30, 1, ctypes.byref(its))
+    assert its.value == 1
+    o.close()
+    return m, J, b, ref
+
+
+def _check_wide(m, J, b, ref):
+    """Both sides round in FP64 over at most 3,000 levels of a diagonally dominant solve: 1e-10."""
+    x, _, its = m.linear_solve(J, b, 1e-30, 1)
+    assert its == 1
+    assert np.linalg.norm(x - ref) <= 1e-10 * np.linalg.norm(ref)
+
+
+@pytest.mark.parametrize("species,n,cell", [(2, 200, "cube"), (2, 300, "simplex"), (2, 480, "cube"), (1, 400, "simplex"),
+                                            (1, 1000, "cube")])
+def test_wide_levels(dca, wl, species, n, cell):
+    """Levels of (n + 2) / 2 rows, two to eight waves of them per solve level: x after one iteration as the oracle's
+    (alpha M^-1 b + omega M^-1 s with M the ILU0 of the same matrix)."""
+    print(f"case: stencil ILU0, wide levels, {species} species {cell} {n}", flush=True)
+    case = _wide(dca, wl, species, n, cell)
+    _check_wide(*case)
+    case[0].close()
+
+
+def test_sizes_of_lds_from_several_threads(dca, wl):
+    """Three models whose kernels want 66 to 160 KiB of LDS, each on its own thread."""
+    print("case: stencil ILU0 from threads", flush=True)
+    cases = [_wide(dca, wl, 2, n, "cube") for n in (205, 330, 480)]
+    errors = []
+
+    def work(case):
+        try:
+            for _ in range(3):
+                _check_wide(*case)
+        except BaseException as e:  # noqa: BLE001 - reported on the test's thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(c,)) for c in cases]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    for c in cases:
+        c[0].close()
