@@ -132,6 +132,29 @@ def test_steps(dca, dim, cells, precision, precond, runtime):
     orc.close()
 
 
+@pytest.mark.parametrize("precond", ["Jacobi", "VertexBlockJacobi"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("dim,cells", [(2, (66, 40)), (3, (9, 8, 17))])
+def test_steps_every_shape(dca, dim, cells, precision, precond):
+    """Steps with each tile shape forced, several tiles and remainders along every axis."""
+    print(f"case: corner form, every shape, {dim}D {precision} {precond}", flush=True)
+    ini = _ini(dim, cells, 6, rk="Alexander2")
+    orc = OracleModel(ini)
+    u0 = np.random.default_rng(4).random(orc.n_dof) * 0.2 + 0.5
+    orc.set_state(u0, 0.0)
+    assert orc.step(0.1)[0] == 0
+    for tile in (0, 1):
+        gpu = dca.Model(ini, f"model.time_step_operator.linear_solver.precision = {precision}\n"
+                             f"model.time_step_operator.linear_solver.preconditioner.type = {precond}\n"
+                             f"model.time_step_operator.linear_solver.point_tile = {tile}\n", 0)
+        assert "dcg_tile_0_e0" in gpu.generated_source()
+        gpu.set_state(u0, 0.0)
+        assert gpu.step(0.0, 0.1).status == 0
+        assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], orc.get_state()[0])) < 1e-8, tile
+        gpu.close()
+    orc.close()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_batch_of_sizes(dca, precision):
     """Members of one module with other sizes, spacings and constants, and one of another block size."""

@@ -110,6 +110,52 @@ def test_steps(dca, dim, cells, species, inner, precision, precond, costly):
     orc.close()
 
 
+@pytest.mark.parametrize("precond", ["Jacobi", "VertexBlockJacobi"])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("species,inner", [(2, 0), (3, 2), (1, 4)])
+def test_steps_every_shape(dca, species, inner, precision, precond):
+    """Steps with each tile shape forced, the walked layers among them: several chunks of layers along z and tiles along
+    x and y with remainders, partial compartments of other block sizes and facet rows, in both precisions."""
+    print(f"case: evaluated form, every shape, {species}+{inner} {precision} {precond}", flush=True)
+    ini = _ini(3, (28, 14, 34), species, inner, extensions=(1.0, 1.0, 1.0))
+    orc = OracleModel(ini)
+    u0 = np.random.default_rng(3).random(orc.n_dof) * 0.2 + 0.5
+    orc.set_state(u0, 0.0)
+    assert orc.step(0.1)[0] == 0
+    ref = orc.get_state()[0]
+    walked = 0
+    for tile in range(7):
+        over = f"model.time_step_operator.linear_solver.point_tile = {tile}\n"
+        gpu = dca.Model(ini, PTS.format(precond, precision) + over, 0)
+        src = gpu.generated_source()
+        assert "dcg_tile_0_e0" in src
+        walked += f"_e{tile}, double, vol0::ApplyShape{tile}, eval_march" in src
+        gpu.set_state(u0, 0.0)
+        assert gpu.step(0.0, 0.1).status == 0
+        assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], ref)) < 1e-8, tile
+        gpu.close()
+    assert walked == 3
+    orc.close()
+
+
+@pytest.mark.parametrize("inner,precision", [(0, "fp64"), (1, "mixed")])
+def test_finished_reductions(dca, inner, precision):
+    """1451^2 vertices: more than 2,048 partials of both operators and of the x and r update (1,024 vertices each), so
+    that every reduction goes through the finishing launch.  The matrix form of the same step is the reference."""
+    print(f"case: evaluated form, finished reductions, inner={inner} {precision}", flush=True)
+    ini = _ini(2, (1450, 1450), 1, inner, extensions=(1.0, 1.0, 1.0))
+    states = []
+    for storage in ("points", "matrix"):
+        m = dca.Model(ini, PTS.format("Jacobi", precision).replace("points", storage), 0)
+        assert ("dcg_tile_0_e0" in m.generated_source()) == (storage == "points")
+        m.set_state(m.initial_state(), 0.0)
+        assert m.step(0.0, 0.1).status == 0
+        states.append(m.get_state()[0])
+        comps = m.compartments()
+        m.close()
+    assert max(rel_l2_per_species(comps, *states)) < 1e-8
+
+
 @pytest.mark.parametrize("cells", [(361, 361), (362, 362)])
 def test_step_slots_per_thread(dca, cells):
     """Meshes just below and above the 131,072 vertices where the x and r update takes four slots per thread."""

@@ -52,6 +52,23 @@ def test_reduce_levels(dca, cells, split):
     m.close()
 
 
+@pytest.mark.parametrize("cells", [(2, 2), (16, 16), (52, 6), (300, 300), (516, 514)])
+def test_fold_order(dca, cells):
+    """A reduction that keeps the later value returns the last one in the order of cells (by parity of their indices, so
+    with even sides the corner cell comes last), whatever level it passes through."""
+    print(f"case: reduce order {cells}", flush=True)
+    m = dca.Model(f"[grid]\ndimension = 2\ncells = {cells[0]} {cells[1]}\nextensions = 2 3\ncell_type = cube\n"
+                  "[compartments]\ndomain.expression = 1\n[model.scalar_field.u]\ncompartment = domain\n"
+                  "storage.expression = 1\ncross_diffusion.u.expression = 0.1\ninitial.expression = position_x\n"
+                  "[model.time_step_operator]\ntype = ImplicitEuler\n", "", 0)
+    m.set_state(m.initial_state(), 0.0)
+    got = m.reduce("[last]\nevaluation.expression = position_x + 10*position_y\nreduction.expression = a, b: a\n"
+                   "initial.value = 7\n")
+    edge = 0.5 - 0.5 * np.sqrt(0.6)
+    assert abs(got["last"] - (2 - edge * 2 / cells[0] + 10 * (3 - edge * 3 / cells[1]))) <= 1e-12 * 32
+    m.close()
+
+
 def test_kept_plans_count_as_footprint(dca):
     """A plan holds (value, defined) pairs per key: one per workgroup of 256 cells and one result."""
     print("case: reduce plans in the footprint", flush=True)
