@@ -499,6 +499,17 @@ static bool uniform(const Ex& e) {
   return true;
 }
 
+// a divisor whose reciprocal serves: uniform, and where its value is known, of
+// a size that neither overflows nor loses bits as a reciprocal
+static bool reciprocal(const Ex& e) {
+  if (!uniform(e)) return false;
+  std::vector<std::string> vars;
+  collect_vars(e, vars);
+  if (!vars.empty()) return true;
+  const double v = std::fabs(evaluate(e, {}));
+  return v >= 0x1p-1021 && v <= 0x1p1021;
+}
+
 int cost(const Ex& e) {
   if (!e) return 0;
   int c = 0;
@@ -507,7 +518,7 @@ int cost(const Ex& e) {
   switch (e->kind) {
     case Kind::Const:
     case Kind::Var: return 0;
-    case Kind::Div: return uniform(e->args[1]) ? cost(e->args[0]) + 1 : c + 14;
+    case Kind::Div: return reciprocal(e->args[1]) ? cost(e->args[0]) + 1 : c + 14;
     case Kind::Pow:
       return is_const(e->args[1], &p) && (p == 2.0 || p == 3.0) ? c * static_cast<int>(p) + static_cast<int>(p) - 1
                                                                 : c + 100;
@@ -540,7 +551,7 @@ std::string emit(const Ex& e, const std::map<std::string, std::string>& map, boo
     case Kind::Sub: return "(" + E(0) + " - " + E(1) + ")";
     case Kind::Mul: return "(" + E(0) + " * " + E(1) + ")";
     case Kind::Div:
-      if (reciprocals && uniform(e->args[1])) return "(" + E(0) + " * (1.0 / " + E(1) + "))";
+      if (reciprocals && reciprocal(e->args[1])) return "(" + E(0) + " * (1.0 / " + E(1) + "))";
       return "(" + E(0) + " / " + E(1) + ")";
     case Kind::Mod: return "fmod(" + E(0) + ", " + E(1) + ")";
     case Kind::Pow: {

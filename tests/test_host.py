@@ -306,6 +306,23 @@ def test_corner_form_sums_in_64_bits(dca, wl):
         assert decl and set(decl) == {"double"}, sums
 
 
+def test_divisors_without_a_reciprocal(dca):
+    """Evaluated coefficients multiply by the reciprocal of a constant divisor, except where that would overflow or lose
+    bits: 1e-310 has no finite reciprocal, 1e308 a subnormal one."""
+    ini = ("[grid]\ndimension = 2\ncells = 8 8\nextensions = 1 1\ncell_type = cube\n[compartments]\n"
+           "domain.expression = 1\n[model.scalar_field.u]\ncompartment = domain\nstorage.expression = 1\n"
+           "cross_diffusion.u.expression = 0.01\nreaction.expression = 1e-305*u*u/{c}\n"
+           "reaction.jacobian.u.expression = 1e-305*u/{c}\n[model.time_step_operator]\ntype = ImplicitEuler\n"
+           "linear_solver.type = BiCGSTAB\nlinear_solver.preconditioner.type = Jacobi\n")
+    for c, product in (("3", True), ("1e-310", False), ("1e308", False)):
+        m = dca.Model(ini.format(c=c), "", -1)
+        src = m.generated_source()
+        m.close()
+        assert "dcg_tile_0_e0" in src
+        body = src[src.index("point_jacobian("):]
+        assert ("* (1.0 / " in body[:body.index("point_block(")]) == product, c
+
+
 _KINETICS = {  # per species: reaction by its neighbour, and its Jacobian entry
     "mass": ("0.9*{b}*{b} - 0.7*{a}*{b}", "-0.7*{b}", "1.8*{b} - 0.7*{a}"),
     "hill": ("{b}^2.5/(0.4+{b}^2.5) - 0.3*{a}", "-0.3",
