@@ -2689,7 +2689,6 @@ __device__ __forceinline__ void eval_march(int tile, int at, dcg_gp<const int> _
   const auto W = (dcg_gp<const T>)(const T*)op.w;
   const auto D = (dcg_gp<T>)(T*)op.d;
   const auto Y = (dcg_gp<T>)(T*)op.y;
-  const auto DI = (dcg_gp<const double>)op.dinv;
   const int mode = op.mode, tid = threadIdx.x, bi = tid & 15, bj = tid >> 4;
   const int ntx = (n0 + 1 + TX - 1) / TX, nty = (n1 + 1 + TY - 1) / TY;
   const int tx = tile % ntx, ty = (tile / ntx) % nty, tz = tile / (ntx * nty);

@@ -37,17 +37,17 @@ struct GeneratedSource {
   // every cell of the grid, word-major: pc[word * cells + cell]
   std::vector<int> point_words;
   // candidate tile shapes of the point apply per compartment (entry points
-  // <tile_kernel>_p<k>, _pf<k> and the batched _pbatch<k>, _pfbatch<k>; see
-  // eval);
-  // the first is the assembly tile
+  // <tile_kernel>_p<k>, _pf<k> and the batched _pbatch<k>, _pfbatch<k>, or
+  // those of eval); the first is the assembly tile
   std::vector<std::vector<std::array<int, 3>>> apply_tiles;
   // per compartment and candidate: the waves per SIMD its registers are
   // bounded for (1: none), and the workgroup size
   std::vector<std::vector<int>> apply_waves, apply_threads;
   // compartments whose point applies evaluate their coefficients at the
-  // linearisation point (no stored words; entry points _e<k>, _ef<k>,
-  // _ebatch<k>, _efbatch<k>), and those of them in the corner form, whose
-  // residual and point set-up run over corner_tiles(dim).front()
+  // linearisation point (no stored words; entry points _e<k>, _ef<k>, the
+  // batched plain apply _ebatch<k> and the batched fused ones _kbatch<k>,
+  // _kfbatch<k>), and those in the corner form, whose residual and point
+  // set-up run over corner_tiles(dim).front()
   std::vector<char> eval, corner;
   // point storage evaluates everywhere and the facets have row form
   // (dcg_facet_rows, _f): BiCGSTAB runs on fused operator launches

@@ -1026,7 +1026,7 @@ void Model::launch_points_setup(const double* x, double t, double cm, double ca)
 // written (the returned count is 0: the caller forms the dots).
 int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp32, const void* w1, const void* w2,
                                double* part) {
-  if (fused()) {
+  if (gen_.fused) {
     // a plain apply of the fused launches (nothing calls it with partials)
     if (part || stop) throw Error("internal: plain operator launch with partials");
     k::KrylovOp op{};
@@ -1045,9 +1045,7 @@ int Model::launch_points_apply(const void* v, void* y, const int* stop, bool fp3
     if (!pc_app_fn_[c] || comp_dev_[c].ntiles <= 0) continue;
     const int* g2l = comp_dev_[c].g2l_identity ? nullptr : comp_dev_[c].g2l.get();
     const unsigned char* cmask = comp_dev_[c].cell_mask_grid.get();
-    const void* pc = gen_.eval[c] ? static_cast<const void*>(lin_x_.get())
-                     : fp32         ? static_cast<const void*>(pc32_[c].get())
-                                    : static_cast<const void*>(pc_[c].get());
+    const void* pc = fp32 ? static_cast<const void*>(pc32_[c].get()) : static_cast<const void*>(pc_[c].get());
     double* pp = part && facet_fn_.empty() ? part + 2 * static_cast<size_t>(nparts) : nullptr;
     // the apply's own tile shape (chosen at set-up) and its tile list
     const int k2 = apply_shape_[c];

@@ -437,7 +437,6 @@ class Model {
   DeviceArray<int2> st_upos_;
   DeviceArray<double> st_pack_, st_lower_, st_upper_;
   bool build_ilu_stencil(const std::vector<int>& lrows, const std::vector<int>& urows);
-  bool ilu_ready_ = false;
   std::vector<std::pair<int, double>> tuning_;
   // profiling
   bool prof_ = false;

@@ -206,8 +206,6 @@ void b_bicg_setup(const BatchWork& w, Skip sk, const double* tol, const IrState*
 template <typename V>
 void b_bicg_init(int B, const BatchWork& w, const MemberView* mv, int b, int x, double* part, BicgScalars* sc,
                  hipStream_t st);
-// one BiCGSTAB iteration on every unfinished member (jacobi: apply dinv)
-// ev (optional, 4 events): recorded before and after each of the two SpMVs
 // A fused iteration's x and r update over the members (after its second
 // operator launch, op: the finish of that launch's partials, and where this
 // one's scalars and partials go; vectors p = op.a, v = op.c), and the finish of
@@ -215,6 +213,8 @@ void b_bicg_init(int B, const BatchWork& w, const MemberView* mv, int b, int x, 
 template <typename V>
 void b_bicg_fused_xr(int B, const BatchWork& w, const MemberView* mv, int x, const BatchOp& op, hipStream_t s);
 void b_bicg_finish(const BatchWork& w, const BicgScalars* in, BicgScalars* out, const double* fin, hipStream_t s);
+// one BiCGSTAB iteration on every unfinished member (jacobi: apply dinv)
+// ev (optional, 4 events): recorded before and after each of the two SpMVs
 template <typename V>
 void b_bicg_iteration(int B, int variant, const BatchWork& w, const MemberView* mv, int x, int jacobi,
                       double* part, BicgScalars* sc, hipStream_t st, hipEvent_t* ev = nullptr,

@@ -1467,10 +1467,15 @@ void bicg_finish(const BicgScalars* in, BicgScalars* out, const double* fin, int
   else if (stage == 2) bicg_finish_k<3><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, 2);
   else bicg_finish_k<2><<<1, 1024, 0, s>>>(in, out, fin, nfin, fstride, stage);
 }
-// Slots per thread of the x and r update: 4 for meshes whose workgroups fill
-// the chip twice over, 1 below, where four times the workgroups load at once
-// (4 slots -> 1: 25^2 FP64 4.7 -> 3.6 us, 48^3 FP32 7.3 -> 5.8 us, 41^3 with 7
-// species FP32 9.2 -> 6.6 us, 301^2 with 4 species FP32 8.7 -> 6.2 us)
+// Slots per thread of the x and r update: 1 up to 131,072 vertices (512
+// workgroups, two per CU), where four times the workgroups load at once (4
+// slots -> 1: 25^2 FP64 4.7 -> 3.6 us, 48^3 FP32 7.3 -> 5.8 us, 41^3 with 7
+// species FP32 9.2 -> 6.6 us, 301^2 with 4 species FP32 8.7 -> 6.2 us); 4 above,
+// with a quarter of the partials.  Past the line the forms are within 20% of
+// each other either way (4 slots -> 1: 138k vertices, 2 species, FP64 8.2 -> 7.7
+// and FP32 8.5 -> 6.1 us, 4 species FP64 10.7 -> 11.3; 263k 11.3 -> 10.3, 10.2 ->
+// 10.5, 17.8 -> 16.5; 520k 15.2 -> 13.6, 9.5 -> 12.2, 22.9 -> 28.4; 1.05M, 2
+// species, 24.4 -> 24.1 and 15.3 -> 16.1 us)
 static int fused_xr_slots(int nslot) { return nslot > kFusedXrWide ? kXrSlots : 1; }
 int bicg_fused_xr_parts(int nslot) {
   const int per = kThreads * fused_xr_slots(nslot);
