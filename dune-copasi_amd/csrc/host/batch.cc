@@ -422,7 +422,10 @@ void Batch::rebuild() {
       g.prange.upload(prange, stream_);
       g.part.resize(2 * std::max<size_t>(std::max(vwork.size(), static_cast<size_t>(g.nitems)), 1) + 64);
       if (g.fused) {
-        g.sck.resize(3 * static_cast<size_t>(M));
+        g.sck.resize(4 * static_cast<size_t>(M));
+        double reads = 0.0;  // partials read if every workgroup of a member sums that member's
+        for (const auto& r : prange) reads += static_cast<double>(r.y - r.x) * (r.y - r.x);
+        g.finish = reads > static_cast<double>(k::kFinishParts) * k::kFinishParts;
         g.kpart.resize(4 * static_cast<size_t>(g.nitems) + 2 * static_cast<size_t>(g.w.nvwork4) + 64);
       }
       const int gi = static_cast<int>(&g - sgroups_.data());
@@ -569,7 +572,8 @@ void Batch::tune(SolverGroup& g) {
 
 // Fused BiCGSTAB iterations: both operator launches form their direction and
 // finish the reductions before them (k::BatchOp), so an iteration is 3
-// launches where it was 8; one more per call leaves the scalars in g.sc.
+// launches where it was 8; one more per call leaves the scalars in g.sc.  Large
+// groups finish each reduction in a launch of its own (g.finish).
 void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* ev) {
   const size_t M = g.mem.size();
   const int np = g.nitems, nx = g.w.nvwork4;
@@ -579,6 +583,13 @@ void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* e
   const k::PcMember* mem = g.pcm.get();
   auto mark = [&](int i) {
     if (ev) DCG_HIP(hipEventRecord(ev[i], stream_));
+  };
+  k::BicgScalars* finished = g.sck.get() + 3 * M;
+  auto finish = [&](k::BatchOp& op, int stage) {
+    if (!g.finish || !op.frange) return;
+    k::b_bicg_finish(g.w, op.frange, op.in, finished, op.fin, op.fstride, stage, stream_);
+    op.in = finished;
+    op.frange = nullptr;
   };
   auto launch = [&](k::BatchOp op) {
     for (int* v : {&op.a, &op.b, &op.c, &op.d, &op.y, &op.w}) *v += base;
@@ -612,6 +623,7 @@ void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* e
     op.range = g.prange.get();
     op.part = pa;
     op.pstride = np;
+    finish(op, 4);
     mark(0);
     launch(op);
     mark(1);
@@ -625,6 +637,7 @@ void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* e
     op.frange = g.prange.get();
     op.fstride = np;
     op.part = pb;
+    finish(op, 1);
     mark(2);
     launch(op);
     mark(3);
@@ -632,6 +645,8 @@ void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* e
     op.in = s[2];
     op.out = s[0];
     op.fin = pb;
+    op.frange = g.prange.get();
+    finish(op, 2);
     op.range = g.w.vrange4;
     op.part = pc;
     op.pstride = nx;
@@ -639,7 +654,7 @@ void Batch::fused_iterations(SolverGroup& g, bool fp32, int count, hipEvent_t* e
     else k::b_bicg_fused_xr<double>(g.B, g.w, g.mv.get(), k::kVZ, op, stream_);
     g.parity = nxt;
   }
-  k::b_bicg_finish(g.w, s[0], g.sc.get(), pc, stream_);
+  k::b_bicg_finish(g.w, g.w.vrange4, s[0], g.sc.get(), pc, nx, 4, stream_);
 }
 
 void Batch::capture(SolverGroup& g, bool fp32) {

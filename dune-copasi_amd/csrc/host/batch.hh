@@ -147,10 +147,16 @@ class Batch {
     k::BatchOperator op64, op32;
     // members that evaluate their coefficients: fused iterations (3 launches
     // per module, 2 of them operators), with the scalars handed from launch to
-    // launch in sck (M each) and partials of their own
+    // launch in sck (M each, the fourth for finished reductions) and partials
+    // of their own
     bool fused = false;
     int parity = 0;  // which of the two p and v a fused iteration reads
     DeviceArray<k::BicgScalars> sck;
+    // reductions finished by a launch of their own, a workgroup per member,
+    // where the members' workgroups would together read more partials than the
+    // kFinishParts squared of a single model (256 members of 32^2 to 512^2,
+    // FP32, about 40 million: operator 271 -> 244 us, step 38.6 -> 37.3 ms)
+    bool finish = false;
     DeviceArray<double> kpart;
   };
   // `count` iterations from the scalars in g.sc and back to them

@@ -453,7 +453,7 @@ __global__ void __launch_bounds__(kThreads) bfused_xr_k(const int2* __restrict__
                                                         const MemberView* __restrict__ mv, int x, BatchOp op) {
   __shared__ double red[32];
   const int2 w = work[blockIdx.x];
-  const int2 fr = op.frange[w.x];
+  const int2 fr = op.frange ? op.frange[w.x] : make_int2(0, 0);
   BicgScalars sc;
   if (!finish_stage<kThreads, 3>(sc, op.in + w.x, op.out + w.x, (int)blockIdx.x == op.range[w.x].x, op.fin + fr.x,
                                  fr.y - fr.x, op.fstride, 2, red))
@@ -512,14 +512,15 @@ __global__ void __launch_bounds__(kThreads) bfused_xr_k(const int2* __restrict__
     op.part[op.pstride + blockIdx.x] = acc[1];
   }
 }
+template <int N>
 __global__ void __launch_bounds__(kThreads) bfinish_k(const int2* __restrict__ range, const BicgScalars* __restrict__ in,
                                                       BicgScalars* __restrict__ out, const double* __restrict__ fin,
-                                                      int fstride) {
+                                                      int fstride, int stage) {
   __shared__ double red[32];
   const int m = blockIdx.x;
   const int2 r = range[m];
   BicgScalars sc;
-  finish_stage<kThreads, 2>(sc, in + m, out + m, true, fin + r.x, r.y - r.x, fstride, 4, red);
+  finish_stage<kThreads, N>(sc, in + m, out + m, true, fin + r.x, r.y - r.x, fstride, stage, red);
 }
 
 // ----------------------------------------------------------------- refinement
@@ -716,8 +717,12 @@ void b_bicg_fused_xr(int B, const BatchWork& w, const MemberView* mv, int x, con
 }
 template void b_bicg_fused_xr<double>(int, const BatchWork&, const MemberView*, int, const BatchOp&, hipStream_t);
 template void b_bicg_fused_xr<float>(int, const BatchWork&, const MemberView*, int, const BatchOp&, hipStream_t);
-void b_bicg_finish(const BatchWork& w, const BicgScalars* in, BicgScalars* out, const double* fin, hipStream_t st) {
-  if (w.members > 0) bfinish_k<<<w.members, kThreads, 0, st>>>(w.vrange4, in, out, fin, w.nvwork4);
+void b_bicg_finish(const BatchWork& w, const int2* range, const BicgScalars* in, BicgScalars* out, const double* fin,
+                   int fstride, int stage, hipStream_t st) {
+  if (w.members <= 0) return;
+  if (stage == 1) bfinish_k<1><<<w.members, kThreads, 0, st>>>(range, in, out, fin, fstride, stage);
+  else if (stage == 2) bfinish_k<3><<<w.members, kThreads, 0, st>>>(range, in, out, fin, fstride, stage);
+  else bfinish_k<2><<<w.members, kThreads, 0, st>>>(range, in, out, fin, fstride, stage);
 }
 
 void b_spmv64(int B, int variant, const BatchWork& w, const MemberView* mv, Skip sk, int x, int y, hipStream_t st) {

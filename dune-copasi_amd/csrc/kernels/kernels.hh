@@ -212,7 +212,8 @@ void b_bicg_init(int B, const BatchWork& w, const MemberView* mv, int b, int x, 
 // its reductions into out for the host and the next block of iterations.
 template <typename V>
 void b_bicg_fused_xr(int B, const BatchWork& w, const MemberView* mv, int x, const BatchOp& op, hipStream_t s);
-void b_bicg_finish(const BatchWork& w, const BicgScalars* in, BicgScalars* out, const double* fin, hipStream_t s);
+void b_bicg_finish(const BatchWork& w, const int2* range, const BicgScalars* in, BicgScalars* out, const double* fin,
+                   int fstride, int stage, hipStream_t s);
 // one BiCGSTAB iteration on every unfinished member (jacobi: apply dinv)
 // ev (optional, 4 events): recorded before and after each of the two SpMVs
 template <typename V>

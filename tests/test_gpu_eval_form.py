@@ -254,3 +254,32 @@ def test_compartments_share_scalars(dca):
     assert np.linalg.norm(b - A @ z) <= 1e-7 * np.linalg.norm(b)
     gpu.close()
     orc.close()
+
+
+@pytest.mark.parametrize("graph", [0, 4])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_batch_finished_reductions(dca, precision, graph):
+    """A 513^2 member in tiles of 16 x 8 rows (2,145 of them) takes its group's reductions through launches of their own;
+    members of other sizes and modules in the same group.  Each member's own steps are the reference."""
+    print(f"case: evaluated form batch, finished reductions {precision} graph_iterations={graph}", flush=True)
+    inis = [_ini(2, (512, 512), 2), _ini(2, (300, 200), 2, extensions=(0.5, 2.0, 1.0)), _ini(2, (9, 7), 2),
+            _ini(3, (12, 9, 7), 2)]
+    batch = dca.Batch(f"precision = {precision}\npreconditioner = Jacobi\ngraph_iterations = {graph}\n"
+                      "iteration_limit = 2000\npoint_tile = 0\n", 0)
+    members, singles = [], []
+    for ini in inis:
+        i = batch.add(ini)
+        batch.set_time_step(i, 0.1)
+        m, s = batch.member(i), dca.Model(ini, PTS.format("Jacobi", precision), 0)
+        u0 = 0.5 + 0.2 * np.random.default_rng(i).random(m.n_dof)
+        for x in (m, s):
+            x.set_state(u0, 0.0)
+        members.append(m)
+        singles.append(s)
+    for k in range(2):
+        assert all(st.status == 0 for st in batch.step())
+        for m, s in zip(members, singles):
+            assert s.step(0.1 * k, 0.1).status == 0
+            assert max(rel_l2_per_species(m.compartments(), m.get_state()[0], s.get_state()[0])) < 1e-8
+    for s in singles:
+        s.close()
