@@ -2456,13 +2456,13 @@ const char* kEvalKrylov = R"(
 namespace %C% {
 // M^-1 q at slot s (jac 0: none, 1: a block per slot, 2: the diagonal)
 template <typename T>
-__device__ __forceinline__ void precondition(int jac, const double* __restrict__ dinv, int s, const T (&q)[BC],
+__device__ __forceinline__ void precondition(int jac, dcg_gp<const double> dinv, int s, const T (&q)[BC],
                                              T (&o)[BC]) {
   if (jac == 2) {
 #pragma unroll
     for (int i = 0; i < BC; ++i) o[i] = (T)(dinv[(size_t)s * DCG_B + i] * (double)q[i]);
   } else if (jac == 1) {
-    const double* d = dinv + (size_t)s * (DCG_B * DCG_B);
+    const auto d = dinv + (size_t)s * (DCG_B * DCG_B);
 #pragma unroll
     for (int i = 0; i < BC; ++i) {
       double v = 0.0;
@@ -2588,7 +2588,7 @@ __device__ __forceinline__ void eval_krylov(int tile, int at, dcg_gp<const int> 
     }
 #pragma unroll
     for (int i = 0; i < BC; ++i) o[i] = q[i];
-    if (s >= 0 && mode) precondition(op.jac, op.dinv, s, q, o);
+    if (s >= 0 && mode) precondition(op.jac, (dcg_gp<const double>)op.dinv, s, q, o);
 #pragma unroll
     for (int i = 0; i < BC; ++i) vs[b * BC + i] = o[i];
   }
@@ -2777,7 +2777,7 @@ __device__ __forceinline__ void eval_march(int tile, int at, dcg_gp<const int> _
         o[i] = q0[i];
         x0[i] = lx[i];
       }
-      if (s >= 0 && mode) precondition(op.jac, op.dinv, s, q0, o);
+      if (s >= 0 && mode) precondition(op.jac, (dcg_gp<const double>)op.dinv, s, q0, o);
       if (mode == 1 && row && s >= 0 && k >= z0 && k <= z1)
 #pragma unroll
         for (int i = 0; i < DCG_B; ++i) D[(size_t)s * DCG_B + i] = i < BC ? q0[i < BC ? i : 0] : T(0);
@@ -3316,7 +3316,7 @@ const char* kCornerOpDirection = R"(      if constexpr (OP == 5) {
         T q[BC], h[BC];
 #pragma unroll
         for (int i = 0; i < BC; ++i) h[i] = q[i] = slot >= 0 ? kdir((size_t)slot * DCG_B + i) : T(0);
-        if (slot >= 0 && kmode) precondition(op->jac, op->dinv, slot, q, h);
+        if (slot >= 0 && kmode) precondition(op->jac, (dcg_gp<const double>)op->dinv, slot, q, h);
 #pragma unroll
         for (int i = 0; i < BC; ++i) vh[i] = (double)h[i];
       }
