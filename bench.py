@@ -286,7 +286,7 @@ def batch_measure(args, dca, wl, precision, warmup, steps, plain_stride, cpu=Tru
     if n:
         gbs = (by / n) / (ms / n * 1e-3) / 1e9
         roofline = {"bound": "hbm", "kernel": f"batched {'FP32' if kind == 'spmv32' else 'FP64'} Krylov operator "
-                                              f"(point apply dcg_tile_0_pfbatch / BCSR bspmv_k)",
+                                              f"(fused dcg_tile_0_kfbatch, point apply dcg_tile_0_pfbatch or BCSR bspmv_k)",
                     "achieved": gbs, "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": gbs / HBM_PEAK_GBS, "traffic": None, "avg_launch_us": 1e3 * ms / n,
                     "algorithmic_bytes_per_launch": by / n, "launches": n}
@@ -658,6 +658,9 @@ def main():
                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": sp["gbs"] / HBM_PEAK_GBS,
                     "traffic": committed_traffic(args.workload, args.precision, kernel),
                     "avg_launch_us": sp["avg_us"], "algorithmic_bytes_per_launch": sp["bytes_per_launch"]}
+        if spmv_kind.startswith("point") and form == "e":
+            # counters of the 96^3 run: waits in half of the wave cycles, vector issue in 45% of the SIMDs'
+            roofline["limited_by"] = "latency and vector issue of the evaluated coefficients, not bandwidth"
 
     probe = None
     if args.copy_probe_mib:

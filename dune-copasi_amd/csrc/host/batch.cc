@@ -884,7 +884,11 @@ void Batch::iterate(SolverGroup& g, bool fp32) {
         if (sc[j].done) continue;
         all = false;
         const Model& mj = *members_[g.mem[j]].m;
-        bytes += mj.point_storage() ? mj.point_apply_bytes(fp32 ? 4 : 8, 1) : mj.spmv_bytes(fp32 ? 4 : 8, fp32 ? 4 : 8, 1);
+        const int vb = fp32 ? 4 : 8;
+        // (a fused iteration's operators read 4 vectors and 1 beside the operand: their mean)
+        bytes += g.fused ? 0.5 * (mj.point_apply_bytes(vb, 4) + mj.point_apply_bytes(vb, 1))
+                 : mj.point_storage() ? mj.point_apply_bytes(vb, 1)
+                                      : mj.spmv_bytes(vb, vb, 1);
       }
       if (all || done_its > opt_.lin_maxit + 4) break;
       if (g.fused)

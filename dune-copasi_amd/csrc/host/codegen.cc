@@ -2646,7 +2646,9 @@ __device__ __forceinline__ void eval_krylov(int tile, int at, dcg_gp<const int> 
 // 47^3 14.5 us against 20.7 us, too few columns: the shapes are timed at set-up
 // and the faster one is taken.  About 350 FP64 instructions per layer and
 // wave, two waves per SIMD (218 registers; bounded for three it spills: 102
-// us); bound by their issue and by what two waves leave of the latency.
+// us).  At 96^3 vector issue fills about 45% of the cycles and waves wait in
+// half of theirs (counters): bound by the latency that two waves leave, then
+// by issue.
 const char* kEvalMarch = R"(
 template <int A>
 __device__ __forceinline__ double lane_next(double v) {  // A 0: of lane + 1, 1: of lane - 1 (of 16)
@@ -3010,10 +3012,10 @@ const char* kEvalBatch = R"(
 // A workgroup takes the cells around TX x TY row vertices of a layer and walks
 // TM layers along the last axis; a layer's corner sums meet in LDS, and what
 // it adds to the next layer's vertices stays in a register.
-// 7 species on 40^3 (68,921 vertices, 34 coefficients per point): apply FP32
-// 27 us and FP64 29 us (SpMV on the assembled matrix 83 and 220 us), set-up
-// 37 us (Jacobian pass 3,330 us and its FP32 copy 200 us), residual 28 us
-// (360 us with the corner values in LDS).  About 500 vector instructions per
+// 7 species on 40^3 (68,921 vertices, 34 coefficients per point): fused FP32
+// operator 42 us and plain FP64 apply 32 us (SpMV on the assembled matrix 83
+// and 220 us), set-up 38 us (Jacobian pass 3,330 us and its FP32 copy 200 us),
+// residual 28 us (360 us with the corner values in LDS).  About 500 vector instructions per
 // wave and layer of 8 cells; bound by their issue and by the two barriers of
 // a layer, not by memory (12 MB per apply).
 const char* kCorner = R"(
