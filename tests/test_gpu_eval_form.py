@@ -283,3 +283,25 @@ def test_batch_finished_reductions(dca, precision, graph):
             assert max(rel_l2_per_species(m.compartments(), m.get_state()[0], s.get_state()[0])) < 1e-8
     for s in singles:
         s.close()
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("cells,species,inner", [(n, b, 0) for n in (1, 2, 126, 127, 128, 300) for b in (1, 2, 4)] +
+                         [(n, b, i) for n in (126, 127, 128, 300) for b, i in ((3, 2), (1, 4))])
+def test_one_dimension(dca, cells, species, inner, precision):
+    """Intervals around the tile's 128 vertices: the apply and a step, with an interface where two compartments fit."""
+    print(f"case: evaluated form 1D {cells} {species}+{inner} {precision}", flush=True)
+    ini = _ini(1, (cells,), species, inner)
+    gpu, orc = dca.Model(ini, PTS.format("Jacobi", precision), 0), OracleModel(ini)
+    assert "dcg_tile_0_e0" in gpu.generated_source()
+    rng = np.random.default_rng(cells)
+    x, v = 0.5 + 0.2 * rng.random(gpu.n_dof), rng.standard_normal(gpu.n_dof)
+    _, vals = orc.assemble(x, 0.4, 1.0, 0.3)
+    ref = orc.csr(vals) @ v
+    assert np.abs(gpu.jacobian_apply(x, 0.4, 1.0, 0.3, v) - ref).max() <= 1e-12 * np.abs(ref).max()
+    for m in (gpu, orc):
+        m.set_state(x, 0.0)
+    assert gpu.step(0.0, 0.1).status == 0 and orc.step(0.1)[0] == 0
+    assert max(rel_l2_per_species(gpu.compartments(), gpu.get_state()[0], orc.get_state()[0])) < 1e-8
+    gpu.close()
+    orc.close()
